@@ -106,7 +106,7 @@ struct JobDev {
 #define LR_WALK_BLAS 0x80000000u
 #define LR_WALK_EXIT 0xffffffffu
 
-enum { K_REGEN = 0, K_EXTEND = 1, K_SHADE = 2, K_SHADOW = 3 };
+enum { K_EXTEND = 0, K_SHADE = 1, K_SHADOW = 2 };
 
 // the engine's counters (device memory, followed by each job slot's progress)
 struct EngCtl {
@@ -115,12 +115,12 @@ struct EngCtl {
     unsigned long long iq_lo, iq_hi;        // the issue records in use
     unsigned long long rays_ext, rays_shadow;
     unsigned long long iter;                // iterations run (its parity picks the ray queue)
-    unsigned long long claimed;             // paths the running iteration's regen started
-    unsigned int count[4];                  // ray queues [0], [1]; shadow queue [2]
-    unsigned int tiles[4];                  // each kernel's tile counter (work-groups claim tiles)
-    unsigned int regen_done;                // regen's work-groups that have finished
+    unsigned long long claimed;             // paths the running iteration's regen started (at the end of
+                                            // the ray queue, past its count; 0 after the iteration)
+    unsigned int count[4];                  // ray queues [0], [1] as shade left them; shadow queue [2]
+    unsigned int tiles[3];                  // extend's, shade's, shadow's tile counters
     unsigned int spar;                      // the parity of the queue the shade kernel appended to
-    unsigned long long pad[3];
+    unsigned long long pad[4];
 };
 
 struct EngProgress {

@@ -13,34 +13,66 @@
 
 namespace {
 
-// The entries [0, n) in tiles of BLK * mult, claimed by the work-groups one at a time through
-// a counter (persistent work-groups loop; a grid that covers n takes one tile each). body(i,
-// live) runs for every lane, live or not, so that it may use wave-wide ballots.
+// The entries [0, n) in tiles of BLK * mult. A work-group's first tile is its own index, the later
+// ones are claimed one at a time through a counter (from the grid's size on): work-groups with
+// no tile, and grids that cover n, make no claim. Claims of one counter are served about 12 ns
+// apart, so 2048 persistent work-groups each finding out by a claim that a queue is (nearly) empty
+// took 30 us a kernel; by their index, 3. body(i, live) runs for every lane, live or not, so
+// that it may use wave-wide ballots.
 template <int BLK, class F>
 __device__ __forceinline__ void for_tiles(unsigned int *ctr, uint32_t n, int mult, F &&body)
 {
     __shared__ uint32_t s_tile;
     const uint32_t width = (uint32_t)BLK * (uint32_t)mult;
-    for (;;) {
-        __syncthreads();
-        if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1u);
-        __syncthreads();
-        const uint64_t base = (uint64_t)s_tile * width;
-        if (base >= n) break;
+    const uint32_t ntiles = (uint32_t)(((uint64_t)n + width - 1) / width);
+    for (uint32_t tile = blockIdx.x; tile < ntiles;) {
+        const uint64_t base = (uint64_t)tile * width;
         for (int j = 0; j < mult; j++) {
             const uint64_t i = base + (uint64_t)j * BLK + threadIdx.x;
             body((uint32_t)i, i < n);
         }
+        if (ntiles <= gridDim.x) break;
+        __syncthreads();
+        if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1u);
+        __syncthreads();
+        tile = gridDim.x + s_tile;
+    }
+}
+
+// The same with every tile claimed, for bodies that wait on the tiles before theirs
+// (ordered_append2): a tile is claimed by a running work-group, in order, so every tile waited
+// on is being worked on however many of the grid's work-groups the chip holds at once. Where the
+// grid covers n, the work-groups past the tiles leave and each of the others claims once.
+template <int BLK, class F>
+__device__ __forceinline__ void for_tiles_ordered(unsigned int *ctr, uint32_t n, F &&body)
+{
+    __shared__ uint32_t s_tile;
+    const uint32_t ntiles = (uint32_t)(((uint64_t)n + BLK - 1) / BLK);
+    if (blockIdx.x >= ntiles) return;
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1u);
+        __syncthreads();
+        const uint32_t tile = s_tile;
+        if (tile >= ntiles) break;
+        const uint64_t i = (uint64_t)tile * BLK + threadIdx.x;
+        body((uint32_t)i, i < n);
+        if (ntiles <= gridDim.x) break;
     }
 }
 
 // Each kernel clears the other kernels' tile counters as it starts (kernels of one stream run
-// one after another, and no kernel follows itself), so every kernel finds its own at zero.
+// one after another, and no kernel follows itself), so every kernel finds its own at zero (regen
+// claims nothing: self = -1).
 __device__ __forceinline__ void reset_tiles(EngCtl *ctl, int self)
 {
-    for (int k = 0; k < 4; k++)
+    for (int k = 0; k < 3; k++)
         if (k != self) ctl->tiles[k] = 0;
 }
+
+// the ray queue's length while an iteration runs: the paths the last iteration's shade appended
+// and those this one's regen started after them
+__device__ __forceinline__ uint32_t queue_len(const EngCtl *ctl, int cur) { return ctl->count[cur] + (uint32_t)ctl->claimed; }
 
 __device__ __forceinline__ long long to_fixed(float x)
 {
@@ -386,54 +418,47 @@ __global__ __launch_bounds__(BLK) void k_regen(EngArgs A)
     const uint32_t start = ctl->count[cur];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctl->claimed = n;
-        reset_tiles(ctl, K_REGEN);
+        reset_tiles(ctl, -1);
     }
-    for_tiles<BLK>(&ctl->tiles[K_REGEN], n, A.mult, [&](uint32_t i, bool live) {
-        if (live) {
-            const unsigned long long g = next + i;
-            // the issue record holding g: the last one that starts at or before it
-            unsigned long long a = lo, b = hi;   // records [a, b); the answer in [a, b)
-            while (b - a > 1) {
-                const unsigned long long mid = a + (b - a) / 2;
-                if (A.iq_start[mid & (LR_ISSUE - 1)] <= g) a = mid;
-                else b = mid;
-            }
-            const uint32_t jslot = A.iq_job[a & (LR_ISSUE - 1)] & (LR_JOBS - 1);
-            const JobDev &J = A.jobs[jslot];
-            const uint32_t q = A.iq_q0[a & (LR_ISSUE - 1)] + (uint32_t)(g - A.iq_start[a & (LR_ISSUE - 1)]);
-            const uint32_t pixel = q % (uint32_t)J.npix;
-            const uint32_t k = J.s0 + q / (uint32_t)J.npix;
-            const int x = (int)(pixel % (uint32_t)J.W), y = (int)(pixel / (uint32_t)J.W);
-            const uint64_t seed = ((uint64_t)J.seed_hi << 32) | J.seed_lo;
-            uint64_t st = pcg_seed((uint64_t)pixel, k, seed);
-            const uint64_t inc = ((uint64_t)pixel << 1u) | 1u;
-            const Smp sm{x, y, k, (uint32_t)seed * 0x9e3779b9u, A.mask, &st, inc};
-            float jx, jy;
-            s2(sm, 0, jx, jy);
-            const float u = ((float)x + jx) / (float)J.W, v = ((float)y + jy) / (float)J.H;
-            // camera_ray (camera.h:38-42)
-            const V3 org = v3(J.cam[0], J.cam[1], J.cam[2]);
-            const V3 ul = v3(J.cam[3], J.cam[4], J.cam[5]), hz = v3(J.cam[6], J.cam[7], J.cam[8]),
-                     vt = v3(J.cam[9], J.cam[10], J.cam[11]);
-            const V3 target = vsub(vadd(ul, vscale(hz, u)), vscale(vt, v));
-            const V3 d = vnorm(vsub(target, org));
-            // every started path has its camera ray and its state: in claim order, after the
-            // queue's paths
-            const uint32_t at = start + i;
-            A.qray[cur][2 * (size_t)at] = make_float4(org.x, org.y, org.z, J.eps);
-            A.qray[cur][2 * (size_t)at + 1] = make_float4(d.x, d.y, d.z, 1e30f);
-            A.qid[cur][at] = jslot << LR_SLOT_BITS;
-            A.thr[cur][at] = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
-            A.rad[cur][at] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(EMIT_FULL));
-            A.rng[cur][at] = st;
-            A.meta[cur][at] = make_uint2(q, 0u);
+    // every path is the same work: no claims, each work-item takes every (grid's size)-th
+    for (uint32_t i = blockIdx.x * BLK + threadIdx.x; i < n; i += gridDim.x * BLK) {
+        const unsigned long long g = next + i;
+        // the issue record holding g: the last one that starts at or before it
+        unsigned long long a = lo, b = hi;   // records [a, b); the answer in [a, b)
+        while (b - a > 1) {
+            const unsigned long long mid = a + (b - a) / 2;
+            if (A.iq_start[mid & (LR_ISSUE - 1)] <= g) a = mid;
+            else b = mid;
         }
-    });
-    // the last work-group to finish sets the queue's length (all have read the old one)
-    __syncthreads();
-    if (threadIdx.x == 0 && atomicAdd(&ctl->regen_done, 1u) == gridDim.x - 1) {
-        ctl->count[cur] = start + n;
-        ctl->regen_done = 0;
+        const uint32_t jslot = A.iq_job[a & (LR_ISSUE - 1)] & (LR_JOBS - 1);
+        const JobDev &J = A.jobs[jslot];
+        const uint32_t q = A.iq_q0[a & (LR_ISSUE - 1)] + (uint32_t)(g - A.iq_start[a & (LR_ISSUE - 1)]);
+        const uint32_t pixel = q % (uint32_t)J.npix;
+        const uint32_t k = J.s0 + q / (uint32_t)J.npix;
+        const int x = (int)(pixel % (uint32_t)J.W), y = (int)(pixel / (uint32_t)J.W);
+        const uint64_t seed = ((uint64_t)J.seed_hi << 32) | J.seed_lo;
+        uint64_t st = pcg_seed((uint64_t)pixel, k, seed);
+        const uint64_t inc = ((uint64_t)pixel << 1u) | 1u;
+        const Smp sm{x, y, k, (uint32_t)seed * 0x9e3779b9u, A.mask, &st, inc};
+        float jx, jy;
+        s2(sm, 0, jx, jy);
+        const float u = ((float)x + jx) / (float)J.W, v = ((float)y + jy) / (float)J.H;
+        // camera_ray (camera.h:38-42)
+        const V3 org = v3(J.cam[0], J.cam[1], J.cam[2]);
+        const V3 ul = v3(J.cam[3], J.cam[4], J.cam[5]), hz = v3(J.cam[6], J.cam[7], J.cam[8]),
+                 vt = v3(J.cam[9], J.cam[10], J.cam[11]);
+        const V3 target = vsub(vadd(ul, vscale(hz, u)), vscale(vt, v));
+        const V3 d = vnorm(vsub(target, org));
+        // every started path has its camera ray and its state: in claim order, after the
+        // queue's paths
+        const uint32_t at = start + i;
+        A.qray[cur][2 * (size_t)at] = make_float4(org.x, org.y, org.z, J.eps);
+        A.qray[cur][2 * (size_t)at + 1] = make_float4(d.x, d.y, d.z, 1e30f);
+        A.qid[cur][at] = jslot << LR_SLOT_BITS;
+        A.thr[cur][at] = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
+        A.rad[cur][at] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(EMIT_FULL));
+        A.rng[cur][at] = st;
+        A.meta[cur][at] = make_uint2(q, 0u);
     }
 }
 
@@ -450,7 +475,8 @@ __device__ __forceinline__ void add_counts(unsigned long long *c, unsigned long 
 }
 
 // extend (wf_ext, trace_wave.wgsl:72-84): the closest hit of every queued ray, each through
-// its own job's tree. Also applies regen's claim to the ring and the issue counter, and clears
+// its own job's tree. Also applies regen's claim to the ring and the issue counter (the claim itself
+// is part of the queue's length until the shadow kernel ends the iteration), and clears
 // the queues the shade kernel appends to. TL: two-level scenes may be queued (without it, such
 // a ray is not walked: flagged, so that the host reports it).
 // Without TL the kernel is held to 64 VGPRs, 8 waves per SIMD: a few registers spill (12 bytes a
@@ -469,12 +495,11 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_extend(E
     __shared__ uint32_t stk[STK][BLK];
     EngCtl *ctl = A.ctl;
     const int cur = (int)(ctl->iter & 1ull);
-    const uint32_t n = ctl->count[cur];
+    const uint32_t n = queue_len(ctl, cur);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         const unsigned long long c = ctl->claimed;
         ctl->head += c;
         ctl->next += c;
-        ctl->claimed = 0;
         ctl->rays_ext += n;
         ctl->count[1 - cur] = 0;
         ctl->count[2] = 0;
@@ -637,12 +662,11 @@ __global__ __launch_bounds__(BLK, walk_waves(BLK, STK)) void k_extend_rf(EngArgs
     __shared__ uint32_t stk[STK][BLK];
     EngCtl *ctl = A.ctl;
     const int par = (int)(ctl->iter & 1ull);
-    const uint32_t n = ctl->count[par];
+    const uint32_t n = queue_len(ctl, par);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         const unsigned long long c = ctl->claimed;
         ctl->head += c;
         ctl->next += c;
-        ctl->claimed = 0;
         ctl->rays_ext += n;
         ctl->count[1 - par] = 0;
         ctl->count[2] = 0;
@@ -695,6 +719,7 @@ __global__ __launch_bounds__(BLK, walk_waves(BLK, STK)) void k_shadow_rf(EngArgs
         reset_tiles(ctl, K_SHADOW);
         ctl->rays_shadow += n;
         ctl->iter += 1;
+        ctl->claimed = 0;   // (the queue regen added to is done with)
     }
     const size_t gtid = (size_t)blockIdx.x * BLK + threadIdx.x;
     const WalkStack S{&stk[0][threadIdx.x], BLK, A.spill + gtid, (size_t)A.spill_stride, STK + A.spill_per};
@@ -872,12 +897,12 @@ __global__ __launch_bounds__(BLK) void k_shade(EngArgs A)
 {
     EngCtl *ctl = A.ctl;
     const int cur = (int)(ctl->iter & 1ull);
-    const uint32_t n = ctl->count[cur];
+    const uint32_t n = queue_len(ctl, cur);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         reset_tiles(ctl, K_SHADE);
         ctl->spar = (unsigned int)(1 - cur);
     }
-    for_tiles<BLK>(&ctl->tiles[K_SHADE], n, 1, [&](uint32_t i, bool live) {
+    for_tiles_ordered<BLK>(&ctl->tiles[K_SHADE], n, [&](uint32_t i, bool live) {
         bool next = false, shadow = false;
         float4 nr0, nr1, sr0, sr1, scon;
         uint32_t jslot = 0, q = 0;
@@ -1125,6 +1150,7 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_shadow(E
         reset_tiles(ctl, K_SHADOW);
         ctl->rays_shadow += n;
         ctl->iter += 1;
+        ctl->claimed = 0;   // (the queue regen added to is done with)
     }
     const size_t gtid = (size_t)blockIdx.x * BLK + threadIdx.x;
     const WalkStack S{&stk[0][threadIdx.x], BLK, A.spill + gtid, (size_t)A.spill_stride, STK + A.spill_per};

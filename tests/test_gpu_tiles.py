@@ -1,0 +1,53 @@
+"""GPU tests of how the engine's kernels share out a queue: a work-group's first tile is its own index,
+later ones are claimed, and work-groups without one leave.
+
+The image of a job does not depend on how its paths are shared out, so each image must equal to
+the bit the plain form's, whose grids cover the queue (one tile a work-group, nothing claimed).
+With 64 work-items a group and one group a compute unit the grid is 64 x (compute units)
+entries wide; the sizes lie around one grid, a few grids, and a single entry.
+"""
+import numpy as np
+import pytest
+
+import little_renderer_amd as lr
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def world():
+    assert torch.cuda.is_available(), "these tests need the GPU"
+    ctx = lr.Context(0)
+    sc = lr.batch_scene(2000, 5)
+    ps = lr.PtScene(ctx, sc["prims"], sc["tris"], sc["mats"], 0, sc["eps"], sc["margin"])
+    yield ctx, ps
+    ctx.close()
+
+
+def image(eng, i, w, h):
+    t = torch.zeros((h, w, 4), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    eng.image(i, t)
+    eng.release(i)
+    return t.cpu().numpy().view(np.uint32)
+
+
+@pytest.mark.parametrize("tile", [1, 4])
+@pytest.mark.parametrize("grids, off", [(0, 1), (0, 65), (1, -1), (1, 0), (1, 1), (3, 17)])
+def test_batched_equals_plain_at_the_grid_s_edges(world, grids, off, tile):
+    ctx, ps = world
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n = grids * 64 * cus + off                     # entries of the first iteration's queue
+    w = next(x for x in range(int(n ** 0.5), 0, -1) if n % x == 0)
+    h = n // w
+    eng = lr.Engine(ctx, slots_log2=18, max_tree_depth=max(64, ps.info()[0]), image_bytes=64 << 20)
+    eng.tune = {"block_trace": 64, "stack": 16, "block_shade": 64, "blocks_per_cu": 1, "tile": tile, "iters_per_graph": 3}
+    job = lr.make_job(ps, lr.batch_camera(9, w, h), w, h, 2, seed=n)
+    i = eng.submit(job)
+    eng.drain()
+    got = image(eng, i, w, h)
+    want = image(eng, eng.plain(job), w, h)
+    assert np.array_equal(got, want)
+    assert np.any(got[..., :3])
+    eng.close()
