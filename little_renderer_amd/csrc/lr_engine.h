@@ -143,7 +143,7 @@ struct EngArgs {
     float4 *thr[2];                         // throughput.rgb, the last bounce's pdf
     float4 *rad[2];                         // radiance.rgb, the emission state
     uint64_t *rng[2];                       // PCG32 state (stream: the pixel)
-    uint2 *meta[2];                         // q (index in the job), depth
+    uint2 *meta[2];                         // q (pass x pixels + pixel), depth
     float4 *qray[2];                        // o.xyz tmin | d.xyz tmax
     uint32_t *qid[2];                       // job << 22
     float4 *hits;                           // t, id, b1, b2 (by queue position)

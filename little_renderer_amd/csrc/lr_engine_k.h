@@ -403,6 +403,22 @@ __device__ WalkHit walk4_tl(const JobDev &J, V3 o, V3 d, float tmin, float tmax,
     return best;
 }
 
+// The r-th pixel of a pass over a W x H image: 8 x 8 tiles (narrower and lower at the right and
+// the bottom edge), tile after tile along bands of 8 rows, row by row in a tile. A wave's 64 camera
+// rays then cover a square and not a strip of 64 pixels, so more of its lanes are at work in each
+// node step of the walks and neighbouring lanes gather the same triangles and materials.
+__device__ __forceinline__ void tile_pixel(uint32_t r, uint32_t W, uint32_t H, uint32_t &x, uint32_t &y)
+{
+    // (8 W < 2^32 wherever there is more than one band: a pass has under 2^32 pixels)
+    const uint32_t band = H <= 8u ? 0u : r / (8u * W), in_band = r - band * (8u * W);
+    const uint32_t bh = min(8u, H - 8u * band);
+    const uint32_t t = in_band / (8u * bh), in_tile = in_band - t * 8u * bh;
+    const uint32_t tw = min(8u, W - 8u * t);
+    const uint32_t row = in_tile / tw;
+    x = 8u * t + (in_tile - row * tw);
+    y = 8u * band + row;
+}
+
 // regen (wf_gen, trace_wave.wgsl:51-70, with trace_image's seeds, tracer.c:335-346): `claimed`
 // free places of the pool start paths next .. next + claimed - 1, each a camera ray and its state
 // at the end of the ray queue
@@ -432,10 +448,15 @@ __global__ __launch_bounds__(BLK) void k_regen(EngArgs A)
         }
         const uint32_t jslot = A.iq_job[a & (LR_ISSUE - 1)] & (LR_JOBS - 1);
         const JobDev &J = A.jobs[jslot];
-        const uint32_t q = A.iq_q0[a & (LR_ISSUE - 1)] + (uint32_t)(g - A.iq_start[a & (LR_ISSUE - 1)]);
-        const uint32_t pixel = q % (uint32_t)J.npix;
-        const uint32_t k = J.s0 + q / (uint32_t)J.npix;
-        const int x = (int)(pixel % (uint32_t)J.W), y = (int)(pixel / (uint32_t)J.W);
+        // the job's paths in the order they start: pass after pass, each pass's pixels by tiles; from
+        // here on q is the path's pass and pixel (row-major)
+        const uint32_t q0 = A.iq_q0[a & (LR_ISSUE - 1)] + (uint32_t)(g - A.iq_start[a & (LR_ISSUE - 1)]);
+        const uint32_t pass = q0 / (uint32_t)J.npix;
+        uint32_t ux, uy;
+        tile_pixel(q0 - pass * (uint32_t)J.npix, (uint32_t)J.W, (uint32_t)J.H, ux, uy);
+        const uint32_t pixel = uy * (uint32_t)J.W + ux, q = pass * (uint32_t)J.npix + pixel;
+        const uint32_t k = J.s0 + pass;
+        const int x = (int)ux, y = (int)uy;
         const uint64_t seed = ((uint64_t)J.seed_hi << 32) | J.seed_lo;
         uint64_t st = pcg_seed((uint64_t)pixel, k, seed);
         const uint64_t inc = ((uint64_t)pixel << 1u) | 1u;

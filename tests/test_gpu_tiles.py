@@ -5,11 +5,17 @@ The image of a job does not depend on how its paths are shared out, so each imag
 the bit the plain form's, whose grids cover the queue (one tile a work-group, nothing claimed).
 With 64 work-items a group and one group a compute unit the grid is 64 x (compute units)
 entries wide; the sizes lie around one grid, a few grids, and a single entry.
+
+A pass starts its pixels by 8 x 8 tiles, narrower at the right and lower at the bottom edge; images
+of less than a tile, of one, and with every kind of edge equal the oracle's sample for sample (its
+paths differ from the device's where a sqrt or a sine rounds differently: the bound of the
+engine's other oracle tests).
 """
 import numpy as np
 import pytest
 
 import little_renderer_amd as lr
+from oracle import lro
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -51,3 +57,20 @@ def test_batched_equals_plain_at_the_grid_s_edges(world, grids, off, tile):
     assert np.array_equal(got, want)
     assert np.any(got[..., :3])
     eng.close()
+
+
+@pytest.mark.parametrize("w, h", [(1, 1), (3, 65), (7, 9), (8, 8), (9, 7), (65, 3), (24, 20)])
+def test_ragged_images_match_the_oracle(world, w, h):
+    ctx, _ = world
+    sc = lr.cornell(w, h)
+    ps = lr.PtScene(ctx, sc["prims"], sc["tris"], sc["mats"], 0, sc["eps"], sc["margin"])
+    eng = lr.Engine(ctx, slots_log2=14, max_tree_depth=64, image_bytes=16 << 20)
+    i = eng.submit(lr.make_job(ps, sc["cam"], w, h, 3, seed=2))
+    eng.drain()
+    got = image(eng, i, w, h).view(np.float32)
+    assert np.all(got[..., 3] == 3)
+    want = lro.pt_image(sc, w, h, 0, 3, seed=2, tab=lr.brdf_tables(), mask=lro.blue_noise())
+    rel = np.abs(got[..., :3] - want) / np.maximum(np.abs(want), 1e-3)
+    assert np.median(rel) < 1e-5 and np.mean(rel > 1e-3) < 0.01
+    eng.close()
+    ps.close()
