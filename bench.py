@@ -476,7 +476,7 @@ def bench_batched(a, torch, lr):
     nodes = c1.node_fetches - c0.node_fetches
     shapes = c1.shape_tests - c0.shape_tests
     rext = c1.rays_ext - c0.rays_ext
-    alg = rf.walk_bytes(rext, nodes, shapes, rf.NODE_BYTES_WIDE)
+    alg = rf.walk_bytes(rext, nodes, shapes, rf.SLOT_BYTES, rf.SLOT_BYTES)
     dom = max(kms, key=kms.get)
     achieved = alg / (kms["extend"] * 1e-3) / 1e9
     traffic, traffic_detail = (None, {"why": "--no-traffic"}) if a.no_traffic else live_traffic(a, tune)
@@ -605,7 +605,7 @@ def bench_caustics(a, torch, lr):
     eng.counting(False)
     lrays = (c1.light_rays - c0.light_rays) + (c1.light_shadow_rays - c0.light_shadow_rays)
     lnodes, lshapes = c1.light_node_fetches - c0.light_node_fetches, c1.light_shape_tests - c0.light_shape_tests
-    alg = rf.walk_bytes(lrays, lnodes, lshapes, rf.NODE_BYTES_WIDE)
+    alg = rf.walk_bytes(lrays, lnodes, lshapes, rf.SLOT_BYTES, rf.SLOT_BYTES)
     achieved = alg / (kms["light"] * 1e-3) / 1e9 if kms["light"] > 0 else 0.0
     if a.no_traffic:
         traffic, traffic_detail = None, {"why": "--no-traffic"}
@@ -898,7 +898,7 @@ def bench_instanced(a, torch, lr):
     c1 = eng.stats()
     eng.counting(False)
     nodes, shapes, rext = c1.node_fetches - c0.node_fetches, c1.shape_tests - c0.shape_tests, c1.rays_ext - c0.rays_ext
-    alg = rf.walk_bytes(rext, nodes, shapes, rf.NODE_BYTES_WIDE)
+    alg = rf.walk_bytes(rext, nodes, shapes, rf.SLOT_BYTES, rf.SLOT_BYTES)
     achieved = alg / (kms["extend"] * 1e-3) / 1e9
     ninst = len(w0["instances"])
     out = {
@@ -960,7 +960,7 @@ def walk_counts(c0, c1, kms, kl):
     d = lambda f: getattr(c1, f) - getattr(c0, f)
     share = lambda a, b: round(a / (64.0 * b), 4) if b else None
     srays, snodes, sshapes = d("rays_shadow"), d("shadow_node_fetches"), d("shadow_shape_tests")
-    salg = rf.walk_bytes(srays, snodes, sshapes, rf.NODE_BYTES_WIDE)
+    salg = rf.walk_bytes(srays, snodes, sshapes, rf.SLOT_BYTES, rf.SLOT_BYTES)
     sach = salg / (kms["shadow"] * 1e-3) / 1e9 if kms["shadow"] > 0 else 0.0
     return {
         "shadow_roofline": {"bound": "hbm", "kernel": "shadow", "achieved": round(sach, 2), "peak": HBM_PEAK_GBS,

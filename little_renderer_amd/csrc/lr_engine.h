@@ -32,17 +32,14 @@
 // one job on the device (written by a kernel with the descriptor as its argument, so the
 // host's copy is never read late)
 struct JobDev {
-    const float4 *nodes;      // 4-wide nodes (walk4); a two-level scene: its top level, 4-wide (walk4_tl)
-    const float4 *bnodes;     // a two-level scene's top level as binary records (k_child_boxes; not walked now)
-    const uint32_t *aux;
+    const float4 *slots;      // the 4-wide tree (walk4's slots); a two-level scene: its top level's (walk4_tl)
     const float4 *tris;
-    const float4 *ltris;      // the triangles again, in leaf order: ltris[3 e..] for aux entry e (the walks)
     const float4 *prims;
     const float4 *mats;       // 3 float4 per material: albedo.rgb type | emission.rgb ior | metallic roughness transmission 0
     long long *accum;         // 3 x int64 per pixel, fixed point
     unsigned long long total; // w * h * spp
     float cam[12];
-    uint32_t root, nprims;
+    uint32_t nprims;
     int W, H, npix, light;
     int max_depth, mis;
     uint32_t s0, seed_lo, seed_hi;
@@ -51,13 +48,10 @@ struct JobDev {
     const float *env_rgb, *env_marg, *env_cond, *env_prob;
     int env_w, env_h;
     float env_scale, env_rot, env_rot_c, env_rot_s;
-    // a two-level scene: nodes/bnodes/aux above are the top level over the instances (aux:
-    // instance ids); the meshes' binary records, 4-wide nodes and aux (global triangle ids into
-    // tris; ltris then holds the meshes' triangles in maux order); per instance 4 float4: world
-    // -> object rows, then (kind, material, mesh root record, mesh root wide slot) as u32
-    const float4 *mnodes;
-    const float4 *mnodes4;
-    const uint32_t *maux;
+    // a two-level scene: slots above is the top level over the instances; the meshes' slots (their
+    // leaves' shape ids: global triangle ids into tris); per instance 4 float4: world -> object
+    // rows, then (kind, material, mesh root record, mesh root entry) as u32
+    const float4 *mslots;
     const float4 *inst;
     int two_level;
     // the glowing shapes sampled as lights (Scene.emitters): 5 float4 each, (centre, ball 1/0 |
@@ -93,17 +87,13 @@ struct JobDev {
 #define LR_MOM2_CAP 1099511627776.0f      // a square saturated at 2^40
 #define LR_MAX_EMITTERS 16
 
-// the compressed 4-wide nodes' leaf references hold a first aux entry in 24 bits (all ones is
-// kept free: a two-level walk's leaf entry then never equals its EXIT entry)
+// the most shapes (or mesh triangles, or instances) of a scene
 #define LR_WIDE_MAX_SHAPES ((1 << 24) - 1)
 
 // instance kinds on the device: a mesh index, or these (trace.wgsl:188-190)
 #define LR_UNIT_SPHERE 0xfffffff0u
 #define LR_UNIT_BOX 0xfffffff1u
-// stack entries of the two-level walks: a top-level node k (< 2^30), INST | instance, BLAS | node
-// (and, in the 4-wide walk, a mesh leaf: 0xc0000000 | (count - 1) << 24 | first maux entry)
-#define LR_WALK_INST 0x40000000u
-#define LR_WALK_BLAS 0x80000000u
+// the two-level walks' stack mark: the entries above it are the entered instance's mesh's
 #define LR_WALK_EXIT 0xffffffffu
 
 enum { K_EXTEND = 0, K_SHADE = 1, K_SHADOW = 2 };
@@ -209,9 +199,7 @@ struct LrhPtScene {
     LrhContext *ctx;
     float4 *prims = nullptr, *tris = nullptr, *mats = nullptr, *boxes = nullptr;
     uint32_t *nodes = nullptr, *aux = nullptr;
-    float4 *wnodes = nullptr;                 // a two-level scene's top level as binary records (k_child_boxes)
-    float4 *w4nodes = nullptr;                // the same tree, 4-wide (walk4)
-    float4 *ltris = nullptr;                  // the triangles in leaf order (zeros at primitives' entries)
+    float4 *slots = nullptr;                  // the same tree, 4-wide (walk4's slots; a two-level scene: its top level's)
     // the sky
     float *env_rgb = nullptr, *env_marg = nullptr, *env_cond = nullptr, *env_prob = nullptr;
     int env_w = 0, env_h = 0;
@@ -222,14 +210,13 @@ struct LrhPtScene {
     uint32_t *tparent = nullptr, *tarrive = nullptr;   // the top level's records' parents; refit arrivals
     double *tcost_dev = nullptr;              // a cost computed on the device
     double tcost_build = 0.0;                 // the top level's cost at its last build (the refit rule's)
-    float4 *mtris = nullptr, *mboxes = nullptr, *mwnodes = nullptr, *inst = nullptr, *ifwd = nullptr;
-    float4 *mw4nodes = nullptr, *tw4nodes = nullptr;   // the meshes' and the top level's 4-wide nodes
-    uint32_t *mroot4 = nullptr;                        // each mesh's root wide slot
+    float4 *mboxes = nullptr, *inst = nullptr, *ifwd = nullptr;
+    float4 *mslots = nullptr;                 // the meshes' slots (mesh m's from slot 2 mesh_first[m] on)
     uint32_t *mnodes = nullptr, *maux = nullptr, *mroot = nullptr;
     float4 *tboxes = nullptr;
     uint32_t *tnodes = nullptr, *taux = nullptr;
     // host copies of the meshes' layout: first triangle (nmeshes + 1 of them), root record,
-    // root wide slot and tree depth of each mesh
+    // root entry and tree depth of each mesh
     std::vector<int> mfirst, mdepth;
     std::vector<uint32_t> mroot_h, mroot4_h;
     float *tab = nullptr;

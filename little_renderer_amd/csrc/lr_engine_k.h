@@ -257,13 +257,12 @@ __device__ __forceinline__ V3 unit_box_normal(V3 p)
     return v3(0.0f, 0.0f, p.z < 0.0f ? -1.0f : 1.0f);
 }
 
-// The closest (ANY: the first) hit in a two-level scene, on the 4-wide trees (walk4's compressed
-// nodes, one entry at a time): the top level's wide nodes, whose leaf references hold
-// instances, and each mesh's. A mesh instance is entered (the ray taken to its space, EXIT
-// pushed under its mesh's root); the hit's b1 carries the instance (as u32). A node's children hit are
-// sorted by their boxes' entry distance, whatever they are (a node, a mesh's leaf, an instance
-// to enter), so all are visited near to far; unit spheres and boxes are tested on the spot. A
-// mesh's triangles are read in leaf order (ltris) beside their aux entries.
+// The closest (ANY: the first) hit in a two-level scene, on the 4-wide trees (walk4's slots, one
+// entry at a time): the top level's, whose leaves are instances, and each mesh's. A mesh instance
+// is entered: the ray taken to its space, EXIT stacked under its mesh's entries; the hit's b1
+// carries the instance (as u32). Which array an entry belongs to is the lane's state (the instance it
+// is in, if any), so entries carry no tags and EXIT is met only on popping. Unit spheres and boxes
+// are tested on the spot.
 template <bool ANY, bool COUNT, int STK>
 __device__ WalkHit walk4_tl(const JobDev &J, V3 o, V3 d, float tmin, float tmax, const WalkStack &S, uint32_t *overflow,
                             WalkCnt &c)
@@ -272,133 +271,69 @@ __device__ WalkHit walk4_tl(const JobDev &J, V3 o, V3 d, float tmin, float tmax,
     // direction is computed again on leaving an instance rather than held
     V3 ro = o, rd = d;
     V3 inv = v3(safe_inv(d.x), safe_inv(d.y), safe_inv(d.z));
-    V3 oi = v3(o.x * inv.x, o.y * inv.y, o.z * inv.z);
-    uint32_t cur = LR_NONE;
+    uint32_t in = LR_NONE;   // the instance the ray is in
     WalkHit best{tmax, LR_NONE, __uint_as_float(LR_NONE), 0.0f};
     int sp = 0;
-    auto push = [&](uint32_t x) {
-        if (sp < STK) S.stk[sp * S.stride] = x;
-        else S.spill[(size_t)(sp - STK) * S.sstride] = x;
-        sp++;
-    };
-    auto pop = [&](uint32_t &x) -> bool {
-        if (sp == 0) return false;
-        sp--;
-        x = stk_get<STK>(S, sp);
-        return true;
-    };
-    // the entry being visited: a top-level node k, INST | i, BLAS | mesh node, MLEAF | (count -
-    // 1) << 24 | first maux entry, EXIT
-    constexpr uint32_t MLEAF = 0xc0000000u;
-    uint32_t e = 0u;
+    uint32_t cur = 0u;
     for (;;) {
-        if (e == LR_WALK_EXIT) {
-            cur = LR_NONE;
-            ro = o;
-            rd = d;
-            inv = v3(safe_inv(d.x), safe_inv(d.y), safe_inv(d.z));
-            oi = v3(o.x * inv.x, o.y * inv.y, o.z * inv.z);
-            if (!pop(e)) break;
-            continue;
-        }
-        const uint32_t tag = e & 0xc0000000u;
-        if (tag == LR_WALK_INST) {
-            const uint32_t i = e & 0x3fffffffu;
-            const uint32_t kind = __float_as_uint(J.inst[4 * (size_t)i + 3].x);
-            if (kind >= LR_UNIT_SPHERE) {   // a unit sphere or box: tested in its space, the ray kept
+        const float4 *p = slot_at(in == LR_NONE ? J.slots : J.mslots, cur);
+        const float4 r0 = ldg4(p, 0), r1 = ldg4(p, 1), r2 = ldg4(p, 2);
+        bool more;
+        if (__float_as_uint(r0.w) & LR_LEAF) {
+            const uint32_t id = __float_as_uint(r1.w);
+            more = false;
+            if (in != LR_NONE) {   // a mesh's triangle, in the instance's space
                 if (COUNT) count_shape(c);
+                float t, u, v;
+                if (hit_tri(r0, r1, r2, ro, rd, tmin, best.t, t, u, v)) {
+                    best = WalkHit{t, id, __uint_as_float(in), 0.0f};
+                    if (ANY) return best;
+                }
+            } else {
+                const uint32_t kind = __float_as_uint(r0.x);
                 V3 oo, od;
-                to_object(J.inst + 4 * (size_t)i, o, d, oo, od);
-                const float th = kind == LR_UNIT_SPHERE ? hit_unit_sphere(oo, od, tmin, best.t) : hit_unit_box(oo, od, tmin, best.t);
-                if (th > 0.0f) {
-                    best = WalkHit{th, kind, __uint_as_float(i), 0.0f};
-                    if (ANY) return best;
-                }
-                if (!pop(e)) break;
-                continue;
-            }
-            to_object(J.inst + 4 * (size_t)i, o, d, ro, rd);
-            inv = v3(safe_inv(rd.x), safe_inv(rd.y), safe_inv(rd.z));
-            oi = v3(ro.x * inv.x, ro.y * inv.y, ro.z * inv.z);
-            cur = i;
-            if (sp + 1 > S.cap) {   // cannot happen with a correct depth: said, never silently dropped
-                atomicOr(overflow, 1u);
-                break;
-            }
-            push(LR_WALK_EXIT);
-            e = LR_WALK_BLAS | __float_as_uint(J.inst[4 * (size_t)i + 3].w);
-            continue;
-        }
-        if (tag == MLEAF) {   // a mesh's leaf, in the instance's space
-            const uint32_t cnt = ((e >> 24) & 0x3fu) + 1u, first = e & 0xffffffu;
-            for (uint32_t j = 0; j < cnt; j++) {
-                if (COUNT) count_shape(c);
-                const uint32_t x = first + j;
-                const uint32_t sid = J.maux[x];
-                const float4 ta = J.ltris[3 * (size_t)x], tb = J.ltris[3 * (size_t)x + 1], tc = J.ltris[3 * (size_t)x + 2];
-                float th, u, v;
-                if (hit_tri(ta, tb, tc, ro, rd, tmin, best.t, th, u, v)) {
-                    best = WalkHit{th, sid, __uint_as_float(cur), 0.0f};
-                    if (ANY) return best;
+                to_object(J.inst + 4 * (size_t)id, o, d, oo, od);
+                if (kind >= LR_UNIT_SPHERE) {   // a unit sphere or box: tested in its space, the ray kept
+                    if (COUNT) count_shape(c);
+                    const float t = kind == LR_UNIT_SPHERE ? hit_unit_sphere(oo, od, tmin, best.t) : hit_unit_box(oo, od, tmin, best.t);
+                    if (t > 0.0f) {
+                        best = WalkHit{t, kind, __uint_as_float(id), 0.0f};
+                        if (ANY) return best;
+                    }
+                } else if (sp >= S.cap) {   // cannot happen with a correct depth: said, never silently dropped
+                    atomicOr(overflow, 1u);
+                } else {
+                    if (sp < STK) S.stk[sp * S.stride] = LR_WALK_EXIT;
+                    else S.spill[(size_t)(sp - STK) * S.sstride] = LR_WALK_EXIT;
+                    sp++;
+                    ro = oo;
+                    rd = od;
+                    inv = v3(safe_inv(rd.x), safe_inv(rd.y), safe_inv(rd.z));
+                    in = id;
+                    cur = __float_as_uint(r0.y);
+                    more = true;
                 }
             }
-            if (!pop(e)) break;
-            continue;
+        } else {
+            if (COUNT) count_node(c);
+            uint32_t key[4];
+            wide_keys(r0, r1, r2, ro, inv, tmin, best.t, key);
+            more = wide_next<STK>(key, __float_as_uint(r1.w), S, sp, cur, overflow);
         }
-        const bool blas = tag == LR_WALK_BLAS;
-        if (COUNT) count_node(c);
-        float t[4];
-        uint32_t ref[4];
-        wide_test(blas ? J.mnodes4 : J.nodes, e & 0x3fffffffu, oi, inv, tmin, best.t, t, ref);
-        float s[4] = {3e38f, 3e38f, 3e38f, 3e38f};
-        uint32_t c[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (!(t[k] < 3e38f)) continue;
-            if (!(ref[k] & LR_LEAF)) {
-                c[k] = (blas ? LR_WALK_BLAS : 0u) | ref[k];
-                s[k] = t[k];
-                continue;
+        if (!more) {
+            if (sp == 0) break;
+            sp--;
+            cur = stk_get<STK>(S, sp);
+            if (cur == LR_WALK_EXIT) {   // out of the instance (its EXIT has a top-level entry under it, or nothing)
+                in = LR_NONE;
+                ro = o;
+                rd = d;
+                inv = v3(safe_inv(d.x), safe_inv(d.y), safe_inv(d.z));
+                if (sp == 0) break;
+                sp--;
+                cur = stk_get<STK>(S, sp);
             }
-            if (blas) {
-                c[k] = MLEAF | (ref[k] & 0x3fffffffu);
-                s[k] = t[k];
-                continue;
-            }
-            // a top-level leaf: its instances, entries (one leaf, one instance: sorted with the rest)
-            const uint32_t cnt = ((ref[k] >> 24) & 0x3fu) + 1u, first = ref[k] & 0xffffffu;
-            if (cnt == 1) {
-                c[k] = LR_WALK_INST | J.aux[first];
-                s[k] = t[k];
-                continue;
-            }
-            if (sp + cnt > (uint32_t)S.cap) {   // cannot happen with a correct depth: said, never silently dropped
-                atomicOr(overflow, 1u);
-                return best;
-            }
-            for (uint32_t j = 0; j < cnt; j++) push(LR_WALK_INST | J.aux[first + j]);
         }
-        // nearest first
-        float s0 = s[0], s1 = s[1], s2 = s[2], s3 = s[3];
-        uint32_t c0 = c[0], c1 = c[1], c2 = c[2], c3 = c[3];
-        cswap_(s0, c0, s1, c1);
-        cswap_(s2, c2, s3, c3);
-        cswap_(s0, c0, s2, c2);
-        cswap_(s1, c1, s3, c3);
-        cswap_(s1, c1, s2, c2);
-        const int m = (s0 < 3e38f) + (s1 < 3e38f) + (s2 < 3e38f) + (s3 < 3e38f);
-        if (m == 0) {
-            if (!pop(e)) break;
-            continue;
-        }
-        if (sp + m - 1 > S.cap) {   // cannot happen with a correct depth: said, never silently dropped
-            atomicOr(overflow, 1u);
-            break;
-        }
-        if (m > 3) push(c3);
-        if (m > 2) push(c2);
-        if (m > 1) push(c1);
-        e = c0;
     }
     return best;
 }
@@ -500,9 +435,9 @@ __device__ __forceinline__ void add_counts(unsigned long long *c, unsigned long 
 // is part of the queue's length until the shadow kernel ends the iteration), and clears
 // the queues the shade kernel appends to. TL: two-level scenes may be queued (without it, such
 // a ray is not walked: flagged, so that the host reports it).
-// Without TL the kernel is held to 64 VGPRs, 8 waves per SIMD: a few registers spill (12 bytes a
-// lane), and the walk, bound by the latency of its node fetches, gains more from the waves (the
-// whole persistent grid of 8 work-groups per compute unit is then resident).
+// Without TL the kernel is held to 64 VGPRs, 8 waves per SIMD (the walk's own 63; the shadow walk
+// spills 12 bytes a lane), so that the whole persistent grid of 8 work-groups per compute unit is
+// resident.
 // waves per SIMD a walk kernel is held to: 8, or fewer where its LDS stack (160 KB per compute
 // unit) allows fewer anyway
 constexpr int walk_waves(int blk, int stk)
@@ -539,7 +474,7 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_extend(E
         WalkHit h;
         if (TL && J.two_level) h = walk4_tl<false, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
         else if (!J.two_level)
-            h = walk4<false, COUNT, STK>(J.nodes, J.aux, J.ltris, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S,
+            h = walk4<false, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S,
                                          A.overflow, wc);
         else {
             atomicOr(A.overflow, 2u);
@@ -551,8 +486,7 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_extend(E
 }
 
 // ---- walks with lanes refilled (dynamic fetch, Aila & Laine 2009) ----------------------------
-// A wave walks its lanes' rays one round at a time (the leaves a lane holds, then one node step:
-// walk4's loop body), and once at least A.refill of its 64 lanes have finished, those take the
+// A wave walks its lanes' rays one round at a time (walk4's step: an entry a lane), and once at least A.refill of its 64 lanes have finished, those take the
 // next entries of the queue: a wave does not run on for its slowest ray with most of its lanes
 // idle. A wave claims the queue 64 entries at a time (the kernel's counter then counts entries,
 // not tiles) and hands them to its idle lanes in order. The walk is walk4's (the same visits in
@@ -561,13 +495,12 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_extend(E
 
 // a lane's walk between rounds
 struct WalkState {
-    V3 o, d, inv;   // (o * inv, the slab test's other term, made again each node step: fewer registers held)
+    V3 o, d, inv;
     float tmin;
     WalkHit best;
     int sp;
     uint32_t cur;
-    const float4 *nodes, *ltris, *prims;
-    const uint32_t *aux;
+    const float4 *slots, *prims;
     uint32_t nprims;
 };
 
@@ -580,60 +513,16 @@ __device__ __forceinline__ void walk_start(WalkState &w, const JobDev &J, float4
     w.best = WalkHit{r1.w, LR_NONE, 0.0f, 0.0f};
     w.sp = 0;
     w.cur = 0u;
-    w.nodes = J.nodes;
-    w.aux = J.aux;
-    w.ltris = J.ltris;
+    w.slots = J.slots;
     w.prims = J.prims;
     w.nprims = J.nprims;
 }
 
-// one round of walk4 (ANY: the first hit ends it); true when the walk has ended (w.best its hit)
+// one step of walk4 (ANY: the first hit ends it); true when the walk has ended (w.best its hit)
 template <bool ANY, bool COUNT, int STK>
 __device__ __forceinline__ bool walk_round(WalkState &w, const WalkStack &S, uint32_t *overflow, WalkCnt &wc)
 {
-    while (w.cur & LR_LEAF) {
-        bool done = false;
-        leaf_hits_(w.aux, w.ltris, w.prims, w.nprims, w.cur & 0xffffffu, ((w.cur >> 24) & 0x3fu) + 1u, w.o, w.d, w.tmin, w.best,
-                   ANY, done, wc, COUNT);
-        if ((ANY && done) || w.sp == 0) return true;
-        w.sp--;
-        w.cur = stk_get<STK>(S, w.sp);
-    }
-    if (COUNT) {
-        count_node(wc);
-        count_uniform(wc, w.nodes, w.cur);
-    }
-    float t[4];
-    uint32_t ref[4];
-    wide_test(w.nodes, w.cur, v3(w.o.x * w.inv.x, w.o.y * w.inv.y, w.o.z * w.inv.z), w.inv, w.tmin, w.best.t, t, ref);
-    const int m = (t[0] < 3e38f) + (t[1] < 3e38f) + (t[2] < 3e38f) + (t[3] < 3e38f);
-    float s0 = t[0], s1 = t[1], s2 = t[2], s3 = t[3];
-    uint32_t c0 = ref[0], c1 = ref[1], c2 = ref[2], c3 = ref[3];
-    cswap_(s0, c0, s1, c1);
-    cswap_(s2, c2, s3, c3);
-    cswap_(s0, c0, s2, c2);
-    cswap_(s1, c1, s3, c3);
-    cswap_(s1, c1, s2, c2);
-    if (m == 0) {
-        if (w.sp == 0) return true;
-        w.sp--;
-        w.cur = stk_get<STK>(S, w.sp);
-        return false;
-    }
-    if (w.sp + m - 1 > S.cap) {   // cannot happen with a correct depth: said, never silently dropped
-        atomicOr(overflow, 1u);
-        return true;
-    }
-    auto push = [&](uint32_t x) {
-        if (w.sp < STK) S.stk[w.sp * S.stride] = x;
-        else S.spill[(size_t)(w.sp - STK) * S.sstride] = x;
-        w.sp++;
-    };
-    if (m > 3) push(c3);
-    if (m > 2) push(c2);
-    if (m > 1) push(c1);
-    w.cur = c0;
-    return false;
+    return !walk4_step<ANY, COUNT, STK>(w.slots, w.prims, w.nprims, w.o, w.d, w.inv, w.tmin, w.best, w.sp, w.cur, S, overflow, wc);
 }
 
 // a wave's claimed queue entries not yet handed out, [rb, re), and whether the counter may still
@@ -1193,7 +1082,7 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_shadow(E
                 WalkHit h;
                 if (TL && J.two_level) h = walk4_tl<true, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
                 else if (!J.two_level)
-                    h = walk4<true, COUNT, STK>(J.nodes, J.aux, J.ltris, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S,
+                    h = walk4<true, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S,
                                                 A.overflow, wc);
                 else {
                     atomicOr(A.overflow, 2u);
@@ -1225,7 +1114,7 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_shadow(E
                     WalkHit h;
                     if (TL && J.two_level) h = walk4_tl<true, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
                     else if (!J.two_level)
-                        h = walk4<true, COUNT, STK>(J.nodes, J.aux, J.ltris, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S,
+                        h = walk4<true, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S,
                                                     A.overflow, wc);
                     else {
                         atomicOr(A.overflow, 2u);
@@ -1287,7 +1176,7 @@ __global__ __launch_bounds__(BLK) void k_guide(JobDev J, float4 *guide, uint32_t
             WalkCnt wc;
             WalkHit h;
             if (TL && J.two_level) h = walk4_tl<false, false, STK>(J, o, d, J.eps, 1e30f, S, overflow, wc);
-            else h = walk4<false, false, STK>(J.nodes, J.aux, J.ltris, J.prims, J.nprims, o, d, J.eps, 1e30f, S, overflow, wc);
+            else h = walk4<false, false, STK>(J.slots, J.prims, J.nprims, o, d, J.eps, 1e30f, S, overflow, wc);
             if (h.id == LR_NONE) break;
             const V3 hp = vadd(o, vscale(d, h.t));
             V3 outward;
@@ -1498,7 +1387,7 @@ __device__ __forceinline__ bool light_vertex(const JobDev &J, const LightCtx &L,
                                              uint32_t &n_shadow, PcLds *pl)
 {
     const uint64_t inc = ((uint64_t)P.path << 1u) | 1u;
-    const WalkHit h = walk4<false, COUNT, STK>(J.nodes, J.aux, J.ltris, J.prims, J.nprims, P.o, P.d, J.eps, 1e30f, S,
+    const WalkHit h = walk4<false, COUNT, STK>(J.slots, J.prims, J.nprims, P.o, P.d, J.eps, 1e30f, S,
                                                overflow, wc);
     n_ext++;
     if (h.id == LR_NONE) return false;
@@ -1539,7 +1428,7 @@ __device__ __forceinline__ bool light_vertex(const JobDev &J, const LightCtx &L,
             if (sx >= 0.0f && sy >= 0.0f && sx < 1.0f && sy < 1.0f) {
                 const int px = (int)(sx * (float)J.W), py = (int)(sy * (float)J.H);
                 if (px < J.W && py < J.H) {
-                    const WalkHit sh = walk4<true, COUNT, STK>(J.nodes, J.aux, J.ltris, J.prims, J.nprims, hp, wo, J.eps,
+                    const WalkHit sh = walk4<true, COUNT, STK>(J.slots, J.prims, J.nprims, hp, wo, J.eps,
                                                                dist * (1.0f - 1e-4f), S, overflow, wc);
                     n_shadow++;
                     if (sh.id == LR_NONE) {

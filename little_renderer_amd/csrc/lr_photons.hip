@@ -86,7 +86,7 @@ __global__ __launch_bounds__(PC_BLK) void k_pc_resolve(JobDev J, const unsigned 
         const V3 d = vnorm(vsub(vsub(vadd(ul, vscale(hz, u)), vscale(vt, v)), org));
         float4 res = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         WalkCnt wc;
-        const WalkHit h = walk4<false, false, PC_STK>(J.nodes, J.aux, J.ltris, J.prims, J.nprims, org, d, J.eps, 1e30f, S,
+        const WalkHit h = walk4<false, false, PC_STK>(J.slots, J.prims, J.nprims, org, d, J.eps, 1e30f, S,
                                                       overflow, wc);
         if (h.id != LR_NONE) {
             const V3 hp = vadd(org, vscale(d, h.t));

@@ -8,61 +8,6 @@
 #include "lr_device.h"
 #include "lr_engine_k.h"
 
-// Binary records with both children's boxes in the parent: for each inner node of the reference
-// layout, both children's boxes and (index | leaf record); a one-shape tree (its root a leaf)
-// gets a record whose left child is that leaf and whose right child is an empty leaf. Made for
-// the two-level scenes' top level and meshes (JobDev bnodes, mnodes); no walk reads them now.
-__global__ __launch_bounds__(256) void k_child_boxes(const float4 *__restrict__ nodes, int i0, int nn, float4 *__restrict__ w)
-{
-    const int i = i0 + (int)(blockIdx.x * 256 + threadIdx.x);   // records i0 .. i0 + nn - 1
-    if (i >= i0 + nn) return;
-    const float4 lo = nodes[2 * (size_t)i], hi = nodes[2 * (size_t)i + 1];
-    const uint32_t b = __float_as_uint(hi.w);
-    if (b & LR_LEAF) return;
-    const uint32_t c[2] = {__float_as_uint(lo.w), b};
-    for (int k = 0; k < 2; k++) {
-        float4 clo = nodes[2 * (size_t)c[k]], chi = nodes[2 * (size_t)c[k] + 1];
-        if (!(__float_as_uint(chi.w) & LR_LEAF)) {
-            clo.w = __uint_as_float(c[k]);
-            chi.w = __uint_as_float(0u);
-        }
-        w[4 * (size_t)i + 2 * k] = clo;
-        w[4 * (size_t)i + 2 * k + 1] = chi;
-    }
-}
-
-// The triangles in leaf order: entry e of aux names shape aux[e]; a triangle's 48 bytes go to
-// ltris[3 e..], a primitive's entry gets zeros (the walks test primitives from prims).
-__global__ __launch_bounds__(256) void k_leaf_tris(const uint32_t *__restrict__ aux, int n, uint32_t nprims,
-                                                   const float4 *__restrict__ tris, float4 *__restrict__ ltris)
-{
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= n) return;
-    const uint32_t sid = aux[e];
-    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a, c = a;
-    if (sid >= nprims) {
-        const size_t t = sid - nprims;
-        a = tris[3 * t];
-        b = tris[3 * t + 1];
-        c = tris[3 * t + 2];
-    }
-    ltris[3 * (size_t)e] = a;
-    ltris[3 * (size_t)e + 1] = b;
-    ltris[3 * (size_t)e + 2] = c;
-}
-
-// A tree whose root is a leaf (one shape) gets a record with that leaf on the left and an
-// empty leaf on the right.
-__global__ void k_root_leaf(const float4 *__restrict__ nodes, uint32_t r, float4 *__restrict__ w)
-{
-    const float4 lo = nodes[2 * (size_t)r], hi = nodes[2 * (size_t)r + 1];
-    if (!(__float_as_uint(hi.w) & LR_LEAF)) return;
-    w[4 * (size_t)r] = lo;
-    w[4 * (size_t)r + 1] = hi;
-    w[4 * (size_t)r + 2] = lo;
-    w[4 * (size_t)r + 3] = make_float4(hi.x, hi.y, hi.z, __uint_as_float(LR_LEAF));
-}
-
 // Each instance's world box: the 8 corners of its object box (its mesh's root box, or [-1, 1]^3)
 // moved to the world, padded by a little more than their rounding.
 __global__ __launch_bounds__(256) void k_inst_boxes(const float4 *__restrict__ fwd, const float4 *__restrict__ inst,
@@ -104,19 +49,45 @@ __global__ __launch_bounds__(256) void k_inst_boxes(const float4 *__restrict__ f
 }
 
 // ---- the 4-wide tree (bvh_make_wide / collapse, engine/rt/bvh.c:487-539): level by level, one
-// wide node per thread. The children are chosen as the reference chooses them; the node is
-// stored compressed (64 bytes instead of put_wide's four 32-byte slots, trace_gpu.c:867-881):
-//   float4 0: the node's box corner lo.xyz, then the three axes' scale exponents (8 bits each,
-//             biased by 127: the scale is 2^(e - 127))
-//   float4 1: the four children's references: a wide node's index; a leaf 0x80000000 |
-//             (count - 1) << 24 | its first aux entry; no child LR_NONE
-//   float4 2: the children's lo.x, lo.y, lo.z, hi.x as 8-bit steps from the corner (byte k:
-//             child k), float4 3: hi.y, hi.z, 0, 0
-// Each child's box is rounded outwards to the steps (lo down, hi up, in exact arithmetic), so it
+// inner slot per thread (walk4's 48-byte slots, lr_walk.h, instead of put_wide's four 32-byte ones,
+// trace_gpu.c:867-881). The children are chosen as the reference chooses them; a node's children's
+// slots are taken side by side, its leaves written at once and its inner children left to the next
+// level's queue. A tree of n leaves and W inner nodes takes n + W <= 2 n - 1 slots.
+// Each child's box is rounded outwards to the node's steps (lo down, hi up, in exact arithmetic), so it
 // holds the child's own box: the walk visits a few more nodes, never misses a hit. ----
 struct WideTask {
-    uint32_t node, wide;   // the binary node the wide node stands for, its index
+    uint32_t node, slot;   // the binary node an inner slot stands for, the slot
 };
+
+// what a tree's leaves are: the shapes of a scene or a mesh (ids below nprims primitives, the rest
+// triangles of tris), or (inst given) the instances of a top level
+struct WideLeaves {
+    const uint32_t *aux;
+    const float4 *tris, *inst;
+    uint32_t nprims;
+};
+
+// the leaf over aux entry e (the builders' leaves hold one shape each) into a slot
+__device__ __forceinline__ void put_leaf(const WideLeaves &L, uint32_t e, float4 *slot)
+{
+    const uint32_t id = L.aux[e];
+    const float tag = __uint_as_float(LR_LEAF), idf = __uint_as_float(id);
+    float4 a = make_float4(0.0f, 0.0f, 0.0f, tag), b = make_float4(0.0f, 0.0f, 0.0f, idf), c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (L.inst) {
+        const float4 info = L.inst[4 * (size_t)id + 3];
+        a.x = info.x;   // the kind
+        a.y = info.w;   // its mesh's root entry
+    } else if (id >= L.nprims) {
+        const size_t t = id - L.nprims;
+        const float4 q = L.tris[3 * t], u = L.tris[3 * t + 1], v = L.tris[3 * t + 2];
+        a = make_float4(q.x, q.y, q.z, tag);
+        b = make_float4(u.x, u.y, u.z, idf);
+        c = make_float4(v.x, v.y, v.z, 0.0f);
+    }
+    slot[0] = a;
+    slot[1] = b;
+    slot[2] = c;
+}
 
 __device__ __forceinline__ float node_area(const float4 *nodes, uint32_t i)   // box_area (bvh.c:30-34), halved
 {
@@ -126,29 +97,31 @@ __device__ __forceinline__ float node_area(const float4 *nodes, uint32_t i)   //
     return dx * dy + dy * dz + dz * dx;
 }
 
-__global__ void k_collapse_init(WideTask *q0, uint32_t *cnt, int levels, uint32_t *nwide, uint32_t root, uint32_t w0)
+// the queue's first task: the root (none when the root is a leaf, written here)
+__global__ void k_collapse_init(const float4 *__restrict__ nodes, WideTask *q0, uint32_t *cnt, int levels, uint32_t *nslots,
+                                uint32_t root, uint32_t slot0, WideLeaves L, float4 *__restrict__ slots)
 {
     for (int l = 0; l <= levels + 1; l++) cnt[l] = 0;
-    q0[0] = WideTask{root, w0};
+    *nslots = slot0 + 1;
+    if (__float_as_uint(nodes[2 * (size_t)root + 1].w) & LR_LEAF) {
+        put_leaf(L, __float_as_uint(nodes[2 * (size_t)root].w), slots + LR_SLOT_F4 * (size_t)slot0);
+        return;
+    }
+    q0[0] = WideTask{root, slot0};
     cnt[0] = 1;
-    *nwide = w0 + 1;
 }
 
 __global__ __launch_bounds__(256) void k_collapse(const float4 *__restrict__ nodes, const WideTask *__restrict__ qin,
                                                   const uint32_t *cin, WideTask *__restrict__ qout, uint32_t *cout,
-                                                  uint32_t *nwide, float4 *__restrict__ w4)
+                                                  uint32_t *nslots, WideLeaves L, float4 *__restrict__ slots)
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= *cin) return;
     const WideTask e = qin[i];
     uint32_t kids[4];
     int n = 0;
-    const uint32_t rb = __float_as_uint(nodes[2 * (size_t)e.node + 1].w);
-    if (rb & LR_LEAF) kids[n++] = e.node;   // a tree that is one leaf
-    else {
-        kids[n++] = __float_as_uint(nodes[2 * (size_t)e.node].w);
-        kids[n++] = rb;
-    }
+    kids[n++] = __float_as_uint(nodes[2 * (size_t)e.node].w);
+    kids[n++] = __float_as_uint(nodes[2 * (size_t)e.node + 1].w);
     // open the inner child of largest area until there are four (or only leaves)
     while (n < 4) {
         int best = -1;
@@ -180,16 +153,12 @@ __global__ __launch_bounds__(256) void k_collapse(const float4 *__restrict__ nod
         }
         ex[a] = k;
     }
-    uint32_t ref[4] = {LR_NONE, LR_NONE, LR_NONE, LR_NONE}, qlo[3] = {0u, 0u, 0u}, qhi[3] = {0u, 0u, 0u};
+    const uint32_t base = atomicAdd(nslots, (uint32_t)n);
+    uint32_t qlo[3] = {0u, 0u, 0u}, qhi[3] = {0u, 0u, 0u};
     for (int k = 0; k < n; k++) {
         const float4 lo = nodes[2 * (size_t)kids[k]], hi = nodes[2 * (size_t)kids[k] + 1];
-        const uint32_t b = __float_as_uint(hi.w);
-        if (b & LR_LEAF) ref[k] = LR_LEAF | (((b & 0x7fffffffu) - 1u) << 24) | __float_as_uint(lo.w);
-        else {
-            const uint32_t w = atomicAdd(nwide, 1u);
-            qout[atomicAdd(cout, 1u)] = WideTask{kids[k], w};
-            ref[k] = w;
-        }
+        if (__float_as_uint(hi.w) & LR_LEAF) put_leaf(L, __float_as_uint(lo.w), slots + LR_SLOT_F4 * (size_t)(base + k));
+        else qout[atomicAdd(cout, 1u)] = WideTask{kids[k], base + (uint32_t)k};
         const float cl[3] = {lo.x, lo.y, lo.z}, ch[3] = {hi.x, hi.y, hi.z};
         for (int a = 0; a < 3; a++) {
             // steps from the corner, exact in double (a float difference, a power-of-two scale)
@@ -201,17 +170,19 @@ __global__ __launch_bounds__(256) void k_collapse(const float4 *__restrict__ nod
             qhi[a] |= h << (8 * k);
         }
     }
-    const uint32_t eb = (uint32_t)(ex[0] + 127) | ((uint32_t)(ex[1] + 127) << 8) | ((uint32_t)(ex[2] + 127) << 16);
-    float4 *o = w4 + 4 * (size_t)e.wide;
-    o[0] = make_float4(plo.x, plo.y, plo.z, __uint_as_float(eb));
-    o[1] = make_float4(__uint_as_float(ref[0]), __uint_as_float(ref[1]), __uint_as_float(ref[2]), __uint_as_float(ref[3]));
-    o[2] = make_float4(__uint_as_float(qlo[0]), __uint_as_float(qlo[1]), __uint_as_float(qlo[2]), __uint_as_float(qhi[0]));
-    o[3] = make_float4(__uint_as_float(qhi[1]), __uint_as_float(qhi[2]), 0.0f, 0.0f);
+    const uint32_t w = ((uint32_t)ex[0] & 0xffu) | (((uint32_t)ex[1] & 0xffu) << 8) | (((uint32_t)ex[2] & 0xffu) << 16) |
+                       ((uint32_t)n << 24);
+    float4 *o = slots + LR_SLOT_F4 * (size_t)e.slot;
+    o[0] = make_float4(plo.x, plo.y, plo.z, __uint_as_float(w));
+    o[1] = make_float4(__uint_as_float(qlo[0]), __uint_as_float(qlo[1]), __uint_as_float(qlo[2]),
+                       __uint_as_float(LR_SLOT_F4 * base));
+    o[2] = make_float4(__uint_as_float(qhi[0]), __uint_as_float(qhi[1]), __uint_as_float(qhi[2]), 0.0f);
 }
 
-// the wide tree of a binary tree (root `root`, n items, depth levels) into w4, its wide nodes
-// numbered from w0 (room for n of them from there); waits for it
-static int collapse_wide(LrhContext *c, const uint32_t *nodes, uint32_t root, int n, int depth, float4 *w4, uint32_t w0 = 0)
+// the slots of a binary tree (root `root`, n leaves, depth levels), from slot0 on (room for 2 n of
+// them from there); waits for them
+static int collapse_wide(LrhContext *c, const uint32_t *nodes, uint32_t root, int n, int depth, const WideLeaves &L, float4 *slots,
+                         uint32_t slot0 = 0)
 {
     const size_t qbytes = lr_align((size_t)(n > 1 ? n : 2) * sizeof(WideTask));
     int rc = lr_scratch_reserve(c, LR_SCRATCH_TRACE, 2 * qbytes + lr_align((size_t)(depth + 4) * 4) + 256);
@@ -219,12 +190,13 @@ static int collapse_wide(LrhContext *c, const uint32_t *nodes, uint32_t root, in
     char *base = (char *)c->scratch[LR_SCRATCH_TRACE].base;
     WideTask *q[2] = {(WideTask *)base, (WideTask *)(base + qbytes)};
     uint32_t *cnt = (uint32_t *)(base + 2 * qbytes);
-    uint32_t *nwide = cnt + depth + 3;
-    hipLaunchKernelGGL(k_collapse_init, dim3(1), dim3(1), 0, c->stream, q[0], cnt, depth, nwide, root, w0);
+    uint32_t *nslots = cnt + depth + 3;
+    hipLaunchKernelGGL(k_collapse_init, dim3(1), dim3(1), 0, c->stream, (const float4 *)nodes, q[0], cnt, depth, nslots, root,
+                       slot0, L, slots);
     const dim3 grid((unsigned)((n + 255) / 256));
     for (int l = 0; l <= depth; l++)
         hipLaunchKernelGGL(k_collapse, grid, dim3(256), 0, c->stream, (const float4 *)nodes, (const WideTask *)q[l & 1],
-                           (const uint32_t *)(cnt + l), q[(l + 1) & 1], cnt + l + 1, nwide, w4);
+                           (const uint32_t *)(cnt + l), q[(l + 1) & 1], cnt + l + 1, nslots, L, slots);
     LR_HIP(hipGetLastError());
     LR_HIP(hipStreamSynchronize(c->stream));
     return 0;
@@ -233,9 +205,9 @@ static int collapse_wide(LrhContext *c, const uint32_t *nodes, uint32_t root, in
 static void pt_scene_release(LrhPtScene *s)
 {
     if (!s) return;
-    void *ps[] = {s->prims, s->tris, s->mats, s->boxes, s->nodes, s->aux, s->tab, s->mask, s->wnodes, s->w4nodes, s->ltris, s->env_rgb,
-                  s->env_marg, s->env_cond, s->env_prob, s->mboxes, s->mwnodes, s->inst, s->ifwd, s->mnodes, s->maux,
-                  s->mroot, s->mw4nodes, s->tw4nodes, s->mroot4, s->tparent, s->tarrive, s->tcost_dev, s->emit, s->inst_emit};
+    void *ps[] = {s->prims, s->tris, s->mats, s->boxes, s->nodes, s->aux, s->tab, s->mask, s->slots, s->env_rgb,
+                  s->env_marg, s->env_cond, s->env_prob, s->mboxes, s->inst, s->ifwd, s->mnodes, s->maux,
+                  s->mroot, s->mslots, s->tparent, s->tarrive, s->tcost_dev, s->emit, s->inst_emit};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     delete s;
@@ -272,7 +244,7 @@ extern "C" int lrh_pt_scene(LrhContext *c, const float *prims, int nprims, const
         return lr_fail(LRH_EINVAL, "lrh_pt_scene: bad arguments");
     if (light >= 0 && prims[24 * light + 7] < 0.5f) return lr_fail(LRH_EINVAL, "lrh_pt_scene: the lamp must be a quad");
     if ((int64_t)nprims + ntris > LR_WIDE_MAX_SHAPES)
-        return lr_fail(LRH_EREFUSED, "lrh_pt_scene: %d shapes, the wide nodes' leaf references take at most %d",
+        return lr_fail(LRH_EREFUSED, "lrh_pt_scene: %d shapes, a scene holds at most %d",
                        nprims + ntris, LR_WIDE_MAX_SHAPES);
     for (int i = 0; i < nprims; i++) {
         const float m = prims[24 * (size_t)i + 11];
@@ -345,28 +317,19 @@ extern "C" int lrh_pt_scene(LrhContext *c, const float *prims, int nprims, const
     }
     s->depth = st.depth;
     // the 4-wide tree the jobs walk; its stack: up to 3 entries per wide level
-    if (hipMalloc((void **)&s->w4nodes, (size_t)n * 64) != hipSuccess) {
+    if (hipMalloc((void **)&s->slots, 2 * (size_t)n * LR_SLOT_F4 * 16) != hipSuccess) {
         (void)hipGetLastError();
         pt_scene_release(s);
         return lr_fail(LRH_ENOMEM, "lrh_pt_scene: device memory for the scene could not be had");
     }
-    rc = collapse_wide(c, s->nodes, 0u, n, st.depth, s->w4nodes);
+    rc = collapse_wide(c, s->nodes, 0u, n, st.depth, WideLeaves{s->aux, s->tris, nullptr, (uint32_t)nprims}, s->slots);
     if (rc) {
         pt_scene_release(s);
         return rc;
     }
-    // the triangles in leaf order: a leaf's triangle is then one load after its node, beside
-    // (not after) its aux entry
-    if (hipMalloc((void **)&s->ltris, (size_t)n * 48) != hipSuccess) {
-        (void)hipGetLastError();
-        pt_scene_release(s);
-        return lr_fail(LRH_ENOMEM, "lrh_pt_scene: device memory for the scene could not be had");
-    }
-    hipLaunchKernelGGL(k_leaf_tris, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, s->aux, n, (uint32_t)nprims,
-                       (const float4 *)s->tris, s->ltris);
     s->depth = 2 * st.depth + 4;
     s->bytes = (size_t)nprims * 96 + (size_t)ntris * 48 + hm.size() * 4 + boxes.size() * 4 + (2 * (size_t)n - 1) * 32 +
-               (size_t)n * 4 + tab.size() * 4 + mask.size() * 2 + (size_t)n * 64 + (size_t)n * 48;
+               (size_t)n * 4 + tab.size() * 4 + mask.size() * 2 + 2 * (size_t)n * LR_SLOT_F4 * 16;
     // the tree is built on the context's stream; the engines that render the scene run on
     // streams of their own, so the scene is complete before it is handed out
     if (hipStreamSynchronize(c->stream) != hipSuccess) {
@@ -637,7 +600,7 @@ static int top_cost(LrhPtScene *s, double *cost)
 }
 
 // The top level over the instances again, from their records on the device: their world boxes,
-// the tree over them, its binary child-box records and its 4-wide copy; the walks' stack depth.
+// the tree over them and its 4-wide copy; the walks' stack depth.
 // Waits for it (collapse_wide does).
 static int rebuild_top(LrhPtScene *s, int builder, LrhBuildStats *stats)
 {
@@ -650,12 +613,8 @@ static int rebuild_top(LrhPtScene *s, int builder, LrhBuildStats *stats)
     int rc = lrh_build(c, (const float *)s->tboxes, ninst, nullptr, builder, 0, 0, 0, s->tnodes, s->taux, nullptr, &st);
     if (rc) return rc;
     const size_t nn = 2 * (size_t)ninst - 1;
-    hipLaunchKernelGGL(k_child_boxes, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, c->stream, (const float4 *)s->tnodes, 0,
-                       (int)nn, s->wnodes);
-    if (ninst == 1) hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(1), 0, c->stream, (const float4 *)s->tnodes, 0u, s->wnodes);
-    LR_HIP(hipGetLastError());
-    // the top level 4-wide (the closest-hit walk's); collapse_wide waits for it
-    rc = collapse_wide(c, s->tnodes, 0u, ninst, st.depth, s->tw4nodes);
+    // the top level 4-wide (the walks'); collapse_wide waits for it
+    rc = collapse_wide(c, s->tnodes, 0u, ninst, st.depth, WideLeaves{s->taux, nullptr, s->inst, 0u}, s->slots);
     if (rc) return rc;
     // for later refits: each record's parent, and this build's cost
     hipLaunchKernelGGL(k_parents, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, c->stream, (const float4 *)s->tnodes,
@@ -690,11 +649,7 @@ static int refit_top(LrhPtScene *s, LrhBuildStats *stats)
     int rc = top_cost(s, &cost);
     if (rc) return rc;
     if (!(cost <= LR_REFIT_GROWTH * s->tcost_build)) return rebuild_top(s, s->top_builder, stats);
-    hipLaunchKernelGGL(k_child_boxes, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, c->stream, (const float4 *)s->tnodes, 0,
-                       nn, s->wnodes);
-    if (ninst == 1) hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(1), 0, c->stream, (const float4 *)s->tnodes, 0u, s->wnodes);
-    LR_HIP(hipGetLastError());
-    rc = collapse_wide(c, s->tnodes, 0u, ninst, s->tlas_depth, s->tw4nodes);   // (waits for it)
+    rc = collapse_wide(c, s->tnodes, 0u, ninst, s->tlas_depth, WideLeaves{s->taux, nullptr, s->inst, 0u}, s->slots);   // (waits for it)
     if (rc) return rc;
     LR_HIP(hipEventRecord(c->ev[1], c->stream));
     LR_HIP(hipEventSynchronize(c->ev[1]));
@@ -821,24 +776,14 @@ extern "C" int lrh_pt_scene_mesh(LrhPtScene *s, int mesh, const float *tris, int
     LR_HIP(hipStreamSynchronize(c->stream));
     LR_HIP(hipMemcpy(s->tris + 3 * (size_t)f, tris, (size_t)n * 48, hipMemcpyHostToDevice));
     // its boxes, its tree in its place (records from its root, aux entries from its first
-    // triangle), the records' child boxes, its 4-wide copy from its first wide slot, its
-    // triangles in leaf order
+    // triangle), its 4-wide copy from its first slot
     int rc = lrh_tri_boxes(c, (const float *)(s->tris + 3 * (size_t)f), n, (float *)(s->mboxes + 2 * (size_t)f));
     LrhBuildStats st;
     if (!rc) rc = lrh_build(c, (const float *)(s->mboxes + 2 * (size_t)f), n, nullptr, builder, root, (uint32_t)f, (uint32_t)f,
                             s->mnodes, s->maux, nullptr, &st);
     if (rc) return rc;
-    const int nn = 2 * n - 1;
-    if (n == 1) hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(1), 0, c->stream, (const float4 *)s->mnodes, root, s->mwnodes);
-    else
-        hipLaunchKernelGGL(k_child_boxes, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, c->stream, (const float4 *)s->mnodes,
-                           (int)root, nn, s->mwnodes);
-    LR_HIP(hipGetLastError());
-    rc = collapse_wide(c, s->mnodes, root, n, st.depth, s->mw4nodes, (uint32_t)f);
+    rc = collapse_wide(c, s->mnodes, root, n, st.depth, WideLeaves{s->maux, s->tris, nullptr, 0u}, s->mslots, 2u * (uint32_t)f);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_leaf_tris, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, s->maux + f, n, 0u,
-                       (const float4 *)s->tris, s->ltris + 3 * (size_t)f);
-    LR_HIP(hipGetLastError());
     s->mdepth[(size_t)mesh] = st.depth;
     s->mesh_depth = 0;
     for (int d : s->mdepth) s->mesh_depth = d > s->mesh_depth ? d : s->mesh_depth;
@@ -862,7 +807,7 @@ extern "C" int lrh_pt_scene_instanced(LrhContext *c, const float *mtris, const i
     const int M = mesh_first[nmeshes];
     if (M > 0 && !mtris) return lr_fail(LRH_EINVAL, "lrh_pt_scene_instanced: no triangles");
     if (M > LR_WIDE_MAX_SHAPES || ninst > LR_WIDE_MAX_SHAPES)
-        return lr_fail(LRH_EREFUSED, "lrh_pt_scene_instanced: the wide nodes' leaf references take at most %d shapes",
+        return lr_fail(LRH_EREFUSED, "lrh_pt_scene_instanced: a scene holds at most %d shapes",
                        LR_WIDE_MAX_SHAPES);
     for (int i = 0; i < M; i++) {
         uint32_t w;
@@ -906,16 +851,14 @@ extern "C" int lrh_pt_scene_instanced(LrhContext *c, const float *mtris, const i
     const size_t tn = 2 * (size_t)ninst - 1;
     bool ok = dev_upload((void **)&s->tris, mtris, (size_t)M * 48) && dev_upload((void **)&s->mboxes, nullptr, (size_t)M * 32) &&
               dev_upload((void **)&s->mnodes, nullptr, nnodes * 32) && dev_upload((void **)&s->maux, nullptr, (size_t)M * 4) &&
-              dev_upload((void **)&s->mwnodes, nullptr, nnodes * 64) &&
               dev_upload((void **)&s->mroot, roots.data(), roots.size() * 4) &&
               dev_upload((void **)&s->mats, hm.data(), hm.size() * 4) && dev_upload((void **)&s->tab, tab.data(), tab.size() * 4) &&
               dev_upload((void **)&s->mask, mask.data(), mask.size() * 2) &&
               dev_upload((void **)&s->inst, nullptr, (size_t)ninst * 64) && dev_upload((void **)&s->ifwd, nullptr, (size_t)ninst * 48) &&
               dev_upload((void **)&s->tboxes, nullptr, (size_t)ninst * 32) && dev_upload((void **)&s->tnodes, nullptr, tn * 32) &&
-              dev_upload((void **)&s->taux, nullptr, (size_t)ninst * 4) && dev_upload((void **)&s->wnodes, nullptr, tn * 64) &&
-              dev_upload((void **)&s->mw4nodes, nullptr, (size_t)M * 64) && dev_upload((void **)&s->ltris, nullptr, (size_t)M * 48) &&
-              dev_upload((void **)&s->tw4nodes, nullptr, (size_t)ninst * 64) &&
-              dev_upload((void **)&s->mroot4, nullptr, (size_t)nmeshes * 4) && dev_upload((void **)&s->tparent, nullptr, tn * 4) &&
+              dev_upload((void **)&s->taux, nullptr, (size_t)ninst * 4) &&
+              dev_upload((void **)&s->mslots, nullptr, 2 * (size_t)M * LR_SLOT_F4 * 16) &&
+              dev_upload((void **)&s->slots, nullptr, 2 * (size_t)ninst * LR_SLOT_F4 * 16) && dev_upload((void **)&s->tparent, nullptr, tn * 4) &&
               dev_upload((void **)&s->tarrive, nullptr, tn * 4) && dev_upload((void **)&s->tcost_dev, nullptr, 8) &&
               dev_upload((void **)&s->emit, nullptr, LR_MAX_EMITTERS * 80) &&
               dev_upload((void **)&s->inst_emit, nullptr, (size_t)ninst * 4);
@@ -937,40 +880,25 @@ extern "C" int lrh_pt_scene_instanced(LrhContext *c, const float *mtris, const i
                        s->mnodes, s->maux, nullptr, &st);
         if (!rc) mdepth[m] = st.depth;
         if (!rc && st.depth > depth) depth = st.depth;
-        if (!rc && n == 1)
-            hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(1), 0, c->stream, (const float4 *)s->mnodes, roots[m], s->mwnodes);
     }
-    if (!rc && nnodes)
-        hipLaunchKernelGGL(k_child_boxes, dim3((unsigned)((nnodes + 255) / 256)), dim3(256), 0, c->stream,
-                           (const float4 *)s->mnodes, 0, (int)nnodes, s->mwnodes);
-    // each mesh 4-wide, its wide nodes from the mesh's first triangle on (a mesh of n
-    // triangles has at most n wide nodes), and the triangles in the meshes' leaf order
+    // each mesh 4-wide (a mesh of n triangles has at most 2 n - 1 slots)
     std::vector<uint32_t> roots4(nmeshes);
     for (int m = 0; !rc && m < nmeshes; m++) {
         const int f = mesh_first[m], n = mesh_first[m + 1] - f;
-        roots4[m] = (uint32_t)f;
-        rc = collapse_wide(c, s->mnodes, roots[m], n, mdepth[m], s->mw4nodes, (uint32_t)f);
+        roots4[m] = LR_SLOT_F4 * 2u * (uint32_t)f;
+        rc = collapse_wide(c, s->mnodes, roots[m], n, mdepth[m], WideLeaves{s->maux, s->tris, nullptr, 0u}, s->mslots, 2u * (uint32_t)f);
     }
-    if (!rc && M) {
-        hipLaunchKernelGGL(k_leaf_tris, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, c->stream, s->maux, M, 0u,
-                           (const float4 *)s->tris, s->ltris);
-        if (hipGetLastError() != hipSuccess) rc = lr_fail(LRH_EDEVICE, "lrh_pt_scene_instanced: a launch failed");
-    }
-    if (!rc && nmeshes && hipMemcpy(s->mroot4, roots4.data(), (size_t)nmeshes * 4, hipMemcpyHostToDevice) != hipSuccess)
-        rc = lr_fail(LRH_EDEVICE, "lrh_pt_scene_instanced: a copy failed");
     if (rc) {
         pt_scene_release(s);
         return rc;
     }
-    // the one-shape meshes' root records were written before the pass over all inner nodes,
-    // which skips leaves: they stay
     s->mesh_depth = depth;
     s->mfirst.assign(mesh_first, mesh_first + nmeshes + 1);
     s->mdepth = mdepth;
     s->mroot_h = roots;
     s->mroot4_h = roots4;
-    s->bytes = (size_t)M * (48 + 32 + 4 + 64 + 48) + nnodes * (32 + 64) + hm.size() * 4 + tab.size() * 4 + mask.size() * 2 +
-               (size_t)ninst * (64 + 48 + 32 + 4 + 64 + 4) + tn * (32 + 64 + 8) + (size_t)nmeshes * 8 + 8 +
+    s->bytes = (size_t)M * (48 + 32 + 4 + 2 * LR_SLOT_F4 * 16) + nnodes * 32 + hm.size() * 4 + tab.size() * 4 + mask.size() * 2 +
+               (size_t)ninst * (64 + 48 + 32 + 4 + 2 * LR_SLOT_F4 * 16 + 4) + tn * (32 + 8) + (size_t)nmeshes * 4 + 8 +
                LR_MAX_EMITTERS * 80;
     rc = lrh_pt_scene_update(s, inst, ninst, LRH_LBVH, nullptr);
     if (rc) {
@@ -983,14 +911,10 @@ extern "C" int lrh_pt_scene_instanced(LrhContext *c, const float *mtris, const i
 
 void lr_job_scene(JobDev &jd, const LrhPtScene *s)
 {
-    jd.nodes = s->two_level ? s->tw4nodes : s->w4nodes;
-    jd.bnodes = s->wnodes;
-    jd.aux = s->aux;
+    jd.slots = s->slots;
     jd.tris = s->tris;
-    jd.ltris = s->ltris;
     jd.prims = s->prims;
     jd.mats = s->mats;
-    jd.root = 0;
     jd.nprims = (uint32_t)s->nprims;
     jd.light = s->light;
     jd.eps = s->eps;
@@ -1006,9 +930,7 @@ void lr_job_scene(JobDev &jd, const LrhPtScene *s)
     jd.env_rot_c = cosf(s->env_rot);
     jd.env_rot_s = sinf(s->env_rot);
     jd.two_level = s->two_level;
-    jd.mnodes = s->mwnodes;
-    jd.mnodes4 = s->mw4nodes;
-    jd.maux = s->maux;
+    jd.mslots = s->mslots;
     jd.inst = s->inst;
     jd.emit = s->emit;
     jd.inst_emit = s->inst_emit;
@@ -1028,7 +950,7 @@ __global__ __launch_bounds__(128) void k_scene_trace(JobDev J, const float4 *__r
     const WalkStack S{&stk[0][threadIdx.x], 128, spill + i, (size_t)n, LR_LDS_STACK + spill_per};
     WalkCnt wc;
     const WalkHit h = J.two_level ? walk4_tl<ANY, false, LR_LDS_STACK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, overflow, wc)
-                                  : walk4<ANY, false, LR_LDS_STACK>(J.nodes, J.aux, J.ltris, J.prims, J.nprims, v3of(r0),
+                                  : walk4<ANY, false, LR_LDS_STACK>(J.slots, J.prims, J.nprims, v3of(r0),
                                                                     v3of(r1), r0.w, r1.w, S, overflow, wc);
     hits[i] = make_float4(h.t, __uint_as_float(h.id), h.b1, h.b2);
 }

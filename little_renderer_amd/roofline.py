@@ -3,9 +3,10 @@ between the compute units and memory, whatever the caches do. A kernel's rooflin
 bytes over its measured time, against the HBM peak.
 
 Walks (k_trace, k_extend, k_shadow, k_scene_trace): per ray its 32-byte ray read and its 16-byte
-hit written, per node record fetched its size (32 bytes for the reference's binary node, 64 for
-the compressed 4-wide node), per shape tested its 48-byte triangle and 4-byte aux entry. The node
-and shape counts are the walks' own counters on the same tree and rays.
+hit written, per node record fetched its size (32 bytes for the reference's binary node), per shape
+tested its 48-byte triangle and 4-byte aux entry; the engine's 4-wide walks read one 48-byte slot
+for either (SLOT_BYTES). The node and shape counts are the walks' own counters on the same tree
+and rays.
 
 LBVH build (k_bounds, k_morton, k_sort_pass x 4, k_lbvh and k_lbvh_top), per primitive:
   bounds    the box read, 32
@@ -35,7 +36,8 @@ passes before it priced as for the LBVH (bounds 32, morton 40, sort 64 per primi
 HBM_PEAK_GBS = 8000.0           # MI355X HBM3E
 
 NODE_BYTES_BINARY = 32          # the reference's node (put_nodes)
-NODE_BYTES_WIDE = 64            # the compressed 4-wide node
+NODE_BYTES_WIDE = 64            # a compressed 4-wide node with its four child references
+SLOT_BYTES = 48                 # the engine's walks: a 4-wide node or a leaf's shape and id
 RAY_BYTES, HIT_BYTES, SHAPE_BYTES = 32, 16, 52
 
 LBVH_BYTES = {"bounds": 32, "morton": 40, "sort": 64, "lbvh": 4 + 32 + 32 + 4 + 64}
@@ -48,9 +50,9 @@ def shade_bytes(entries, continued, shadow_rays):
     return (SHADE_IN + SHADE_HIT) * entries + SHADE_NEXT * continued + SHADE_SHADOW * shadow_rays
 
 
-def walk_bytes(rays, node_fetches, shape_tests, node_bytes):
+def walk_bytes(rays, node_fetches, shape_tests, node_bytes, shape_bytes=SHAPE_BYTES):
     """a walk kernel's algorithmic bytes"""
-    return (RAY_BYTES + HIT_BYTES) * rays + node_bytes * node_fetches + SHAPE_BYTES * shape_tests
+    return (RAY_BYTES + HIT_BYTES) * rays + node_bytes * node_fetches + shape_bytes * shape_tests
 
 
 def lbvh_bytes(n, with_bounds=True):
