@@ -59,6 +59,21 @@ def test_batched_equals_plain_at_the_grid_s_edges(world, grids, off, tile):
     eng.close()
 
 
+def test_more_jobs_in_a_tile_than_a_work_group_counts_apart(world):
+    # 97 jobs of 3 x 2 to 9 x 8 pixels at once: their paths share tiles, and job slots 32 apart
+    # meet in a work-group's counters; every job ends, with the image it has alone
+    ctx, ps = world
+    eng = lr.Engine(ctx, slots_log2=12, max_tree_depth=max(64, ps.info()[0]), image_bytes=16 << 20)
+    sizes = [(3 + k % 7, 2 + k % 7) for k in range(97)]
+    jobs = [lr.make_job(ps, lr.batch_camera(k, w, h), w, h, 1 + k % 3, seed=k) for k, (w, h) in enumerate(sizes)]
+    ids = [eng.submit(j) for j in jobs]
+    eng.drain()
+    got = [image(eng, i, w, h) for i, (w, h) in zip(ids, sizes)]
+    for j, g, (w, h) in zip(jobs, got, sizes):
+        assert np.array_equal(g, image(eng, eng.plain(j), w, h))
+    eng.close()
+
+
 @pytest.mark.parametrize("w, h", [(1, 1), (3, 65), (7, 9), (8, 8), (9, 7), (65, 3), (24, 20)])
 def test_ragged_images_match_the_oracle(world, w, h):
     ctx, _ = world
