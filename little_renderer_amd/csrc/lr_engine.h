@@ -110,7 +110,9 @@ struct EngCtl {
     unsigned int count[4];                  // ray queues [0], [1] as shade left them; shadow queue [2]
     unsigned int tiles[3];                  // extend's, shade's, shadow's tile counters
     unsigned int spar;                      // the parity of the queue the shade kernel appended to
-    unsigned long long pad[4];
+    unsigned int ordered;                   // the queue's first entries that regen put in perm's order (else 0)
+    unsigned int pad0;
+    unsigned long long pad[3];
 };
 
 struct EngProgress {
@@ -135,7 +137,8 @@ struct EngArgs {
     uint64_t *rng[2];                       // PCG32 state (stream: the pixel)
     uint2 *meta[2];                         // q (pass x pixels + pixel), depth
     float4 *qray[2];                        // o.xyz tmin | d.xyz tmax
-    uint32_t *qid[2];                       // job << 22
+    uint32_t *qid[2];                       // job << 22 | the direction's cell (a bounce ray's)
+    uint32_t *perm;                         // the order the extension walk takes the bounce rays in
     float4 *hits;                           // t, id, b1, b2 (by queue position)
     float4 *sray;
     uint32_t *sid;                          // job << 22 | the path's next queue position
@@ -157,6 +160,7 @@ struct EngArgs {
     unsigned long long *counts;             // node records and shapes walked (counting extend only)
     unsigned long long *ostat;              // shade's tiles: look-back status of its ordered appends
     int mult;                               // a tile is mult work-groups' widths of entries
+    int order;                              // regen orders the bounce rays for the extension walk
     int refill;                             // k_extend_rf: idle lanes of a wave that take new rays
     int refill_shadow;                      // k_shadow_rf: the same
 };

@@ -74,6 +74,23 @@ def test_more_jobs_in_a_tile_than_a_work_group_counts_apart(world):
     eng.close()
 
 
+@pytest.mark.parametrize("block_shade", [64, 128, 256])
+@pytest.mark.parametrize("w, h, spp", [(901, 613, 1), (1024, 1024, 3)])
+def test_ordered_bounce_rays_change_no_image(world, w, h, spp, block_shade):
+    # enough bounce rays (from 262,144 on) of a scene of over 1000 shapes: the walk takes them by
+    # direction, in windows of every size with a ragged last one; the plain form takes them as queued
+    ctx, ps = world
+    eng = lr.Engine(ctx, slots_log2=22, max_tree_depth=max(64, ps.info()[0]), image_bytes=64 << 20)
+    eng.tune = {"block_shade": block_shade}
+    job = lr.make_job(ps, lr.batch_camera(4, w, h), w, h, spp, seed=w)
+    i = eng.submit(job)
+    eng.drain()
+    got = image(eng, i, w, h)
+    assert np.array_equal(got, image(eng, eng.plain(job), w, h))
+    assert np.any(got[..., :3])
+    eng.close()
+
+
 @pytest.mark.parametrize("w, h", [(1, 1), (3, 65), (7, 9), (8, 8), (9, 7), (65, 3), (24, 20)])
 def test_ragged_images_match_the_oracle(world, w, h):
     ctx, _ = world
