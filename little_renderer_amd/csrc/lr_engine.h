@@ -104,15 +104,16 @@ struct EngCtl {
     unsigned long long next, issue_end;     // the next path index to start; the end of those issued
     unsigned long long iq_lo, iq_hi;        // the issue records in use
     unsigned long long rays_ext, rays_shadow;
-    unsigned long long iter;                // iterations run (its parity picks the ray queue)
+    unsigned long long iter;                // iterations run
     unsigned long long claimed;             // paths the running iteration's regen started (at the end of
-                                            // the ray queue, past its count; 0 after the iteration)
+                                            // the ray queue, past its count)
     unsigned int count[4];                  // ray queues [0], [1] as shade left them; shadow queue [2]
-    unsigned int tiles[3];                  // extend's, shade's, shadow's tile counters
-    unsigned int spar;                      // the parity of the queue the shade kernel appended to
-    unsigned int ordered;                   // the queue's first entries that regen put in perm's order (else 0)
+    unsigned int tiles[3];                  // the walks', shade's, the shadow walk's (alone) tile counters
+    unsigned int spar;                      // the parity of the queue shade appended to: the next walks'
+    unsigned int ordered;                   // that queue's first entries that regen put in perm's order (else 0)
+    unsigned int qpar, qlen;                // the queue the walks went through, for shade: parity, length
     unsigned int pad0;
-    unsigned long long pad[3];
+    unsigned long long pad[2];
 };
 
 struct EngProgress {
@@ -184,6 +185,7 @@ typedef void (*LrLightFn)(hipStream_t s, const JobDev &J, uint32_t nlp, uint64_t
 // in fewer registers)
 struct LrEngTable {
     LrEngFn regen[3], shade[3][2];
+    LrEngFn walks[3][3][2][2];   // extend and shadow in one launch
     LrEngFn extend[3][3][2], extend_count[3][3][2], shadow[3][3][2][2], shadow_count[3][3][2][2];
     // [block][stack][counting]: the walks with lanes refilled (single-level scenes; the shadow
     // walk's with one shadow ray a vertex)

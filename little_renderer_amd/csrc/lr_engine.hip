@@ -238,7 +238,8 @@ EngArgs args_for(const LrhEngine *e, int stack, size_t threads, int mult, int re
     return A;
 }
 
-// the persistent grids of the batched form; ev (profiling): 5 events around the 4 kernels
+// One iteration in the persistent grids of the batched form: regen, the walks, shade. ev (profiling):
+// 5 events around regen, the extension walk, the shadow walk and shade, each a launch of its own
 void launch_iteration(LrhEngine *e, const LrhTune &t, hipEvent_t *ev = nullptr)
 {
     const LrEngTable &T = table();
@@ -247,18 +248,21 @@ void launch_iteration(LrhEngine *e, const LrhTune &t, hipEvent_t *ev = nullptr)
     const EngArgs At = args_for(e, t.stack, (size_t)gt.x * t.block_trace, t.tile, t.refill, t.refill_shadow);
     EngArgs As = args_for(e, t.stack, 0, t.tile);
     As.order = e->order && !e->two_level ? 1 : 0;
+    const int tl = e->two_level ? 1 : 0, ml = e->multi ? 1 : 0, cnt = e->counting ? 1 : 0;
+    const bool rf = !tl && t.refill > 0, srf = !tl && !ml && t.refill_shadow > 0;
     if (ev) (void)hipEventRecord(ev[0], e->stream);
     T.regen[bs](gs, e->stream, As);
     if (ev) (void)hipEventRecord(ev[1], e->stream);
-    const int tl = e->two_level ? 1 : 0;
-    if (!tl && t.refill > 0) T.extend_rf[bt][sk][e->counting ? 1 : 0](gt, e->stream, At);
-    else (e->counting ? T.extend_count : T.extend)[bt][sk][tl](gt, e->stream, At);
-    if (ev) (void)hipEventRecord(ev[2], e->stream);
-    const int ml = e->multi ? 1 : 0;
-    T.shade[bs][ml](gs, e->stream, As);
+    if (!ev && !cnt && !rf && !srf) T.walks[bt][sk][tl][ml](gt, e->stream, At);
+    else {
+        if (rf) T.extend_rf[bt][sk][cnt](gt, e->stream, At);
+        else (cnt ? T.extend_count : T.extend)[bt][sk][tl](gt, e->stream, At);
+        if (ev) (void)hipEventRecord(ev[2], e->stream);
+        if (srf) T.shadow_rf[bt][sk][cnt](gt, e->stream, At);
+        else (cnt ? T.shadow_count : T.shadow)[bt][sk][tl][ml](gt, e->stream, At);
+    }
     if (ev) (void)hipEventRecord(ev[3], e->stream);
-    if (!tl && !ml && t.refill_shadow > 0) T.shadow_rf[bt][sk][e->counting ? 1 : 0](gt, e->stream, At);
-    else (e->counting ? T.shadow_count : T.shadow)[bt][sk][tl][ml](gt, e->stream, At);
+    T.shade[bs][ml](gs, e->stream, As);
     if (ev) (void)hipEventRecord(ev[4], e->stream);
 }
 
@@ -274,12 +278,13 @@ int launch_profiled(LrhEngine *e)
     for (int i = 0; i < G; i++) launch_iteration(e, e->tune, &e->pevs[5 * i]);
     ENG_HIP(hipGetLastError());
     ENG_HIP(hipEventSynchronize(e->pevs[5 * G - 1]));
+    constexpr int stat[4] = {0, 1, 3, 2};   // (the stats' order: regen, extend, shade, shadow)
     for (int i = 0; i < G; i++)
         for (int k = 0; k < 4; k++) {
             float ms = 0.0f;
             ENG_HIP(hipEventElapsedTime(&ms, e->pevs[5 * i + k], e->pevs[5 * i + k + 1]));
-            e->kms[k] += ms;
-            e->klaunch[k]++;
+            e->kms[stat[k]] += ms;
+            e->klaunch[stat[k]]++;
         }
     return 0;
 }
@@ -979,11 +984,14 @@ int lrh_engine_plain(LrhEngine *e, const LrhJob *job, int64_t *id)
         // the pass: the job's paths s * npix .. (s + 1) * npix - 1, one per pixel
         rc = issue_chunk(e, slot, npix);
         if (rc) return rc;
+        // (a vertex's shadow rays are walked with the next one's rays: once more past the last vertex)
         T.regen[bs](gs, e->stream, As);
-        for (int d = 0; d <= job->max_depth; d++) {
-            (e->counting ? T.extend_count : T.extend)[bt][sk][tl](gt, e->stream, At);
+        for (int d = 0; d <= job->max_depth + 1; d++) {
+            if (e->counting) {
+                T.extend_count[bt][sk][tl](gt, e->stream, At);
+                T.shadow_count[bt][sk][tl][ml](gt, e->stream, At);
+            } else T.walks[bt][sk][tl][ml](gt, e->stream, At);
             T.shade[bs][ml](gs, e->stream, As);
-            (e->counting ? T.shadow_count : T.shadow)[bt][sk][tl][ml](gt, e->stream, At);
         }
     }
     ENG_HIP(hipGetLastError());

@@ -1,4 +1,4 @@
-// lr_engine_k.h - the engine's four wavefront kernels, templated on the work-group size (and
+// lr_engine_k.h - the engine's wavefront kernels, templated on the work-group size (and
 // the walks on their LDS stack depth). Included once per work-group size by
 // lr_engine_b64.hip, lr_engine_b128.hip and lr_engine_b256.hip, each filling the launch table
 // (lr_engine.h) for its size.
@@ -39,6 +39,28 @@ __device__ __forceinline__ void for_tiles(unsigned int *ctr, uint32_t n, int mul
     }
 }
 
+// The same over two queues, the tiles of the first before those of the second
+template <int BLK, class F, class G>
+__device__ __forceinline__ void for_tiles2(unsigned int *ctr, uint32_t n, uint32_t m, int mult, F &&body, G &&body2)
+{
+    __shared__ uint32_t s_tile;
+    const uint32_t width = (uint32_t)BLK * (uint32_t)mult;
+    const uint32_t nt = (uint32_t)(((uint64_t)n + width - 1) / width), ntiles = nt + (uint32_t)(((uint64_t)m + width - 1) / width);
+    for (uint32_t tile = blockIdx.x; tile < ntiles;) {
+        const uint64_t base = (uint64_t)(tile < nt ? tile : tile - nt) * width;
+        for (int j = 0; j < mult; j++) {
+            const uint64_t i = base + (uint64_t)j * BLK + threadIdx.x;
+            if (tile < nt) body((uint32_t)i, i < n);
+            else body2((uint32_t)i, i < m);
+        }
+        if (ntiles <= gridDim.x) break;
+        __syncthreads();
+        if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1u);
+        __syncthreads();
+        tile = gridDim.x + s_tile;
+    }
+}
+
 // The same with every tile claimed, for bodies that wait on the tiles before theirs
 // (ordered_append2): a tile is claimed by a running work-group, in order, so every tile waited
 // on is being worked on however many of the grid's work-groups the chip holds at once. Where the
@@ -61,6 +83,12 @@ __device__ __forceinline__ void for_tiles_ordered(unsigned int *ctr, uint32_t n,
     }
 }
 
+// An iteration is regen, the walks (extend and shadow, as one kernel or two), shade. The shadow rays
+// that shade makes are walked in the next iteration, beside the extension rays. A word of the
+// counters that a kernel's work-groups read is written by another kernel: regen and the walks read
+// the queue's parity (spar), its length (count, claimed, ordered) and the shadow queue's, which shade
+// writes (regen: claimed, ordered); shade reads the parity and length the walks leave it (qpar, qlen).
+//
 // Each kernel clears the other kernels' tile counters as it starts (kernels of one stream run
 // one after another, and no kernel follows itself), so every kernel finds its own at zero (regen
 // claims nothing: self = -1).
@@ -70,9 +98,22 @@ __device__ __forceinline__ void reset_tiles(EngCtl *ctl, int self)
         if (k != self) ctl->tiles[k] = 0;
 }
 
-// the ray queue's length while an iteration runs: the paths the last iteration's shade appended
-// and those this one's regen started after them
+// the ray queue's length for the walks: the paths the last iteration's shade appended and those this
+// one's regen started after them
 __device__ __forceinline__ uint32_t queue_len(const EngCtl *ctl, int cur) { return ctl->count[cur] + (uint32_t)ctl->claimed; }
+
+// the walks' part of the counters (one thread of the extension walk): regen's claim applied to the
+// ring and the issue counter, the rays counted, the queue handed to shade
+__device__ __forceinline__ void walk_begin(EngCtl *ctl, int cur, uint32_t n)
+{
+    const unsigned long long c = ctl->claimed;
+    ctl->head += c;
+    ctl->next += c;
+    ctl->rays_ext += n;
+    ctl->iter += 1;
+    ctl->qpar = (unsigned int)cur;
+    ctl->qlen = n;
+}
 
 __device__ __forceinline__ long long to_fixed(float x)
 {
@@ -496,7 +537,7 @@ __global__ __launch_bounds__(BLK) void k_regen(EngArgs A)
     const unsigned long long lo = ctl->iq_lo, hi = ctl->iq_hi;
     const unsigned long long free_n = tail - head, todo = iend - next;
     const uint32_t n = (uint32_t)(free_n < todo ? free_n : todo);
-    const int cur = (int)(ctl->iter & 1ull);
+    const int cur = (int)ctl->spar;
     const uint32_t start = ctl->count[cur];
     // the bounce rays shade left, ordered for the walk (start: their number), in windows as large as
     // leave two to each of 256 compute units, 8 to 32 rounds
@@ -568,14 +609,106 @@ __device__ __forceinline__ void add_counts(unsigned long long *c, unsigned long 
     }
 }
 
-// extend (wf_ext, trace_wave.wgsl:72-84): the closest hit of every queued ray, each through
-// its own job's tree. Also applies regen's claim to the ring and the issue counter (the claim itself
-// is part of the queue's length until the shadow kernel ends the iteration), and clears
-// the queues the shade kernel appends to. TL: two-level scenes may be queued (without it, such
-// a ray is not walked: flagged, so that the host reports it).
-// Without TL the kernel is held to 64 VGPRs, 8 waves per SIMD (the walk's own 63; the shadow walk
-// spills 12 bytes a lane), so that the whole persistent grid of 8 work-groups per compute unit is
-// resident.
+// extend (wf_ext, trace_wave.wgsl:72-84): the closest hit of the queue's k-th ray in the walk's order,
+// through its own job's tree. TL: two-level scenes may be queued (without it, such a ray is not
+// walked: flagged, so that the host reports it).
+template <bool COUNT, bool TL, int STK>
+__device__ __forceinline__ void extend_entry(const EngArgs &A, int cur, uint32_t k, uint32_t ordered, const WalkStack &S, WalkCnt &wc)
+{
+    const uint32_t i = k < ordered ? A.perm[k] : k;
+    const uint32_t id = A.qid[cur][i];
+    const JobDev &J = A.jobs[id >> LR_SLOT_BITS];
+    const float4 r0 = A.qray[cur][2 * (size_t)i], r1 = A.qray[cur][2 * (size_t)i + 1];
+    WalkHit h;
+    if (TL && J.two_level) h = walk4_tl<false, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
+    else if (!J.two_level)
+        h = walk4<false, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
+    else {
+        atomicOr(A.overflow, 2u);
+        h = WalkHit{r1.w, LR_NONE, 0.0f, 0.0f};
+    }
+    A.hits[i] = make_float4(h.t, __uint_as_float(h.id), h.b1, h.b2);
+}
+
+// shadow (wf_shadow, trace_wave.wgsl:335-355): any hit before the lamp; if none, the
+// contribution joins the path's radiance. Paths whose last vertex made the shadow ray end here.
+// Every lane of the wave calls this (live: it has entry i).
+template <bool COUNT, bool TL, bool MULTI, int STK>
+__device__ __forceinline__ void shadow_entry(const EngArgs &A, int par, uint32_t i, bool live, const WalkStack &S, WalkCnt &wc,
+                                             RetireSums &R)
+{
+    bool ends = false;
+    uint32_t jslot = 0, q = 0;
+    float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    int nx = 0;
+    bool glow = false;
+    auto walk = [&](const JobDev &J, float4 r0, float4 r1) {
+        if (TL && J.two_level) return walk4_tl<true, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
+        if (!J.two_level) return walk4<true, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
+        atomicOr(A.overflow, 2u);
+        return WalkHit{0.0f, 0u, 0.0f, 0.0f};   // occluded: adds nothing
+    };
+    if (live) {
+        const uint32_t id = A.sid[i];
+        const uint32_t at = id & LR_SLOT_MASK;
+        jslot = id >> LR_SLOT_BITS;
+        glow = (at & 1u) != 0u;   // (read only for a path that ends here: then at holds its glow flag)
+        const JobDev &J = A.jobs[jslot];
+        if constexpr (!MULTI) {
+            const WalkHit h = walk(J, A.sray[2 * (size_t)i], A.sray[2 * (size_t)i + 1]);
+            const float4 c = A.scon[i];
+            ends = c.w != 0.0f;
+            const bool lit = h.id == LR_NONE;
+            if (lit || ends) {
+                r = A.srad[i];
+                if (lit) {
+                    r.x += c.x;
+                    r.y += c.y;
+                    r.z += c.z;
+                }
+                if (!ends) A.rad[par][at] = r;   // the path's state in the queue (shade wrote it without this)
+                else q = A.sq[i];
+            }
+        } else {
+            // (0 in an entry that a one-light shade left before this engine's first of several lights:
+            // the array is clear until then)
+            const uint32_t x = A.sx[i];
+            nx = (int)(x >> 30);                       // the vertex's rays past the first
+            const uint32_t src = x & LR_SLOT_MASK;     // where shade left them
+            const float4 c0 = A.scon[i];
+            ends = c0.w != 0.0f;
+            uint32_t lit = 0;                          // bit j: ray j reached its light
+            for (int j = 0; j <= nx; j++) {
+                const float4 *rr = j == 0 ? A.sray + 2 * (size_t)i : (j == 1 ? A.xsray[0] : A.xsray[1]) + 2 * (size_t)src;
+                const WalkHit h = walk(J, rr[0], rr[1]);
+                if (h.id == LR_NONE) lit |= 1u << j;
+            }
+            if (lit || ends) {
+                // the lights' contributions join the path's radiance in the order shade made them
+                r = A.srad[i];
+                for (int j = 0; j <= nx; j++)
+                    if (lit >> j & 1u) {
+                        const float4 c = j == 0 ? c0 : (j == 1 ? A.xscon[0] : A.xscon[1])[src];
+                        r.x += c.x;
+                        r.y += c.y;
+                        r.z += c.z;
+                    }
+                if (!ends) A.rad[par][at] = r;   // the path's state in the queue (shade wrote it without these)
+                else q = A.sq[i];
+            }
+        }
+    }
+    // the rays past an entry's first are shadow rays too: counted a wave at a time
+    if constexpr (MULTI) {
+        if (__ballot(nx > 0)) {
+            int cnt = nx;
+            for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
+            if ((threadIdx.x & 63) == 0) atomicAdd(&A.ctl->rays_shadow, (unsigned long long)cnt);
+        }
+    }
+    retire(A, R, ends, jslot, q, r, glow);
+}
+
 // waves per SIMD a walk kernel is held to: 8, or fewer where its LDS stack (160 KB per compute
 // unit) allows fewer anyway
 constexpr int walk_waves(int blk, int stk)
@@ -583,46 +716,88 @@ constexpr int walk_waves(int blk, int stk)
     return (163840 / (stk * blk * 4 + 4)) * (blk / 64) / 4 < 8 ? (163840 / (stk * blk * 4 + 4)) * (blk / 64) / 4 : 8;
 }
 
+// shade's look-back status words, one per tile of at least 64 entries, cleared before it
+__device__ __forceinline__ void clear_ostat(const EngArgs &A, uint32_t n, size_t gtid, size_t threads)
+{
+    for (size_t k = gtid; k < (size_t)n / 64 + 2; k += threads) A.ostat[k] = 0ull;
+}
+
+// Both walks of an iteration in one launch: the extension rays' tiles, then the tiles of the shadow
+// rays that the last iteration's shade made. Neither waits for the other's slowest rays, which in a
+// queue too small to fill the chip are most of a walk's time, and an iteration is a launch shorter:
+// two 0.92M-path frames of an instanced scene 19.4 -> 15.9 ms, a 1280 x 720 still of 8 samples 11.1 ->
+// 9.0 ms, a 256 x 256 preview 0.86 -> 0.69 ms, a 54M-path queue 53.7 -> 50.4 ms.
+// Without TL the kernel is held to 64 VGPRs, 8 waves per SIMD, so that the whole persistent grid of 8
+// work-groups per compute unit is resident.
+template <int BLK, int STK, bool TL, bool MULTI>
+__global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_walks(EngArgs A)
+{
+    __shared__ uint32_t stk[STK][BLK];
+    EngCtl *ctl = A.ctl;
+    const int cur = (int)ctl->spar;
+    const uint32_t n = queue_len(ctl, cur), m = ctl->count[2], ordered = ctl->ordered;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        walk_begin(ctl, cur, n);
+        atomicAdd(&ctl->rays_shadow, (unsigned long long)m);
+        reset_tiles(ctl, K_EXTEND);
+    }
+    const size_t gtid = (size_t)blockIdx.x * BLK + threadIdx.x;
+    clear_ostat(A, n, gtid, (size_t)gridDim.x * BLK);
+    const WalkStack S{&stk[0][threadIdx.x], BLK, A.spill + gtid, (size_t)A.spill_stride, STK + A.spill_per};
+    WalkCnt wc;
+    __shared__ RetireSums R;
+    retire_begin(R);
+    for_tiles2<BLK>(&ctl->tiles[K_EXTEND], n, m, A.mult,
+                    [&](uint32_t k, bool live) {
+                        if (live) extend_entry<false, TL, STK>(A, cur, k, ordered, S, wc);
+                    },
+                    [&](uint32_t i, bool live) { shadow_entry<false, TL, MULTI, STK>(A, cur, i, live, S, wc, R); });
+    retire_end(A, R);
+}
+
+// the extension walk alone (profiled, counting its steps, or beside a refilled shadow walk)
 template <int BLK, int STK, bool COUNT, bool TL>
 __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_extend(EngArgs A)
 {
     __shared__ uint32_t stk[STK][BLK];
     EngCtl *ctl = A.ctl;
-    const int cur = (int)(ctl->iter & 1ull);
-    const uint32_t n = queue_len(ctl, cur);
+    const int cur = (int)ctl->spar;
+    const uint32_t n = queue_len(ctl, cur), ordered = ctl->ordered;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const unsigned long long c = ctl->claimed;
-        ctl->head += c;
-        ctl->next += c;
-        ctl->rays_ext += n;
-        ctl->count[1 - cur] = 0;
-        ctl->count[2] = 0;
+        walk_begin(ctl, cur, n);
         reset_tiles(ctl, K_EXTEND);
     }
     const size_t gtid = (size_t)blockIdx.x * BLK + threadIdx.x;
-    // the shade kernel's look-back status words, one per tile of at least 64 entries
-    for (size_t k = gtid; k < (size_t)n / 64 + 2; k += (size_t)gridDim.x * BLK) A.ostat[k] = 0ull;
+    clear_ostat(A, n, gtid, (size_t)gridDim.x * BLK);
     const WalkStack S{&stk[0][threadIdx.x], BLK, A.spill + gtid, (size_t)A.spill_stride, STK + A.spill_per};
     WalkCnt wc;
-    const uint32_t ordered = ctl->ordered;
     for_tiles<BLK>(&ctl->tiles[K_EXTEND], n, A.mult, [&](uint32_t k, bool live) {
-        if (!live) return;
-        const uint32_t i = k < ordered ? A.perm[k] : k;
-        const uint32_t id = A.qid[cur][i];
-        const JobDev &J = A.jobs[id >> LR_SLOT_BITS];
-        const float4 r0 = A.qray[cur][2 * (size_t)i], r1 = A.qray[cur][2 * (size_t)i + 1];
-        WalkHit h;
-        if (TL && J.two_level) h = walk4_tl<false, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
-        else if (!J.two_level)
-            h = walk4<false, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S,
-                                         A.overflow, wc);
-        else {
-            atomicOr(A.overflow, 2u);
-            h = WalkHit{r1.w, LR_NONE, 0.0f, 0.0f};
-        }
-        A.hits[i] = make_float4(h.t, __uint_as_float(h.id), h.b1, h.b2);
+        if (live) extend_entry<COUNT, TL, STK>(A, cur, k, ordered, S, wc);
     });
     if (COUNT) add_counts(A.counts, A.counts + 8, wc);
+}
+
+// the shadow walk alone, after the extension walk
+template <int BLK, int STK, bool COUNT, bool TL, bool MULTI>
+__global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_shadow(EngArgs A)
+{
+    __shared__ uint32_t stk[STK][BLK];
+    EngCtl *ctl = A.ctl;
+    const uint32_t n = ctl->count[2];
+    const int par = (int)ctl->spar;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        reset_tiles(ctl, K_SHADOW);
+        atomicAdd(&ctl->rays_shadow, (unsigned long long)n);
+    }
+    const size_t gtid = (size_t)blockIdx.x * BLK + threadIdx.x;
+    const WalkStack S{&stk[0][threadIdx.x], BLK, A.spill + gtid, (size_t)A.spill_stride, STK + A.spill_per};
+    WalkCnt wc;
+    __shared__ RetireSums R;
+    retire_begin(R);
+    for_tiles<BLK>(&ctl->tiles[K_SHADOW], n, A.mult,
+                   [&](uint32_t i, bool live) { shadow_entry<COUNT, TL, MULTI, STK>(A, par, i, live, S, wc, R); });
+    retire_end(A, R);
+    if (COUNT) add_counts(A.counts + 4, A.counts + 9, wc);
 }
 
 // ---- walks with lanes refilled (dynamic fetch, Aila & Laine 2009) ----------------------------
@@ -711,19 +886,14 @@ __global__ __launch_bounds__(BLK, walk_waves(BLK, STK)) void k_extend_rf(EngArgs
 {
     __shared__ uint32_t stk[STK][BLK];
     EngCtl *ctl = A.ctl;
-    const int par = (int)(ctl->iter & 1ull);
+    const int par = (int)ctl->spar;
     const uint32_t n = queue_len(ctl, par);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const unsigned long long c = ctl->claimed;
-        ctl->head += c;
-        ctl->next += c;
-        ctl->rays_ext += n;
-        ctl->count[1 - par] = 0;
-        ctl->count[2] = 0;
+        walk_begin(ctl, par, n);
         reset_tiles(ctl, K_EXTEND);
     }
     const size_t gtid = (size_t)blockIdx.x * BLK + threadIdx.x;
-    for (size_t k = gtid; k < (size_t)n / 64 + 2; k += (size_t)gridDim.x * BLK) A.ostat[k] = 0ull;
+    clear_ostat(A, n, gtid, (size_t)gridDim.x * BLK);
     const WalkStack S{&stk[0][threadIdx.x], BLK, A.spill + gtid, (size_t)A.spill_stride, STK + A.spill_per};
     WalkCnt wc;
     Refill f;
@@ -769,10 +939,7 @@ __global__ __launch_bounds__(BLK, walk_waves(BLK, STK)) void k_shadow_rf(EngArgs
     const int par = (int)ctl->spar;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         reset_tiles(ctl, K_SHADOW);
-        ctl->rays_shadow += n;
-        ctl->iter += 1;
-        ctl->claimed = 0;   // (the queue regen added to is done with)
-        ctl->ordered = 0;
+        atomicAdd(&ctl->rays_shadow, (unsigned long long)n);
     }
     const size_t gtid = (size_t)blockIdx.x * BLK + threadIdx.x;
     const WalkStack S{&stk[0][threadIdx.x], BLK, A.spill + gtid, (size_t)A.spill_stride, STK + A.spill_per};
@@ -817,7 +984,7 @@ __global__ __launch_bounds__(BLK, walk_waves(BLK, STK)) void k_shadow_rf(EngArgs
                     r.y += c.y;
                     r.z += c.z;
                 }
-                if (!ends) A.rad[par][at] = r;   // the path's next state (shade wrote it without this)
+                if (!ends) A.rad[par][at] = r;   // the path's state in the queue (shade wrote it without this)
                 else q = A.sq[i];
             }
             i = LR_NONE;
@@ -952,11 +1119,14 @@ template <int BLK, bool MULTI>
 __global__ __launch_bounds__(BLK) void k_shade(EngArgs A)
 {
     EngCtl *ctl = A.ctl;
-    const int cur = (int)(ctl->iter & 1ull);
-    const uint32_t n = queue_len(ctl, cur);
+    const int cur = (int)ctl->qpar;
+    const uint32_t n = ctl->qlen;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         reset_tiles(ctl, K_SHADE);
         ctl->spar = (unsigned int)(1 - cur);
+        ctl->claimed = 0;   // (regen's paths are in this queue; the next walk's are what it appends, and regen's next)
+        ctl->ordered = 0;
+        if (n == 0) ctl->count[1 - cur] = ctl->count[2] = 0;   // (else the last tile writes them)
     }
     __shared__ RetireSums R;
     retire_begin(R);
@@ -1193,114 +1363,6 @@ __global__ __launch_bounds__(BLK) void k_shade(EngArgs A)
         retire(A, R, live && !next && !shadow, jslot, q, rad_out, glow);
     });
     retire_end(A, R);
-}
-
-// shadow (wf_shadow, trace_wave.wgsl:335-355): any hit before the lamp; if none, the
-// contribution joins the path's radiance. Paths whose last vertex made the shadow ray end here.
-// TL and the register bound as for extend.
-template <int BLK, int STK, bool COUNT, bool TL, bool MULTI>
-__global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_shadow(EngArgs A)
-{
-    __shared__ uint32_t stk[STK][BLK];
-    EngCtl *ctl = A.ctl;
-    const uint32_t n = ctl->count[2];
-    const int par = (int)ctl->spar;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        reset_tiles(ctl, K_SHADOW);
-        ctl->rays_shadow += n;
-        ctl->iter += 1;
-        ctl->claimed = 0;   // (the queue regen added to is done with)
-        ctl->ordered = 0;
-    }
-    const size_t gtid = (size_t)blockIdx.x * BLK + threadIdx.x;
-    const WalkStack S{&stk[0][threadIdx.x], BLK, A.spill + gtid, (size_t)A.spill_stride, STK + A.spill_per};
-    WalkCnt wc;
-    __shared__ RetireSums R;
-    retire_begin(R);
-    for_tiles<BLK>(&ctl->tiles[K_SHADOW], n, A.mult, [&](uint32_t i, bool live) {
-        bool ends = false;
-        uint32_t jslot = 0, q = 0;
-        float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        int nx = 0;
-        bool glow = false;
-        if (live) {
-            const uint32_t id = A.sid[i];
-            const uint32_t at = id & LR_SLOT_MASK;
-            jslot = id >> LR_SLOT_BITS;
-            glow = (at & 1u) != 0u;   // (read only for a path that ends here: then at holds its glow flag)
-            const JobDev &J = A.jobs[jslot];
-            if constexpr (!MULTI) {
-                const float4 r0 = A.sray[2 * (size_t)i], r1 = A.sray[2 * (size_t)i + 1];
-                WalkHit h;
-                if (TL && J.two_level) h = walk4_tl<true, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
-                else if (!J.two_level)
-                    h = walk4<true, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S,
-                                                A.overflow, wc);
-                else {
-                    atomicOr(A.overflow, 2u);
-                    h = WalkHit{0.0f, 0u, 0.0f, 0.0f};   // occluded: adds nothing
-                }
-                const float4 c = A.scon[i];
-                ends = c.w != 0.0f;
-                const bool lit = h.id == LR_NONE;
-                if (lit || ends) {
-                    r = A.srad[i];
-                    if (lit) {
-                        r.x += c.x;
-                        r.y += c.y;
-                        r.z += c.z;
-                    }
-                    if (!ends) A.rad[par][at] = r;   // the path's next state (shade wrote it without this)
-                    else q = A.sq[i];
-                }
-            } else {
-                const uint32_t x = A.sx[i];
-                nx = (int)(x >> 30);                       // the vertex's rays past the first
-                const uint32_t src = x & LR_SLOT_MASK;     // where shade left them
-                const float4 c0 = A.scon[i];
-                ends = c0.w != 0.0f;
-                uint32_t lit = 0;                          // bit j: ray j reached its light
-                for (int j = 0; j <= nx; j++) {
-                    const float4 *rr = j == 0 ? A.sray + 2 * (size_t)i : (j == 1 ? A.xsray[0] : A.xsray[1]) + 2 * (size_t)src;
-                    const float4 r0 = rr[0], r1 = rr[1];
-                    WalkHit h;
-                    if (TL && J.two_level) h = walk4_tl<true, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
-                    else if (!J.two_level)
-                        h = walk4<true, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S,
-                                                    A.overflow, wc);
-                    else {
-                        atomicOr(A.overflow, 2u);
-                        h = WalkHit{0.0f, 0u, 0.0f, 0.0f};   // occluded: adds nothing
-                    }
-                    if (h.id == LR_NONE) lit |= 1u << j;
-                }
-                if (lit || ends) {
-                    // the lights' contributions join the path's radiance in the order shade made them
-                    r = A.srad[i];
-                    for (int j = 0; j <= nx; j++)
-                        if (lit >> j & 1u) {
-                            const float4 c = j == 0 ? c0 : (j == 1 ? A.xscon[0] : A.xscon[1])[src];
-                            r.x += c.x;
-                            r.y += c.y;
-                            r.z += c.z;
-                        }
-                    if (!ends) A.rad[par][at] = r;   // the path's next state (shade wrote it without these)
-                    else q = A.sq[i];
-                }
-            }
-        }
-        // the rays past an entry's first are shadow rays too: counted a wave at a time
-        if constexpr (MULTI) {
-            if (__ballot(nx > 0)) {
-                int cnt = nx;
-                for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
-                if ((threadIdx.x & 63) == 0) atomicAdd(&ctl->rays_shadow, (unsigned long long)cnt);
-            }
-        }
-        retire(A, R, ends, jslot, q, r, glow);
-    });
-    retire_end(A, R);
-    if (COUNT) add_counts(A.counts + 4, A.counts + 9, wc);
 }
 
 // The denoiser's guide of a job (trace.wgsl:1034-1107, guide): each pixel's ray through its
@@ -1764,6 +1826,11 @@ void L_shade(dim3 g, hipStream_t s, const EngArgs &A)
 {
     hipLaunchKernelGGL((k_shade<BLK, MULTI>), g, dim3(BLK), 0, s, A);
 }
+template <int BLK, int STK, bool TL, bool MULTI>
+void L_walks(dim3 g, hipStream_t s, const EngArgs &A)
+{
+    hipLaunchKernelGGL((k_walks<BLK, STK, TL, MULTI>), g, dim3(BLK), 0, s, A);
+}
 template <int BLK, int STK, bool COUNT, bool TL>
 void L_extend(dim3 g, hipStream_t s, const EngArgs &A)
 {
@@ -1789,6 +1856,10 @@ template <int BLK, int STK, int K>
 void fill_walks(LrEngTable &t)
 {
     const int b = lr_blk_index(BLK);
+    t.walks[b][K][0][0] = L_walks<BLK, STK, false, false>;
+    t.walks[b][K][1][0] = L_walks<BLK, STK, true, false>;
+    t.walks[b][K][0][1] = L_walks<BLK, STK, false, true>;
+    t.walks[b][K][1][1] = L_walks<BLK, STK, true, true>;
     t.extend[b][K][0] = L_extend<BLK, STK, false, false>;
     t.extend[b][K][1] = L_extend<BLK, STK, false, true>;
     t.extend_count[b][K][0] = L_extend<BLK, STK, true, false>;

@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 
 import little_renderer_amd as lr
+from glow_scenes import glow_scene
 from oracle import lro
 
 pytestmark = pytest.mark.gpu
@@ -72,6 +73,29 @@ def test_more_jobs_in_a_tile_than_a_work_group_counts_apart(world):
     for j, g, (w, h) in zip(jobs, got, sizes):
         assert np.array_equal(g, image(eng, eng.plain(j), w, h))
     eng.close()
+
+
+@pytest.mark.parametrize("graphs", [1, 2, 5])
+def test_a_scene_of_several_lights_joins_while_shadow_rays_wait(world, graphs):
+    # shadow rays wait for the next iteration's walks: those a one-light shade left are walked by the
+    # kernels for several lights and two-level scenes once a job that needs them is submitted
+    ctx, ps = world
+    _, (mtris, first, mats, inst) = glow_scene(box=True)
+    glow = lr.PtScene.instanced(ctx, mtris, first, mats, inst, eps=2e-3)
+    glow.set_sky(lr.sky(64))
+    eng = lr.Engine(ctx, slots_log2=15, max_tree_depth=max(64, ps.info()[0], glow.info()[0]), image_bytes=16 << 20)
+    eng.tune = {"iters_per_graph": 1}
+    a = lr.make_job(ps, lr.batch_camera(11, 190, 110), 190, 110, 3, seed=1)
+    b = lr.make_job(glow, lr.camera_make((-200, 20, 0), (0, 20, 0), (0, 1, 0), 40.0, 1.5), 90, 60, 2, seed=2)
+    i = eng.submit(a)
+    eng.pump(graphs)
+    j = eng.submit(b)
+    eng.drain()
+    got = image(eng, i, 190, 110), image(eng, j, 90, 60)
+    assert np.array_equal(got[0], image(eng, eng.plain(a), 190, 110))
+    assert np.array_equal(got[1], image(eng, eng.plain(b), 90, 60))
+    eng.close()
+    glow.close()
 
 
 @pytest.mark.parametrize("block_shade", [64, 128, 256])
