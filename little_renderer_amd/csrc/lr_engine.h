@@ -112,7 +112,7 @@ struct EngCtl {
     unsigned int spar;                      // the parity of the queue shade appended to: the next walks'
     unsigned int ordered;                   // that queue's first entries that regen put in perm's order (else 0)
     unsigned int qpar, qlen;                // the queue the walks went through, for shade: parity, length
-    unsigned int pad0;
+    unsigned int overflow;                  // a walk's stack ran out (1), or met a scene not its own (2)
     unsigned long long pad[2];
 };
 

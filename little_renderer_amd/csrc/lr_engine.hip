@@ -163,7 +163,7 @@ struct LrhEngine {
     EngProgress *prog = nullptr;
     JobDev *jobs = nullptr;
     unsigned long long *iq_start = nullptr, *counts = nullptr, *clk = nullptr;
-    uint32_t *iq_job = nullptr, *iq_q0 = nullptr, *overflow = nullptr;
+    uint32_t *iq_job = nullptr, *iq_q0 = nullptr;
     EngArgs base{};
     // host
     EngProgress *pin[2] = {nullptr, nullptr};
@@ -172,6 +172,7 @@ struct LrhEngine {
     unsigned long long seq[2] = {0, 0}, seq_next = 0;
     int pk = 0;
     EngProgress last{};
+    unsigned long long last_seq = 0;    // (last is the snapshot of this number, if any was taken)
     HostJob hj[LR_JOBS];
     std::map<size_t, size_t> free_blocks;      // arena: offset -> bytes
     std::map<int64_t, int> by_id;
@@ -347,6 +348,7 @@ void pilot_decide(LrhEngine *e, int slot, const long long *sums)
 void absorb(LrhEngine *e, const EngProgress &p, unsigned long long seq)
 {
     e->last = p;
+    e->last_seq = seq;
     for (int s = 0; s < LR_JOBS; s++) {
         HostJob &j = e->hj[s];
         if (j.state != LRH_JOB_RUNNING || seq < j.min_seq) continue;
@@ -391,11 +393,10 @@ int progress_flush(LrhEngine *e)
     return rc;
 }
 
+// the walks' overflow flags, as the last snapshot has them (taken after everything launched)
 int check_overflow(LrhEngine *e)
 {
-    uint32_t f = 0;
-    ENG_HIP(hipMemcpyAsync(&f, e->overflow, 4, hipMemcpyDeviceToHost, e->stream));
-    ENG_HIP(hipStreamSynchronize(e->stream));
+    const uint32_t f = e->last.ctl.overflow;
     if (f & 2u) return lr_fail(LRH_EDEVICE, "engine: a two-level scene's ray reached a one-level walk");
     if (f) return lr_fail(LRH_EREFUSED, "engine: a walk needed more stack than the engine's tree depth allows");
     return 0;
@@ -600,7 +601,7 @@ int job_admit(LrhEngine *e, const LrhJob *j, int *slot_out)
         // between the graphs' kernels)
         const size_t threads = std::min((npix + 255) / 256 * 256, (size_t)e->threads_cap / 256 * 256);
         table().guide[s->two_level ? 1 : 0](dim3((unsigned)(threads / 256)), e->stream, jd, (float4 *)jd.guide, e->base.spill,
-                                             threads, e->spill_cap, e->base.tab, e->overflow);
+                                             threads, e->spill_cap, e->base.tab, e->base.overflow);
         ENG_HIP(hipGetLastError());
     }
     if (caustics) {
@@ -617,7 +618,7 @@ int job_admit(LrhEngine *e, const LrhJob *j, int *slot_out)
         const uint64_t chunk = std::min<uint64_t>(LR_LIGHT_CHUNK, (uint64_t)e->threads_cap / 256 * 256);
         for (uint64_t g0 = 0; g0 < (uint64_t)paths; g0 += chunk) {
             const uint32_t n = (uint32_t)std::min<uint64_t>(chunk, (uint64_t)paths - g0);
-            table().light[e->counting ? 1 : 0](e->stream, jd, nlp, g0, n, e->base.spill, e->spill_cap, e->base.tab, e->overflow,
+            table().light[e->counting ? 1 : 0](e->stream, jd, nlp, g0, n, e->base.spill, e->spill_cap, e->base.tab, e->base.overflow,
                                                 e->lq, e->lqn, e->counts + 10);
             ENG_HIP(hipGetLastError());
         }
@@ -675,6 +676,24 @@ int top_up(LrhEngine *e)
     return 0;
 }
 
+// The iterations after which every admitted job is done, where that is known: all paths issued, none
+// waiting for a place in the pool (the last snapshot's count of those not yet retired fits it), so
+// each starts in the next iteration at the latest and has its max_depth + 1 vertices shaded in as many
+// iterations (the last makes no shadow ray). 0: not known.
+int tail_iterations(const LrhEngine *e)
+{
+    unsigned long long left = 0;
+    int depth = 0;
+    for (int s = 0; s < LR_JOBS; s++) {
+        const HostJob &h = e->hj[s];
+        if (h.state != LRH_JOB_RUNNING) continue;
+        if (h.pilot || h.issued < h.total) return 0;
+        left += h.total - (e->last_seq >= h.min_seq ? e->last.jret[s] : 0);
+        depth = std::max(depth, std::min(h.desc.max_depth, 1 << 20));
+    }
+    return left <= e->C ? depth + 1 : 0;
+}
+
 int job_slot(const LrhEngine *e, int64_t id)
 {
     auto it = e->by_id.find(id);
@@ -712,10 +731,9 @@ int lr_engine_create(LrhContext *c, int slots_log2, int max_tree_depth, size_t i
         C * 32, C * 32, C * 4, C * 4, C * 16,                                        // 9..13 qray qray qid qid hits
         C * 32, C * 4, C * 16,                                                       // 14..16 sray sid scon
         e->threads_cap * (size_t)(e->spill_cap > 0 ? e->spill_cap : 1) * 4,          // 17 spill
-        2112 * 4, 4096 * 2, 256, 256, 256,                                           // 18..22 tab mask counts clk overflow
+        2112 * 4, 4096 * 2, 256, 256, C * 4,                                         // 18..22 tab mask counts clk perm
         LR_ISSUE * 4, (C / 64 + 4) * 8, C * 16,                                      // 23 iq_q0, 24 ostat, 25 srad
-        2 * C * 32, 2 * C * 16, C * 4,                                               // 26..28 xsray xscon sx
-        C * 4};                                                                      // 29 perm
+        2 * C * 32, 2 * C * 16, C * 4};                                              // 26..28 xsray xscon sx
     constexpr int NS = sizeof(sizes) / sizeof(sizes[0]);
     size_t total = 0;
     for (size_t z : sizes) total += lr_align(z);
@@ -740,7 +758,6 @@ int lr_engine_create(LrhContext *c, int slots_log2, int max_tree_depth, size_t i
     e->iq_q0 = (uint32_t *)p[23];
     e->counts = (unsigned long long *)p[20];
     e->clk = (unsigned long long *)p[21];
-    e->overflow = (uint32_t *)p[22];
     EngArgs &A = e->base;
     A.ctl = &e->prog->ctl;
     A.jobs = e->jobs;
@@ -763,7 +780,7 @@ int lr_engine_create(LrhContext *c, int slots_log2, int max_tree_depth, size_t i
         A.xscon[b] = (float4 *)p[27] + b * C;
     }
     A.sx = (uint32_t *)p[28];
-    A.perm = (uint32_t *)p[29];
+    A.perm = (uint32_t *)p[22];
     A.qray[0] = (float4 *)p[9];
     A.qray[1] = (float4 *)p[10];
     A.qid[0] = (uint32_t *)p[11];
@@ -777,7 +794,7 @@ int lr_engine_create(LrhContext *c, int slots_log2, int max_tree_depth, size_t i
     A.mask = (const uint16_t *)p[19];
     A.counts = e->counts;
     A.ostat = (unsigned long long *)p[24];
-    A.overflow = e->overflow;
+    A.overflow = &e->prog->ctl.overflow;
     A.mult = 1;
     std::vector<float> tab(2112);
     std::vector<uint16_t> mask(4096);
@@ -933,10 +950,26 @@ int lrh_engine_pump(LrhEngine *e, int graphs)
 int lrh_engine_drain(LrhEngine *e)
 {
     if (!e) return lr_fail(LRH_EINVAL, "lrh_engine_drain: no engine");
+    (void)hipSetDevice(e->device);
     unsigned long long seen = ~0ull;
     int still = 0;
     while (e->running > 0) {
-        int rc = lrh_engine_pump(e, 1);
+        int rc = make_graph(e);
+        if (!rc) rc = top_up(e);
+        if (rc) return rc;
+        const int G = e->tune.iters_per_graph, tail = e->profiling ? 0 : tail_iterations(e);
+        if (tail > 0 && tail <= 4 * G) {
+            // the end is in sight: as many iterations as it takes and no graph past them (whole graphs,
+            // then kernels), instead of finding out from snapshots a graph or two late
+            for (int g = 0; g < tail / G; g++) {
+                hipError_t le = hipGraphLaunch(e->gexec, e->stream);
+                if (le != hipSuccess) return eng_fail_dev("hipGraphLaunch", le);
+            }
+            for (int i = 0; i < tail % G; i++) launch_iteration(e, e->tune);
+            ENG_HIP(hipGetLastError());
+            rc = progress_enqueue(e);
+            if (!rc) rc = progress_flush(e);
+        } else rc = lrh_engine_pump(e, 1);
         if (rc < 0) return rc;
         // a stall (no path retired over many graphs) would be a defect: said, not waited on
         const unsigned long long t = e->last.ctl.tail;
