@@ -36,11 +36,11 @@ constexpr int SORT_WAVES = SORT_BLOCK / 64;
 constexpr int SORT_PASSES = 4;                  // 30-bit codes: bits 0-7, 8-15, 16-23, 24-29
 constexpr int HIST_COPIES = 8;                  // one global histogram per XCD (less contention)
 constexpr int PLOC_R = 16;
-constexpr int PLOC_PER = 2;                     // positions a thread takes in a PLOC round
-constexpr int PLOC_TILE = 256 * PLOC_PER;        // positions a work-group takes (one claim)
-constexpr int PLOC_WIN = PLOC_TILE + 4 * PLOC_R;   // boxes of positions base-2R .. base+PLOC_TILE+2R
-constexpr int PLOC_NN = PLOC_TILE + 2 * PLOC_R;    // nearest of positions base-R .. base+PLOC_TILE+R
 constexpr int PLOC_MAX_ROUNDS = 128;
+// the clusters (estimated) from which a round takes 4 positions a lane (fewer instructions a pair) rather
+// than 2 (more waves, each sooner done): at 114k 12.2 against 12.5 us, at 400k 19 against 27, below
+// 50k 11 against 8
+constexpr int PLOC_BIG = 1 << 17;
 constexpr int BOUNDS_BLOCKS = 512;
 
 constexpr uint32_t FLAG_AGG = 1u << 30;
@@ -669,7 +669,8 @@ struct PlocState {
     uint32_t nc;          // clusters in the current list
     uint32_t parity;      // which of the two lists is current
     uint64_t live;        // the live clusters summed over the rounds (the build's traffic)
-    uint32_t pad[60];
+    uint32_t made;        // the rounds k_ploc_round made (a launch may find nothing left to do)
+    uint32_t pad[59];
     uint32_t ctr[PLOC_MAX_ROUNDS];   // each round's tile counter
 };
 
@@ -698,25 +699,26 @@ __device__ __forceinline__ void put_final(LrNode *slot, uint32_t x, float4 lo, f
     else put_node(slot, lo.x, lo.y, lo.z, ref0 + x - (n - 1u), hi.x, hi.y, hi.z, 0x80000001u);
 }
 
-// merge (trace_ploc.wgsl:39-46): clusters c (the lower position) and d into internal k
+// merge (trace_ploc.wgsl:39-46): clusters c (the lower position) and d into internal k. A cluster's
+// box carries its height in its first word's fourth place (one load less for each side of a merge)
+__device__ __forceinline__ uint32_t height_of(float4 lo) { return __float_as_uint(lo.w); }
 __device__ __forceinline__ void ploc_merge(uint32_t k, uint32_t c, float4 clo, float4 chi, uint32_t d, float4 dlo, float4 dhi,
-                                           uint32_t n, uint32_t node0, uint32_t ref0, float4 *bx, LrNode *nodes, uint32_t *height)
+                                           uint32_t n, uint32_t node0, uint32_t ref0, float4 *bx, LrNode *nodes)
 {
-    const float4 lo = make_float4(wmin(clo.x, dlo.x), wmin(clo.y, dlo.y), wmin(clo.z, dlo.z), 0.0f);
+    const float4 lo = make_float4(wmin(clo.x, dlo.x), wmin(clo.y, dlo.y), wmin(clo.z, dlo.z),
+                                  __uint_as_float(1u + max(height_of(clo), height_of(dlo))));
     const float4 hi = make_float4(wmax(chi.x, dhi.x), wmax(chi.y, dhi.y), wmax(chi.z, dhi.z), 0.0f);
     bx[2 * (size_t)k] = lo;
     bx[2 * (size_t)k + 1] = hi;
     put_final(&nodes[1 + 2 * (size_t)k], c, clo, chi, n, node0, ref0);
     put_final(&nodes[2 + 2 * (size_t)k], d, dlo, dhi, n, node0, ref0);
-    const uint32_t hc = height[c], hd = height[d];
-    height[k] = 1 + (hc > hd ? hc : hd);
     if (k == 0) put_node(&nodes[0], lo.x, lo.y, lo.z, node0 + 1u, hi.x, hi.y, hi.z, node0 + 2u);
 }
 
 // init (trace_ploc.wgsl:68-82): the leaves in Morton order are the first clusters
 __global__ __launch_bounds__(BLOCK) void k_ploc_init(const uint32_t *__restrict__ items, const float4 *__restrict__ boxes, int n,
                                                        uint32_t ref0, uint32_t ref_add, uint32_t *aux, float4 *bx, uint32_t *list0,
-                                                       uint32_t *height, PlocState *st, uint64_t *status, size_t status_words)
+                                                       PlocState *st, uint64_t *status, size_t status_words)
 {
     const size_t g = blockIdx.x * (size_t)BLOCK + threadIdx.x;
     for (size_t i = g; i < status_words; i += (size_t)gridDim.x * BLOCK) status[i] = 0;
@@ -725,96 +727,244 @@ __global__ __launch_bounds__(BLOCK) void k_ploc_init(const uint32_t *__restrict_
     const int i = (int)g;
     const uint32_t item = items[i];
     const size_t x = (size_t)n - 1 + i;
-    bx[2 * x] = boxes[2 * (size_t)item];
+    const float4 lo = boxes[2 * (size_t)item];
+    bx[2 * x] = make_float4(lo.x, lo.y, lo.z, __uint_as_float(1u));
     bx[2 * x + 1] = boxes[2 * (size_t)item + 1];
     aux[i] = item + ref_add;
-    height[x] = 1;
     list0[i] = (uint32_t)x;
 }
 
-// the nearest of position i (< nc) among the window held in LDS: wlo/whi[l] is position base - 2R + l
-__device__ __forceinline__ uint32_t nearest_in(int i, int base, uint32_t nc, const float4 *wlo, const float4 *whi)
+// The nearest search of a wave, P adjacent positions a lane (their boxes b: three lows, three highs).
+// Each pair i, i + k (k <= R) is measured once, for both: by the lane of i, against a copy of the
+// boxes that turns by one lane after another, along with the best found so far for its positions
+// from below. No memory is read, and a distance serves two positions: 11 to 14 instructions a position
+// and neighbour, where a search of R neighbours a side from LDS took about 40 and waited for each. off: the nearest as an offset (0: none) by
+// nearer's order (of equal ones the lower position), right for the wave's positions that have all
+// R neighbours in it on either side (the others' are not to be used). Where there is no position,
+// NEAR_NONE boxes: their distances are infinite and never taken. Floats compare as in nearer but
+// for NaN, so boxes must be `measurable`; others take nearest_in.
+constexpr float NEAR_NONE = 1e30f;   // lows -, highs +: the area overflows
+__device__ __forceinline__ bool measurable(float lx, float ly, float lz, float hx, float hy, float hz)
 {
-    const int li = i - base + 2 * PLOC_R;
-    const float4 lo = wlo[li], hi = whi[li];
-    const int j0 = i - PLOC_R > 0 ? i - PLOC_R : 0;
-    const int j1 = i + PLOC_R < (int)nc - 1 ? i + PLOC_R : (int)nc - 1;
+    // finite, and any two boxes' area finite: at most 3 (2e18)^2
+    return fabsf(lx) + fabsf(ly) + fabsf(lz) + fabsf(hx) + fabsf(hy) + fabsf(hz) <= 1e18f;
+}
+__device__ __forceinline__ float turn_lane(float v)   // lane l gets lane l + 1's, the last the first's
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x134, 0xf, 0xf, true));
+}
+__device__ __forceinline__ int turn_lane(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x134, 0xf, 0xf, true); }
+
+template <int P>
+__device__ __forceinline__ void nearest_wave(const float (&b)[6][P], int (&off)[P])
+{
+    static_assert(PLOC_R % P == 0, "a lane's positions divide the radius");
+    const float inf = __builtin_inff();
+    float s[6][P], fd[P], sd[P];   // the turning boxes; the best distance above, below
+    int fk[P], sk[P];
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+        for (int c = 0; c < 6; c++) s[c][q] = b[c][q];
+        fd[q] = sd[q] = inf;
+        fk[q] = sk[q] = 0;
+    }
+#pragma unroll
+    for (int t = 0; t <= PLOC_R / P; t++) {
+        if (t > 0) {
+#pragma unroll
+            for (int q = 0; q < P; q++) {
+                for (int c = 0; c < 6; c++) s[c][q] = turn_lane(s[c][q]);
+                sd[q] = turn_lane(sd[q]);
+                sk[q] = turn_lane(sk[q]);
+            }
+        }
+        // (in this order both sides see their distances by rising k: above, the first of equal
+        // ones is the lower position; below, the last)
+#pragma unroll
+        for (int r = P - 1; r >= 0; r--)
+#pragma unroll
+            for (int q = 0; q < P; q++) {
+                const int k = t * P + q - r;
+                if (k < 1 || k > PLOC_R) continue;
+                const float d = half_area(fminf(b[0][r], s[0][q]), fminf(b[1][r], s[1][q]), fminf(b[2][r], s[2][q]),
+                                          fmaxf(b[3][r], s[3][q]), fmaxf(b[4][r], s[4][q]), fmaxf(b[5][r], s[5][q]));
+                if (d < fd[r]) { fd[r] = d; fk[r] = k; }
+                if (d <= sd[q]) { sd[q] = d; sk[q] = k; }
+            }
+    }
+    const int home = ((int)(threadIdx.x & 63u) - PLOC_R / P) & 63;
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+        const float bd = __shfl(sd[q], home, 64);
+        const int bk = __shfl(sk[q], home, 64);
+        off[q] = bd <= fd[q] ? (bd < inf ? -bk : 0) : fk[q];
+    }
+}
+
+// the offset to the nearest of position i (< nc) in a list of nc whose boxes are l[0..5][at + position]:
+// any boxes, NaN too
+template <class Arr>
+__device__ int nearest_in(int i, int nc, int at, const Arr &l)
+{
+    const int j0 = max(i - PLOC_R, 0), j1 = min(i + PLOC_R, nc - 1);
+    const int li = at + i;
     float bd = 0.0f;
     uint32_t bj = LR_NONE;
     for (int j = j0; j <= j1; j++) {
         if (j == i) continue;
-        const int lj = j - base + 2 * PLOC_R;
-        const float4 ol = wlo[lj], oh = whi[lj];
-        const float d = half_area(wmin(lo.x, ol.x), wmin(lo.y, ol.y), wmin(lo.z, ol.z),
-                                  wmax(hi.x, oh.x), wmax(hi.y, oh.y), wmax(hi.z, oh.z));
+        const int lj = at + j;
+        const float d = half_area(wmin(l[0][li], l[0][lj]), wmin(l[1][li], l[1][lj]), wmin(l[2][li], l[2][lj]),
+                                  wmax(l[3][li], l[3][lj]), wmax(l[4][li], l[4][lj]), wmax(l[5][li], l[5][lj]));
         if (nearer(d, (uint32_t)i, (uint32_t)j, bd, bj)) { bd = d; bj = (uint32_t)j; }
     }
-    return bj;
+    return bj == LR_NONE ? 0 : (int)bj - i;
+}
+
+// The nearest of the positions i0 .. i0 + 64 P - 2R of a list of nc, by one wave, as offsets to
+// nn[i - i0], from boxes in LDS (l[c][at + position]; readable from position i0 - R to
+// i0 + 64 P - R, whatever they hold where there is none). at + i0 - R is a multiple of P.
+template <int P, class Arr>
+__device__ __forceinline__ void nearest_range(int i0, int nc, int at, const Arr &l, int8_t *nn)
+{
+    const int lane = (int)(threadIdx.x & 63u), p0 = i0 - PLOC_R + P * lane;
+    float b[6][P];
+    bool bad = false;
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+        struct alignas(4 * P) Row { float v[P]; };
+        const Row row = *reinterpret_cast<const Row *>(&l[c][at + p0]);
+#pragma unroll
+        for (int q = 0; q < P; q++) b[c][q] = row.v[q];
+    }
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+        const bool is = p0 + q >= 0 && p0 + q < nc;
+        bad |= is && !measurable(b[0][q], b[1][q], b[2][q], b[3][q], b[4][q], b[5][q]);
+#pragma unroll
+        for (int c = 0; c < 6; c++) b[c][q] = is ? b[c][q] : c < 3 ? -NEAR_NONE : NEAR_NONE;
+    }
+    if (__any(bad)) {
+        for (int o = lane; o < 64 * P - 2 * PLOC_R; o += 64)
+            if (i0 + o >= 0 && i0 + o < nc) nn[o] = (int8_t)nearest_in(i0 + o, nc, at, l);
+        return;
+    }
+    int off[P];
+    nearest_wave<P>(b, off);
+#pragma unroll
+    for (int q = 0; q < P; q++) {
+        const int o = P * lane + q - PLOC_R;
+        if (o >= 0 && o < 64 * P - 2 * PLOC_R && i0 + o >= 0 && i0 + o < nc) nn[o] = (int8_t)off[q];
+    }
+}
+
+// The places of a thread's positions among a work-group's that stay and that merge (high and low 16
+// bits; PER adjacent positions a thread, so the order is the positions'), from ballots: `total`
+// the work-group's, by one barrier. wsum (NW words) is free again at the caller's next barrier.
+template <int NW, int PER>
+__device__ __forceinline__ uint32_t places(const bool (&keep)[PER], const bool (&merge)[PER], uint32_t *total, uint32_t *wsum)
+{
+    uint32_t before = 0, sum = 0;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const uint64_t kb = __ballot(keep[q]), mb = __ballot(merge[q]);
+        before += (__builtin_amdgcn_mbcnt_hi((uint32_t)(kb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kb, 0u)) << 16) +
+                  __builtin_amdgcn_mbcnt_hi((uint32_t)(mb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mb, 0u));
+        sum += ((uint32_t)__popcll(kb) << 16) + (uint32_t)__popcll(mb);
+    }
+    if constexpr (NW > 1) {
+        const uint32_t w = threadIdx.x >> 6;
+        if ((threadIdx.x & 63u) == 0) wsum[w] = sum;
+        __syncthreads();
+        sum = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < NW; k++) {
+            const uint32_t v = wsum[k];
+            before += k < w ? v : 0u;
+            sum += v;
+        }
+    }
+    *total = sum;
+    return before;
 }
 
 // One PLOC round (nn + mark + top + scatter of trace_ploc.wgsl:84-234 in one kernel): tiles of
-// 256 positions taken in order from a counter; each loads the boxes of its positions +- 2R
+// positions taken in order from a counter; each loads the boxes of its positions +- 2R
 // into LDS, finds the nearest of positions +- R, marks who stays and who merges, takes its
 // place in the next list from the tiles before it (look-back), writes the merged nodes and
-// its part of the next list. Blocks loop over tiles, so any grid size covers the round.
-__global__ __launch_bounds__(BLOCK, 7) void k_ploc_round(int round, int n, uint32_t small, uint32_t node0, uint32_t ref0,
+// its part of the next list. Blocks loop over tiles, so any grid size covers the round. Large rounds
+// are bound by their claims, gathers and searches together (1M clusters: 94 -> 45 us), small ones by
+// the chain of one tile (launch, claim, list, boxes, search, look-back: 26 -> 8 us, of which the search
+// was half); a grid short of the tiles made a round twice as long (49 us).
+constexpr int ploc_tile(int P) { return (BLOCK / 64) * (64 * P - 2 * PLOC_R) - 2 * PLOC_R; }   // 864 of P = 4, 352 of P = 2
+constexpr int PLOC_CLEAR = (ploc_tile(4) + ploc_tile(2) - 1) / ploc_tile(2);   // the next round's tiles a tile may stand for
+
+template <int P>
+__global__ __launch_bounds__(BLOCK, 4) void k_ploc_round(int round, int n, uint32_t small, uint32_t node0, uint32_t ref0,
                                                         float4 *bx, uint32_t *list0, uint32_t *list1, LrNode *nodes,
-                                                        uint32_t *height, PlocState *st, uint64_t *status0, uint64_t *status1)
+                                                        PlocState *st, uint64_t *status0, uint64_t *status1, uint32_t status_n)
 {
-    __shared__ float4 wlo[PLOC_WIN], whi[PLOC_WIN];
-    __shared__ uint32_t wid[PLOC_WIN];
-    __shared__ int8_t snn[PLOC_NN];   // the nearest as an offset from the position (within +-R; 0: none)
+    constexpr int TILE = ploc_tile(P), WIN = TILE + 4 * PLOC_R, NN = TILE + 2 * PLOC_R, RANGE = 64 * P - 2 * PLOC_R;
+    constexpr int PER = (TILE + BLOCK - 1) / BLOCK, LOADS = (WIN + BLOCK - 1) / BLOCK;
+    __shared__ __attribute__((aligned(16))) float l[6][WIN];
+    __shared__ uint32_t wid[WIN], wh[WIN];
+    __shared__ int8_t snn[NN];   // the nearest as an offset from the position (within +-R; 0: none)
     __shared__ uint32_t s_wsum[BLOCK / 64];
     __shared__ uint32_t s_tile, s_ek, s_em;
     const int tid = threadIdx.x;
     for (;;) {
         if (tid == 0) s_tile = atomicAdd(&st->ctr[round], 1u);
+        // (beside the claim: the round's last tile changes them, once every tile of the round is claimed)
+        const uint32_t nc = ld_dev(&st->nc), p = ld_dev(&st->parity);
         __syncthreads();
         const uint32_t tile = s_tile;
-        const uint32_t nc = ld_dev(&st->nc), p = ld_dev(&st->parity);
-        const uint32_t ntiles = (nc + PLOC_TILE - 1) / PLOC_TILE;
+        const uint32_t ntiles = (nc + TILE - 1) / TILE;
         if (nc <= small || tile >= ntiles) return;
         const uint32_t *cur = p ? list1 : list0;
         uint32_t *nxt = p ? list0 : list1;
         uint64_t *status = p ? status1 : status0;
         uint64_t *status_next = p ? status0 : status1;
-        if (tid == 0) status_next[tile] = 0;       // (the next round's, cleared for it)
-        const int base = (int)tile * PLOC_TILE;
-        for (int l = tid; l < PLOC_WIN; l += BLOCK) {
-            const int g = base - 2 * PLOC_R + l;
-            if (g >= 0 && g < (int)nc) {
-                const uint32_t x = cur[g];
-                wid[l] = x;
-                wlo[l] = bx[2 * (size_t)x];
-                whi[l] = bx[2 * (size_t)x + 1];
-            }
-        }
-        __syncthreads();
-        for (int q = tid; q < PLOC_NN; q += BLOCK) {
-            const int i = base - PLOC_R + q;
-            const uint32_t bj = (i >= 0 && i < (int)nc) ? nearest_in(i, base, nc, wlo, whi) : LR_NONE;
-            snn[q] = bj == LR_NONE ? (int8_t)0 : (int8_t)((int)bj - i);
-        }
-        __syncthreads();
-        // keep_merge (trace_ploc.wgsl:130-145): PLOC_PER adjacent positions a thread, so that the
-        // scans of the threads' sums keep the positions' order
-        uint32_t j[PLOC_PER], keep[PLOC_PER], merge[PLOC_PER], kc = 0, mc = 0;
+        // (the next round's, cleared for it: it may have smaller tiles)
+        if (tid < PLOC_CLEAR && tile * PLOC_CLEAR + tid < status_n) status_next[tile * PLOC_CLEAR + tid] = 0;
+        const int base = (int)tile * TILE;
+        uint32_t x[LOADS];
 #pragma unroll
-        for (int q = 0; q < PLOC_PER; q++) {
-            const int o = PLOC_PER * tid + q, i = base + o;
-            const bool valid = i < (int)nc;
+        for (int q = 0; q < LOADS; q++) {
+            const int o = tid + q * BLOCK, g = base - 2 * PLOC_R + o;
+            x[q] = o < WIN && g >= 0 && g < (int)nc ? cur[g] : LR_NONE;
+        }
+#pragma unroll
+        for (int q = 0; q < LOADS; q++) {
+            const int o = tid + q * BLOCK;
+            if (x[q] == LR_NONE) continue;
+            const float4 lo = bx[2 * (size_t)x[q]], hi = bx[2 * (size_t)x[q] + 1];
+            wid[o] = x[q];
+            wh[o] = height_of(lo);
+            l[0][o] = lo.x; l[1][o] = lo.y; l[2][o] = lo.z;
+            l[3][o] = hi.x; l[4][o] = hi.y; l[5][o] = hi.z;
+        }
+        __syncthreads();
+        {
+            const int w = tid >> 6;
+            nearest_range<P>(base - PLOC_R + w * RANGE, (int)nc, 2 * PLOC_R - base, l, snn + w * RANGE);
+        }
+        __syncthreads();
+        // keep_merge (trace_ploc.wgsl:130-145)
+        uint32_t j[PER];
+        bool keep[PER], merge[PER];
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            const int o = PER * tid + q, i = base + o;
+            const bool valid = o < TILE && i < (int)nc;
             const int dj = valid ? (int)snn[o + PLOC_R] : 0;
             j[q] = dj != 0 ? (uint32_t)(i + dj) : LR_NONE;
             bool mu = false;
             if (j[q] < nc) mu = (int)j[q] + (int)snn[(int)j[q] - base + PLOC_R] == i;
             keep[q] = valid && !(mu && (uint32_t)i > j[q]);
             merge[q] = valid && mu && (uint32_t)i < j[q];
-            kc += keep[q];
-            mc += merge[q];
         }
-        uint32_t tk, tm;
-        const uint32_t xk = block_excl_scan<BLOCK / 64>(kc, &tk, s_wsum);
-        const uint32_t xm = block_excl_scan<BLOCK / 64>(mc, &tm, s_wsum);
+        uint32_t both;
+        const uint32_t xkm = places<BLOCK / 64>(keep, merge, &both, s_wsum);
+        const uint32_t xk = xkm >> 16, xm = xkm & 0xffffu, tk = both >> 16, tm = both & 0xffffu;
         if (tid < 64) {
             // the look-back by the first wave, 64 predecessor tiles at once (lane l: tile t - l):
             // the nearest inclusive prefix among them ends it; a needed tile not yet posted means
@@ -857,22 +1007,26 @@ __global__ __launch_bounds__(BLOCK, 7) void k_ploc_round(int round, int n, uint3
                     st_dev(&st->nc, (uint32_t)ek + tk);
                     st_dev(&st->parity, 1u - p);
                     st_dev64(&st->live, ld_dev64(&st->live) + nc);   // (one writer a round)
+                    st_dev(&st->made, ld_dev(&st->made) + 1u);
                 }
             }
         }
         __syncthreads();
         uint32_t dk = s_ek + xk, dm = s_em + xm;
 #pragma unroll
-        for (int q = 0; q < PLOC_PER; q++) {
+        for (int q = 0; q < PER; q++) {
             if (!keep[q]) continue;
-            const int li = PLOC_PER * tid + q + 2 * PLOC_R;
+            const int li = PER * tid + q + 2 * PLOC_R;
             const uint32_t c = wid[li];
             uint32_t out = c;
             if (merge[q]) {
                 const int lj = (int)j[q] - base + 2 * PLOC_R;
                 const uint32_t k = ((uint32_t)n - 2u) - ((uint32_t)n - nc + dm);
                 dm++;
-                ploc_merge(k, c, wlo[li], whi[li], wid[lj], wlo[lj], whi[lj], (uint32_t)n, node0, ref0, bx, nodes, height);
+                ploc_merge(k, c, make_float4(l[0][li], l[1][li], l[2][li], __uint_as_float(wh[li])),
+                           make_float4(l[3][li], l[4][li], l[5][li], 0.0f), wid[lj],
+                           make_float4(l[0][lj], l[1][lj], l[2][lj], __uint_as_float(wh[lj])),
+                           make_float4(l[3][lj], l[4][lj], l[5][lj], 0.0f), (uint32_t)n, node0, ref0, bx, nodes);
                 out = k;
             }
             nxt[dk++] = out;
@@ -882,41 +1036,109 @@ __global__ __launch_bounds__(BLOCK, 7) void k_ploc_round(int round, int n, uint3
 }
 
 // small (trace_ploc.wgsl:236-301): the rounds left, in one workgroup, from 1024 clusters (the
-// context's ploc_small: below it a round's launch costs more than its work; above it the
-// nearest search, bound by one compute unit's VALU, is better spread over the chip). While
+// context's ploc_small: below it a round's launch costs more than its work). While
 // more than SMALL_MAX clusters are left (only when the rounds before could not merge enough:
 // boxes that tie everywhere merge one pair a round) a round goes through device memory; from
-// SMALL_MAX down, the list, its boxes (six arrays of floats) and heights live in LDS, the
-// nearest search reads its 2R neighbours there, and only the merged nodes' records go out.
+// SMALL_MAX down, the list, its boxes (six arrays of floats) and heights live in LDS, and only the
+// merged nodes' records go out. From 96 clusters down one wave goes on alone, without barriers:
+// most of the rounds are there. Bound by one compute unit's VALU down to some 100 clusters (3 waves
+// a SIMD search), then by the chain of a round (2 us): 5001 boxes' 292 -> 127 us.
 constexpr int SMALL_BLOCK = 1024;
 constexpr int SMALL_MAX = 4096;
-constexpr int SMALL_PER = SMALL_MAX / SMALL_BLOCK;   // positions a thread holds in an LDS round
+constexpr int SMALL_PAD = 64 * 2 + PLOC_R;   // LDS places around the list that a wave's search may read
+struct SmallLds {
+    __attribute__((aligned(16))) float b[6][SMALL_MAX + SMALL_PAD];   // position i at i + R
+    uint32_t id[SMALL_MAX], h[SMALL_MAX];
+    int8_t nn[SMALL_MAX];
+    uint32_t wsum[SMALL_BLOCK / 64];
+};
 
-// the nearest of position i among the LDS list of nc (positions +- R; the tie rule of nearer)
-__device__ __forceinline__ uint32_t nearest_lds(int i, int nc, const float *lx, const float *ly, const float *lz,
-                                                const float *hx, const float *hy, const float *hz)
+// one round of the list of nc in LDS by the first WAVES waves, P positions a lane in the search, PER a
+// thread after it; returns the clusters left
+template <int P, int PER, int WAVES>
+__device__ __forceinline__ uint32_t small_round(SmallLds &S, uint32_t nc, uint32_t n, uint32_t node0, uint32_t ref0, LrNode *nodes)
 {
-    const float ax = lx[i], ay = ly[i], az = lz[i], bx_ = hx[i], by = hy[i], bz = hz[i];
-    const int j0 = i - PLOC_R > 0 ? i - PLOC_R : 0;
-    const int j1 = i + PLOC_R < nc - 1 ? i + PLOC_R : nc - 1;
-    float bd = 0.0f;
-    uint32_t bj = LR_NONE;
-    for (int j = j0; j <= j1; j++) {
-        if (j == i) continue;
-        const float d = half_area(wmin(ax, lx[j]), wmin(ay, ly[j]), wmin(az, lz[j]), wmax(bx_, hx[j]), wmax(by, hy[j]),
-                                  wmax(bz, hz[j]));
-        if (nearer(d, (uint32_t)i, (uint32_t)j, bd, bj)) { bd = d; bj = (uint32_t)j; }
+    constexpr int RANGE = 64 * P - 2 * PLOC_R;
+    const int tid = threadIdx.x;
+    auto sync = [] {
+        if constexpr (WAVES == 1) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            // (LDS only: the records on their way out are not waited for)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        }
+    };
+    for (int i0 = (tid >> 6) * RANGE; i0 < (int)nc; i0 += WAVES * RANGE)
+        nearest_range<P>(i0, (int)nc, PLOC_R, S.b, S.nn + i0);
+    sync();
+    // each thread takes a run of positions, holds what it writes in registers, and writes after
+    // every read of the round is done
+    uint32_t j[PER];
+    bool keep[PER], merge[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int i = PER * tid + q;
+        keep[q] = merge[q] = false;
+        if (i >= (int)nc) continue;
+        const int dj = S.nn[i];
+        const bool mu = dj != 0 && S.nn[i + dj] == -dj;
+        j[q] = (uint32_t)(i + dj);
+        keep[q] = !(mu && dj < 0);
+        merge[q] = mu && dj > 0;
     }
-    return bj;
+    uint32_t both;
+    const uint32_t x = places<WAVES>(keep, merge, &both, S.wsum);
+    uint32_t dk = x >> 16, dm = x & 0xffffu;
+    uint32_t o_id[PER], o_h[PER];
+    float o_b[PER][6];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int i = PER * tid + q;
+        if (!keep[q]) continue;
+#pragma unroll
+        for (int c = 0; c < 6; c++) o_b[q][c] = S.b[c][PLOC_R + i];
+        o_id[q] = S.id[i];
+        o_h[q] = S.h[i];
+        if (!merge[q]) continue;
+        const uint32_t k = (n - 2u) - (n - nc + dm);
+        dm++;
+        float d[6];
+#pragma unroll
+        for (int c = 0; c < 6; c++) d[c] = S.b[c][PLOC_R + j[q]];
+        put_final(&nodes[1 + 2 * (size_t)k], o_id[q], make_float4(o_b[q][0], o_b[q][1], o_b[q][2], 0.0f),
+                  make_float4(o_b[q][3], o_b[q][4], o_b[q][5], 0.0f), n, node0, ref0);
+        put_final(&nodes[2 + 2 * (size_t)k], S.id[j[q]], make_float4(d[0], d[1], d[2], 0.0f), make_float4(d[3], d[4], d[5], 0.0f),
+                  n, node0, ref0);
+#pragma unroll
+        for (int c = 0; c < 6; c++) o_b[q][c] = c < 3 ? wmin(o_b[q][c], d[c]) : wmax(o_b[q][c], d[c]);
+        if (k == 0)
+            put_node(&nodes[0], o_b[q][0], o_b[q][1], o_b[q][2], node0 + 1u, o_b[q][3], o_b[q][4], o_b[q][5], node0 + 2u);
+        o_id[q] = k;
+        o_h[q] = 1u + max(o_h[q], S.h[j[q]]);
+    }
+    sync();
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        if (!keep[q]) continue;
+        S.id[dk] = o_id[q];
+        S.h[dk] = o_h[q];
+#pragma unroll
+        for (int c = 0; c < 6; c++) S.b[c][PLOC_R + dk] = o_b[q][c];
+        dk++;
+    }
+    sync();
+    return both >> 16;
 }
 
 __global__ __launch_bounds__(SMALL_BLOCK) void k_ploc_small(int n, uint32_t node0, uint32_t ref0, float4 *bx, uint32_t *list0,
-                                                              uint32_t *list1, uint32_t *nnbuf, LrNode *nodes, uint32_t *height,
-                                                              PlocState *st, uint32_t *rounds_out, uint32_t *depth_out)
+                                                              uint32_t *list1, uint32_t *nnbuf, LrNode *nodes,
+                                                              PlocState *st, int planned, uint32_t *rounds_out, uint32_t *depth_out)
 {
-    __shared__ uint32_t s_wsum[SMALL_BLOCK / 64];
-    __shared__ float s_lx[SMALL_MAX], s_ly[SMALL_MAX], s_lz[SMALL_MAX], s_hx[SMALL_MAX], s_hy[SMALL_MAX], s_hz[SMALL_MAX];
-    __shared__ uint32_t s_id[SMALL_MAX], s_nn[SMALL_MAX], s_h[SMALL_MAX];
+    __shared__ SmallLds S;
+    uint32_t *const s_wsum = S.wsum;
     const int tid = threadIdx.x;
     uint32_t nc = st->nc, p = st->parity;
     uint32_t rounds = 0;
@@ -967,7 +1189,7 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_ploc_small(int n, uint32_t node
                 const uint32_t k = ((uint32_t)n - 2u) - ((uint32_t)n - nc + dm);
                 dm++;
                 ploc_merge(k, c, bx[2 * (size_t)c], bx[2 * (size_t)c + 1], d, bx[2 * (size_t)d], bx[2 * (size_t)d + 1],
-                           (uint32_t)n, node0, ref0, bx, nodes, height);
+                           (uint32_t)n, node0, ref0, bx, nodes);
                 out = k;
             }
             nxt[dk++] = out;
@@ -989,80 +1211,28 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_ploc_small(int n, uint32_t node
         for (int i = tid; i < (int)nc; i += SMALL_BLOCK) {
             const uint32_t x = cur[i];
             const float4 lo = bx[2 * (size_t)x], hi = bx[2 * (size_t)x + 1];
-            s_id[i] = x;
-            s_lx[i] = lo.x; s_ly[i] = lo.y; s_lz[i] = lo.z;
-            s_hx[i] = hi.x; s_hy[i] = hi.y; s_hz[i] = hi.z;
-            s_h[i] = height[x];
+            S.id[i] = x;
+            S.h[i] = height_of(lo);
+            S.b[0][PLOC_R + i] = lo.x; S.b[1][PLOC_R + i] = lo.y; S.b[2][PLOC_R + i] = lo.z;
+            S.b[3][PLOC_R + i] = hi.x; S.b[4][PLOC_R + i] = hi.y; S.b[5][PLOC_R + i] = hi.z;
         }
         __syncthreads();
     }
+    constexpr int WAVES = SMALL_BLOCK / 64;
     while (nc > 1) {
+        if (nc <= 96 && tid >= 64) return;   // one wave goes on
+        const uint32_t left = nc > SMALL_BLOCK ? small_round<2, SMALL_MAX / SMALL_BLOCK, WAVES>(S, nc, (uint32_t)n, node0, ref0, nodes)
+                              : nc > 96        ? small_round<2, 1, WAVES>(S, nc, (uint32_t)n, node0, ref0, nodes)
+                              : nc > 32        ? small_round<2, 2, 1>(S, nc, (uint32_t)n, node0, ref0, nodes)
+                                               : small_round<1, 1, 1>(S, nc, (uint32_t)n, node0, ref0, nodes);
         live += nc;
-        for (int i = tid; i < (int)nc; i += SMALL_BLOCK) s_nn[i] = nearest_lds(i, (int)nc, s_lx, s_ly, s_lz, s_hx, s_hy, s_hz);
-        __syncthreads();
-        // each thread takes a run of positions (the list's order is kept by the scans), holds
-        // what it writes in registers, and writes after every read of the round is done
-        const int per = ((int)nc + SMALL_BLOCK - 1) / SMALL_BLOCK;
-        const int s0 = min(tid * per, (int)nc), s1 = min(s0 + per, (int)nc);
-        uint32_t ck = 0, cm = 0;
-        for (int i = s0; i < s1; i++) {
-            const uint32_t j = s_nn[i];
-            const bool mu = j < nc && s_nn[j] == (uint32_t)i;
-            ck += !(mu && (uint32_t)i > j);
-            cm += mu && (uint32_t)i < j;
-        }
-        uint32_t tk, tm;
-        const uint32_t dk0 = block_excl_scan<SMALL_BLOCK / 64>(ck, &tk, s_wsum);
-        uint32_t dm = block_excl_scan<SMALL_BLOCK / 64>(cm, &tm, s_wsum);
-        uint32_t o_id[SMALL_PER], o_h[SMALL_PER];
-        float o_b[SMALL_PER][6];
-        int m = 0;
-#pragma unroll
-        for (int q = 0; q < SMALL_PER; q++) {
-            const int i = s0 + q;
-            if (i >= s1) break;
-            const uint32_t j = s_nn[i];
-            const bool mu = j < nc && s_nn[j] == (uint32_t)i;
-            if (mu && (uint32_t)i > j) continue;
-            float b0 = s_lx[i], b1 = s_ly[i], b2 = s_lz[i], b3 = s_hx[i], b4 = s_hy[i], b5 = s_hz[i];
-            uint32_t id = s_id[i], h = s_h[i];
-            if (mu && (uint32_t)i < j) {
-                const uint32_t k = ((uint32_t)n - 2u) - ((uint32_t)n - nc + dm);
-                dm++;
-                const float4 clo = make_float4(b0, b1, b2, 0.0f), chi = make_float4(b3, b4, b5, 0.0f);
-                const float4 dlo = make_float4(s_lx[j], s_ly[j], s_lz[j], 0.0f), dhi = make_float4(s_hx[j], s_hy[j], s_hz[j], 0.0f);
-                b0 = wmin(clo.x, dlo.x); b1 = wmin(clo.y, dlo.y); b2 = wmin(clo.z, dlo.z);
-                b3 = wmax(chi.x, dhi.x); b4 = wmax(chi.y, dhi.y); b5 = wmax(chi.z, dhi.z);
-                put_final(&nodes[1 + 2 * (size_t)k], id, clo, chi, (uint32_t)n, node0, ref0);
-                put_final(&nodes[2 + 2 * (size_t)k], s_id[j], dlo, dhi, (uint32_t)n, node0, ref0);
-                const uint32_t hd = s_h[j];
-                h = 1 + (h > hd ? h : hd);
-                if (k == 0) put_node(&nodes[0], b0, b1, b2, node0 + 1u, b3, b4, b5, node0 + 2u);
-                id = k;
-            }
-            o_id[m] = id;
-            o_h[m] = h;
-            o_b[m][0] = b0; o_b[m][1] = b1; o_b[m][2] = b2; o_b[m][3] = b3; o_b[m][4] = b4; o_b[m][5] = b5;
-            m++;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < SMALL_PER; q++) {
-            if (q >= m) break;
-            const uint32_t d = dk0 + (uint32_t)q;
-            s_id[d] = o_id[q];
-            s_h[d] = o_h[q];
-            s_lx[d] = o_b[q][0]; s_ly[d] = o_b[q][1]; s_lz[d] = o_b[q][2];
-            s_hx[d] = o_b[q][3]; s_hy[d] = o_b[q][4]; s_hz[d] = o_b[q][5];
-        }
-        __syncthreads();
-        if (tk >= nc) break;   // merged nothing (NaN boxes): ends instead of spinning
-        nc = tk;
+        if (left >= nc) break;   // merged nothing (NaN boxes): ends instead of spinning
+        nc = left;
         rounds++;
     }
     if (tid == 0) {
-        *rounds_out = rounds;
-        *depth_out = nc == 1 ? s_h[0] : height[0];
+        *rounds_out = rounds + max((uint32_t)planned, st->made);
+        *depth_out = nc == 1 ? S.h[0] : height_of(bx[0]);
         st->live += live;
     }
 }
@@ -1070,7 +1240,7 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_ploc_small(int n, uint32_t node
 // ---- the scratch layout of one build --------------------------------------------------------------
 struct Layout {
     size_t params, bounds_tmp, hist, ticket, bucket, keys0, vals0, keys1, vals1, zero, zero_words, status,
-        ctr, depth, other, height, bx, list0, list1, nnbuf, pst, pstatus, pstatus_words, rounds, total;
+        ctr, depth, other, esc_count, bx, list0, list1, nnbuf, pst, pstatus, pstatus_words, rounds, total;
 };
 
 Layout layout(int n)
@@ -1078,7 +1248,7 @@ Layout layout(int n)
     Layout L;
     const size_t N = n > 0 ? (size_t)n : 1;
     const size_t tiles = (N + SORT_TILE - 1) / SORT_TILE;
-    const size_t ptiles = (N + PLOC_TILE - 1) / PLOC_TILE;
+    const size_t ptiles = (N + ploc_tile(2) - 1) / ploc_tile(2);
     size_t o = 0;
     auto take = [&](size_t bytes) { size_t at = o; o += lr_align(bytes); return at; };
     L.params = take(sizeof(LrBuildParamsDev));
@@ -1099,7 +1269,7 @@ Layout layout(int n)
     L.zero_words = (o - L.zero) / 4;
     // PLOC's; an LBVH build's listed nodes (k_lbvh's slots, 16 bytes each) and their counts
     const size_t groups = (N + LBVH_GROUP - 1) / LBVH_GROUP;
-    L.height = take(std::max(8 * N, groups * 4));
+    L.esc_count = take(groups * 4);
     L.bx = take(std::max((2 * N) * 32, groups * LBVH_SLOTS * 16));
     L.list0 = take(N * 4);
     L.list1 = take(N * 4);
@@ -1112,12 +1282,22 @@ Layout layout(int n)
     return L;
 }
 
-// ploc_rounds (trace_gpu.c:563): the rounds from n down to `small`, two more to be safe
+// ploc_rounds (trace_gpu.c:563): the rounds from n down to `small`, two more to be safe: those a
+// build counts even where fewer are made
 int ploc_rounds(int n, int small)
 {
     int r = 0;
     for (int64_t m = n; m > small; m = m * 5 / 6) r++;
-    return r ? r + 2 : 0;
+    return std::min(r ? r + 2 : 0, PLOC_MAX_ROUNDS);
+}
+
+// the rounds launched: a round leaves 0.84 to 0.87 of its clusters, and one left to k_ploc_small above its
+// best size costs it 30 us, where a launch with nothing left to do takes 2 and a round 8
+int ploc_launches(int n, int small)
+{
+    int r = 0;
+    for (double m = n; m > small; m *= 0.87) r++;
+    return std::min(r ? r + 1 : 0, PLOC_MAX_ROUNDS);
 }
 
 }  // namespace
@@ -1188,13 +1368,11 @@ int build_at(LrhContext *c, char *S, const float *boxes, int n, const float *hos
     if (sorted_codes_out) LR_HIP(hipMemcpyAsync(sorted_codes_out, k0, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
     if (sorted_items_out) LR_HIP(hipMemcpyAsync(sorted_items_out, v0, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
     uint32_t *depth = (uint32_t *)at(L.depth);
-    uint32_t *height = (uint32_t *)at(L.height);
-    int rounds = 0;
     const bool ploc = builder == LRH_PLOC && n > 2;
     if (!ploc) {
         const int groups = (n + LBVH_GROUP - 1) / LBVH_GROUP;
         uint4 *esc = (uint4 *)at(L.bx);
-        uint32_t *esc_count = (uint32_t *)at(L.height);
+        uint32_t *esc_count = (uint32_t *)at(L.esc_count);
         hipLaunchKernelGGL(k_lbvh, dim3(groups), dim3(LBVH_GROUP), 0, s, k0, v0, reinterpret_cast<const float4 *>(boxes), n, node0,
                            ref0, ref_add, nd, ax, esc, esc_count, depth);
         LR_HIP(hipGetLastError());
@@ -1215,43 +1393,43 @@ int build_at(LrhContext *c, char *S, const float *boxes, int n, const float *hos
         uint64_t *ps = (uint64_t *)at(L.pstatus);
         const size_t ptiles = L.pstatus_words / 2;
         hipLaunchKernelGGL(k_ploc_init, dim3((n + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, s, v0,
-                           reinterpret_cast<const float4 *>(boxes), n, ref0, ref_add, ax, bx, l0, height, pst, ps,
+                           reinterpret_cast<const float4 *>(boxes), n, ref0, ref_add, ax, bx, l0, pst, ps,
                            L.pstatus_words);
         LR_HIP(hipGetLastError());
         const int small = std::min(c->ploc_small > 0 ? c->ploc_small : 1024, SMALL_MAX);
-        int nr = ploc_rounds(n, small);
-        if (nr > PLOC_MAX_ROUNDS) nr = PLOC_MAX_ROUNDS;
+        const int planned = ploc_rounds(n, small), nr = std::max(planned, ploc_launches(n, small));
+        // the grid from an estimate of the clusters left (a round leaves 0.84 to 0.87 of them; work-groups
+        // without a tile end at once, one with two makes the round twice as long)
         double est = n;
         for (int r = 0; r < nr; r++) {
-            int grid = (int)((est + PLOC_TILE - 1) / PLOC_TILE);
-            if (grid < 16) grid = 16;
-            if (grid > 4096) grid = 4096;
-            hipLaunchKernelGGL(k_ploc_round, dim3(grid), dim3(BLOCK), 0, s, r, n, (uint32_t)small, node0, ref0, bx, l0, l1,
-                               nd, height, pst, ps, ps + ptiles);
+            const bool big = est >= PLOC_BIG;
+            const int tile = big ? ploc_tile(4) : ploc_tile(2);
+            const int grid = std::clamp((int)((est + tile - 1) / tile), 16, 4096);
+            hipLaunchKernelGGL((big ? k_ploc_round<4> : k_ploc_round<2>), dim3(grid), dim3(BLOCK), 0, s, r, n, (uint32_t)small,
+                               node0, ref0, bx, l0, l1, nd, pst, ps, ps + ptiles, (uint32_t)ptiles);
             LR_HIP(hipGetLastError());
-            est *= 0.84;
+            est *= 0.88;
         }
         hipLaunchKernelGGL(k_ploc_small, dim3(1), dim3(SMALL_BLOCK), 0, s, n, node0, ref0, bx, l0, l1,
-                           (uint32_t *)at(L.nnbuf), nd, height, pst, (uint32_t *)at(L.rounds), depth);
+                           (uint32_t *)at(L.nnbuf), nd, pst, planned, (uint32_t *)at(L.rounds), depth);
         LR_HIP(hipGetLastError());
-        rounds = nr;
     }
     if (stats) {
         LR_HIP(hipEventRecord(c->ev[1], s));
         LR_HIP(hipEventSynchronize(c->ev[1]));
         float ms = 0;
         LR_HIP(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
-        uint32_t dep = 0, small_rounds = 0;
+        uint32_t dep = 0, rounds = 0;
         uint64_t live = 0;
         LR_HIP(hipMemcpy(&dep, depth, 4, hipMemcpyDeviceToHost));
         if (ploc) {
-            LR_HIP(hipMemcpy(&small_rounds, at(L.rounds), 4, hipMemcpyDeviceToHost));
+            LR_HIP(hipMemcpy(&rounds, at(L.rounds), 4, hipMemcpyDeviceToHost));
             LR_HIP(hipMemcpy(&live, (const char *)at(L.pst) + offsetof(PlocState, live), 8, hipMemcpyDeviceToHost));
         }
         stats->clusters = live;
         stats->refitted = 0;
         stats->depth = (int)dep;
-        stats->rounds = ploc ? rounds + (int)small_rounds : 0;
+        stats->rounds = (int)rounds;
         stats->ms = ms;
         c->last_build_ms = ms;
     }
