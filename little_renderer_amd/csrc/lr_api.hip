@@ -68,6 +68,7 @@ int lrh_create(LrhContext **out, int device, void *stream)
         c->own_stream = true;
     }
     if (hipEventCreate(&c->ev[0]) != hipSuccess || hipEventCreate(&c->ev[1]) != hipSuccess ||
+        hipHostMalloc((void **)&c->built, sizeof(LrBuildResult), hipHostMallocDefault) != hipSuccess ||
         hipMalloc(&c->flags, 256) != hipSuccess || hipMemsetAsync(c->flags, 0, 256, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess) {
         lrh_destroy(c);
@@ -91,6 +92,7 @@ void lrh_destroy(LrhContext *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (auto &s : c->scratch)
         if (s.base) (void)hipFree(s.base);
+    if (c->built) (void)hipHostFree(c->built);
     if (c->flags) (void)hipFree(c->flags);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);

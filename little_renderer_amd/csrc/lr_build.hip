@@ -60,6 +60,12 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
     return v;
 }
 
+// to the host's memory, seen there once the kernel has ended
+__device__ __forceinline__ void tell_depth(LrBuildResult *res, uint32_t depth)
+{
+    if (res) __hip_atomic_store(&res->depth, depth, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // exclusive scan of one value per thread over a block of NW waves; *total gets the sum
 template <int NW>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *total, uint32_t *s_wsum)
@@ -488,7 +494,7 @@ __global__ __launch_bounds__(LBVH_GROUP) void k_lbvh(const uint32_t *__restrict_
                                                 const float4 *__restrict__ boxes, int n, uint32_t node0, uint32_t ref0,
                                                 uint32_t ref_add, LrNode *__restrict__ nodes, uint32_t *__restrict__ aux,
                                                 uint4 *__restrict__ esc, uint32_t *__restrict__ esc_count,
-                                                uint32_t *depth_out)
+                                                LrBuildResult *res)
 {
     __shared__ int s_d[LBVH_GROUP + 1];        // d(B0 - 1 + i); -1 (below every delta) off the keys' ends
     __shared__ int s_pmin[LBVH_GROUP + 1];     // min of s_d[0 .. i]
@@ -510,7 +516,7 @@ __global__ __launch_bounds__(LBVH_GROUP) void k_lbvh(const uint32_t *__restrict_
         if (n > 1) put_node(&nodes[n - 1 + j], lx, ly, lz, ref0 + (uint32_t)j, hx, hy, hz, 0x80000001u);
         else {
             put_node(&nodes[0], lx, ly, lz, ref0, hx, hy, hz, 0x80000001u);
-            atomicMax(depth_out, 1u);
+            tell_depth(res, 1u);
         }
     }
     if (n == 1) {   // (uniform: the one group returns before any barrier)
@@ -574,7 +580,7 @@ __global__ __launch_bounds__(LBVH_GROUP) void k_lbvh(const uint32_t *__restrict_
         l = L; r = R;
         if (l == 0 && r == n - 1) {
             put_node(&nodes[0], lx, ly, lz, node0 + (uint32_t)lc, hx, hy, hz, node0 + (uint32_t)rc);
-            atomicMax(depth_out, h);
+            tell_depth(res, h);
             break;
         }
         left = s_d[r - B0 + 1] > s_d[l - B0];
@@ -588,7 +594,7 @@ template <bool BUF>
 __global__ __launch_bounds__(BLOCK) void k_lbvh_top(const uint32_t *__restrict__ codes, const uint32_t *__restrict__ items,
                                                       const float4 *__restrict__ boxes, int n, int groups, uint32_t node0,
                                                       LrNode *nodes, unsigned long long *other, const uint4 *__restrict__ esc,
-                                                      const uint32_t *__restrict__ esc_count, uint32_t *depth_out)
+                                                      const uint32_t *__restrict__ esc_count, LrBuildResult *res)
 {
     const int g = blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6);   // one wave per group's list
     if (g >= groups) return;
@@ -653,7 +659,7 @@ __global__ __launch_bounds__(BLOCK) void k_lbvh_top(const uint32_t *__restrict__
             l = L; r = R;
             if (l == 0 && r == n - 1) {
                 put_node(&nodes[0], lx, ly, lz, node0 + (uint32_t)lc, hx, hy, hz, node0 + (uint32_t)rc);
-                atomicMax(depth_out, h);
+                tell_depth(res, h);
                 break;
             }
             left = is_left(codes, n, l, r);
@@ -1135,7 +1141,7 @@ __device__ __forceinline__ uint32_t small_round(SmallLds &S, uint32_t nc, uint32
 
 __global__ __launch_bounds__(SMALL_BLOCK) void k_ploc_small(int n, uint32_t node0, uint32_t ref0, float4 *bx, uint32_t *list0,
                                                               uint32_t *list1, uint32_t *nnbuf, LrNode *nodes,
-                                                              PlocState *st, int planned, uint32_t *rounds_out, uint32_t *depth_out)
+                                                              PlocState *st, int planned, LrBuildResult *res)
 {
     __shared__ SmallLds S;
     uint32_t *const s_wsum = S.wsum;
@@ -1231,16 +1237,19 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_ploc_small(int n, uint32_t node
         rounds++;
     }
     if (tid == 0) {
-        *rounds_out = rounds + max((uint32_t)planned, st->made);
-        *depth_out = nc == 1 ? S.h[0] : height_of(bx[0]);
-        st->live += live;
+        if (res) {
+            __hip_atomic_store(&res->rounds, rounds + max((uint32_t)planned, st->made), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(&res->live, st->live + live, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        tell_depth(res, nc == 1 ? S.h[0] : height_of(bx[0]));
     }
 }
 
 // ---- the scratch layout of one build --------------------------------------------------------------
 struct Layout {
     size_t params, bounds_tmp, hist, ticket, bucket, keys0, vals0, keys1, vals1, zero, zero_words, status,
-        ctr, depth, other, esc_count, bx, list0, list1, nnbuf, pst, pstatus, pstatus_words, rounds, total;
+        ctr, other, esc_count, bx, list0, list1, nnbuf, pst, pstatus, pstatus_words, total;
 };
 
 Layout layout(int n)
@@ -1260,10 +1269,9 @@ Layout layout(int n)
     L.vals0 = take(N * 4);
     L.keys1 = take(N * 4);
     L.vals1 = take(N * 4);
-    // one region the Morton kernel clears: tile counters, depth, look-back states, arrivals
+    // one region the Morton kernel clears: tile counters, look-back states, arrivals
     L.zero = o;
     L.ctr = take(64);
-    L.depth = take(64);
     L.status = take(SORT_PASSES * tiles * 256 * 4);
     L.other = take(N * 8);
     L.zero_words = (o - L.zero) / 4;
@@ -1277,7 +1285,6 @@ Layout layout(int n)
     L.pst = take(sizeof(PlocState));
     L.pstatus_words = 2 * (ptiles + 1);
     L.pstatus = take(L.pstatus_words * 8);
-    L.rounds = take(64);
     L.total = o;
     return L;
 }
@@ -1367,24 +1374,25 @@ int build_at(LrhContext *c, char *S, const float *boxes, int n, const float *hos
     // sorted: k0 (codes), v0 (items)
     if (sorted_codes_out) LR_HIP(hipMemcpyAsync(sorted_codes_out, k0, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
     if (sorted_items_out) LR_HIP(hipMemcpyAsync(sorted_items_out, v0, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
-    uint32_t *depth = (uint32_t *)at(L.depth);
+    LrBuildResult *res = stats ? c->built : nullptr;
+    if (res) *res = LrBuildResult{};
     const bool ploc = builder == LRH_PLOC && n > 2;
     if (!ploc) {
         const int groups = (n + LBVH_GROUP - 1) / LBVH_GROUP;
         uint4 *esc = (uint4 *)at(L.bx);
         uint32_t *esc_count = (uint32_t *)at(L.esc_count);
         hipLaunchKernelGGL(k_lbvh, dim3(groups), dim3(LBVH_GROUP), 0, s, k0, v0, reinterpret_cast<const float4 *>(boxes), n, node0,
-                           ref0, ref_add, nd, ax, esc, esc_count, depth);
+                           ref0, ref_add, nd, ax, esc, esc_count, res);
         LR_HIP(hipGetLastError());
         // the climbs above the groups; the buffer path while the records lie within 2 GiB of
         // the array's base
         const dim3 tgrid((unsigned)((groups + BLOCK / 64 - 1) / (BLOCK / 64)));
         if ((2 * (size_t)n - 1) * 32 < 0x7fffffffu)
             hipLaunchKernelGGL(k_lbvh_top<true>, tgrid, dim3(BLOCK), 0, s, k0, v0, reinterpret_cast<const float4 *>(boxes), n,
-                               groups, node0, nd, (unsigned long long *)at(L.other), esc, esc_count, depth);
+                               groups, node0, nd, (unsigned long long *)at(L.other), esc, esc_count, res);
         else
             hipLaunchKernelGGL(k_lbvh_top<false>, tgrid, dim3(BLOCK), 0, s, k0, v0, reinterpret_cast<const float4 *>(boxes), n,
-                               groups, node0, nd, (unsigned long long *)at(L.other), esc, esc_count, depth);
+                               groups, node0, nd, (unsigned long long *)at(L.other), esc, esc_count, res);
         LR_HIP(hipGetLastError());
     } else {
         float4 *bx = (float4 *)at(L.bx);
@@ -1411,7 +1419,7 @@ int build_at(LrhContext *c, char *S, const float *boxes, int n, const float *hos
             est *= 0.88;
         }
         hipLaunchKernelGGL(k_ploc_small, dim3(1), dim3(SMALL_BLOCK), 0, s, n, node0, ref0, bx, l0, l1,
-                           (uint32_t *)at(L.nnbuf), nd, pst, planned, (uint32_t *)at(L.rounds), depth);
+                           (uint32_t *)at(L.nnbuf), nd, pst, planned, res);
         LR_HIP(hipGetLastError());
     }
     if (stats) {
@@ -1419,17 +1427,10 @@ int build_at(LrhContext *c, char *S, const float *boxes, int n, const float *hos
         LR_HIP(hipEventSynchronize(c->ev[1]));
         float ms = 0;
         LR_HIP(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
-        uint32_t dep = 0, rounds = 0;
-        uint64_t live = 0;
-        LR_HIP(hipMemcpy(&dep, depth, 4, hipMemcpyDeviceToHost));
-        if (ploc) {
-            LR_HIP(hipMemcpy(&rounds, at(L.rounds), 4, hipMemcpyDeviceToHost));
-            LR_HIP(hipMemcpy(&live, (const char *)at(L.pst) + offsetof(PlocState, live), 8, hipMemcpyDeviceToHost));
-        }
-        stats->clusters = live;
+        stats->clusters = res->live;
         stats->refitted = 0;
-        stats->depth = (int)dep;
-        stats->rounds = (int)rounds;
+        stats->depth = (int)res->depth;
+        stats->rounds = (int)res->rounds;
         stats->ms = ms;
         c->last_build_ms = ms;
     }

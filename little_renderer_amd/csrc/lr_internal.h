@@ -23,6 +23,13 @@ struct LrScratch {
 
 enum { LR_SCRATCH_BUILD = 0, LR_SCRATCH_TRACE = 1, LR_SCRATCH_PT = 2, LR_SCRATCH_COUNT = 3 };
 
+// what a build with statistics tells of itself: its kernels write it to the host's (pinned) memory, so
+// the wait for the build is the only one (copies of three words after it took 90 us)
+struct LrBuildResult {
+    uint32_t depth, rounds;   // rounds, live: PLOC
+    uint64_t live;
+};
+
 struct LrhContext {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -32,6 +39,7 @@ struct LrhContext {
     hipEvent_t ev[2] = {nullptr, nullptr};
     int ploc_small = 1024;   // PLOC: the clusters from which the rounds run in one work-group
     float last_build_ms = 0.0f;
+    LrBuildResult *built = nullptr;   // pinned; builds without statistics do not touch it
     LrhEngine *engine = nullptr;  // lrh_pt_render's engine, made on first use
 };
 
