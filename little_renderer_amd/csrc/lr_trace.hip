@@ -7,6 +7,7 @@
 namespace {
 
 constexpr int TBLOCK = 128;
+constexpr int STK = 10;   // a ray's stack entries in LDS (two words each): 10 KB a work-group, 8 waves a SIMD
 
 // COUNT: also sums the node records fetched (the root's, an inner node's two children's, a
 // popped node's) and the triangles tested, into counts[0], counts[1] (the algorithmic traffic)
@@ -16,15 +17,15 @@ __global__ __launch_bounds__(TBLOCK) void k_trace(const float4 *__restrict__ nod
                                                     const uint32_t *count, float4 *__restrict__ hits, uint32_t *spill,
                                                     int spill_per, uint32_t *overflow, unsigned long long *counts)
 {
-    __shared__ uint32_t stk[LR_LDS_STACK][TBLOCK];
+    __shared__ uint32_t stk[2 * STK][TBLOCK];
     const int tid = threadIdx.x;
     const int i = blockIdx.x * TBLOCK + tid;
     const int live = count ? min(n, (int)*count) : n;   // a queue's count, on the device
     if (i >= live) return;
     const float4 r0 = rays[2 * (size_t)i], r1 = rays[2 * (size_t)i + 1];
-    const WalkStack S{&stk[0][tid], TBLOCK, spill + i, (size_t)n, LR_LDS_STACK + spill_per};
+    const WalkStack S{&stk[0][tid], TBLOCK, spill + i, (size_t)n, STK + spill_per};
     uint32_t cn = 0, ct = 0;
-    const WalkHit h = walk<ANY, false, COUNT>(nodes, root, aux, tris, nullptr, 0, v3of(r0), v3of(r1), r0.w, r1.w, S,
+    const WalkHit h = walk<ANY, false, COUNT, STK>(nodes, root, aux, tris, nullptr, 0, v3of(r0), v3of(r1), r0.w, r1.w, S,
                                               overflow, cn, ct);
     hits[i] = make_float4(h.t, __uint_as_float(h.id), h.b1, h.b2);
     if (COUNT) {
@@ -45,7 +46,7 @@ void launch(LrhContext *c, const uint32_t *nodes, uint32_t root, const uint32_t 
 
 }  // namespace
 
-int lr_spill_per(int max_depth) { return max_depth + 2 > LR_LDS_STACK ? max_depth + 2 - LR_LDS_STACK : 0; }
+int lr_spill_per(int max_depth) { return max_depth + 2 > STK ? max_depth + 2 - STK : 0; }
 
 int lr_launch_trace(LrhContext *c, const uint32_t *nodes, uint32_t root, const uint32_t *aux, const float *tris,
                     const float *rays, int nrays, const uint32_t *count, int any, float *hits, int max_depth,

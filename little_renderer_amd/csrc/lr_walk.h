@@ -9,7 +9,8 @@
 // entries of each ray live in LDS (interleaved by lane: no bank conflicts) and deeper ones
 // spill to device memory, sized from the tree's depth, so nothing is ever dropped. Sixteen
 // LDS entries (8 KB for a work-group of 128) leave the walk kernels at their register-bound
-// occupancy; the binary walk pushes only the farther child, so deep entries are rare.
+// occupancy; the binary walk pushes only the farther child (two words of it, for 10 entries), so deep
+// entries are rare.
 #pragma once
 
 #include "lr_device.h"
@@ -42,6 +43,32 @@ __device__ __forceinline__ float box_t(float4 lo, float4 hi, V3 o, V3 inv, float
     const float enter = wmax(wmax(wmin(t0x, t1x), wmin(t0y, t1y)), wmax(wmin(t0z, t1z), tmin));
     const float leave = wmin(wmin(wmax(t0x, t1x), wmax(t0y, t1y)), wmin(wmax(t0z, t1z), tmax));
     return leave < enter ? -1.0f : enter;
+}
+
+// box_t of two boxes for the binary walk, by minima and maxima that pass a NaN on (one instruction
+// each, three operands, where wmin and wmax are a compare and a select): the same answers unless a NaN
+// is in one of them, which shows in its entry or exit, and then box_t's own
+__device__ __forceinline__ float nmin(float a, float b) { return __builtin_elementwise_minimum(a, b); }
+__device__ __forceinline__ float nmax(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ void slab_(float4 lo, float4 hi, V3 o, V3 inv, float tmin, float tmax, float &enter, float &leave)
+{
+    const float t0x = (lo.x - o.x) * inv.x, t0y = (lo.y - o.y) * inv.y, t0z = (lo.z - o.z) * inv.z;
+    const float t1x = (hi.x - o.x) * inv.x, t1y = (hi.y - o.y) * inv.y, t1z = (hi.z - o.z) * inv.z;
+    enter = nmax(nmax(nmax(nmin(t0x, t1x), nmin(t0y, t1y)), nmin(t0z, t1z)), tmin);
+    leave = nmin(nmin(nmin(nmax(t0x, t1x), nmax(t0y, t1y)), nmax(t0z, t1z)), tmax);
+}
+__device__ __forceinline__ void box_t2(float4 alo, float4 ahi, float4 blo, float4 bhi, V3 o, V3 inv, float tmin, float tmax,
+                                       float &ta, float &tb)
+{
+    float ea, la, eb, lb;
+    slab_(alo, ahi, o, inv, tmin, tmax, ea, la);
+    slab_(blo, bhi, o, inv, tmin, tmax, eb, lb);
+    ta = la < ea ? -1.0f : ea;
+    tb = lb < eb ? -1.0f : eb;
+    if (__builtin_isunordered(ea, la) || __builtin_isunordered(eb, lb)) {
+        ta = box_t(alo, ahi, o, inv, tmin, tmax);
+        tb = box_t(blo, bhi, o, inv, tmin, tmax);
+    }
 }
 
 // hit_tri (trace.wgsl:159-173): t in (tmin, tmax) and the barycentrics
@@ -175,12 +202,16 @@ __device__ __forceinline__ uint32_t stk_get(const WalkStack &S, int sp)
 // The nodes are visited in the reference's order (pop a node; test its two children's boxes;
 // push the farther hit child, then the nearer, and pop again), but the nearer child is not
 // pushed and popped: it stays in registers as the next entry, with its two child fields
-// (lo.w, hi.w), which its parent's box test has already loaded. Only a popped (farther) child
-// fetches those two words of its record; the reference fetches the whole record of every node
-// it pops. Same visits, same tests, same hits: one dependent load fewer on each step down.
-// COUNT adds the node records fetched (the root's, each inner node's two children, each
-// popped node's) and the shapes tested to cn, ct.
-template <bool ANY, bool PRIMS, bool COUNT, int STK = LR_LDS_STACK>
+// (lo.w, hi.w), which its parent's box test has already loaded. A farther child's two words go to
+// the stack in its place, while they fit in LDS (S.stk holds 2 STK words a ray); past it its index
+// does, and the pop fetches them. The reference fetches the whole record of every node it pops. Same
+// visits, same tests, same hits. Bound by the loads' data path (a wave's lanes are at different
+// nodes, so a load takes 16 cycles or more whatever its width): without the pop's two loads, and with
+// box_t2, 1920 x 1080 camera rays through 1M triangles took 2.33 ms, before 2.56 (box_t2 alone 2.49;
+// with 14 stack entries in LDS instead of 10, and fewer waves, 2.75).
+// COUNT adds the node records the reference's walk fetches past the first test of them (the root's,
+// each inner node's two children, each popped node's) and the shapes tested to cn, ct.
+template <bool ANY, bool PRIMS, bool COUNT, int STK>
 __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32_t root, const uint32_t *__restrict__ aux,
                                         const float4 *__restrict__ tris, const float4 *__restrict__ prims, uint32_t nprims,
                                         V3 o, V3 d, float tmin, float tmax, const WalkStack &S, uint32_t *overflow,
@@ -194,6 +225,18 @@ __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32
     uint32_t na = __float_as_uint(words[8 * (size_t)root + 3]), nb = __float_as_uint(words[8 * (size_t)root + 7]);
     if (COUNT) cn++;
     int sp = 0;
+    auto pop = [&] {
+        sp--;
+        if (sp < STK) {
+            na = S.stk[2 * sp * S.stride];
+            nb = S.stk[(2 * sp + 1) * S.stride];
+        } else {
+            const uint32_t ni = S.spill[(size_t)(sp - STK) * S.sstride];
+            na = __float_as_uint(words[8 * (size_t)ni + 3]);
+            nb = __float_as_uint(words[8 * (size_t)ni + 7]);
+        }
+        if (COUNT) cn++;
+    };
     for (;;) {
         while (nb & LR_LEAF) {
             const uint32_t cnt = nb & 0x7fffffffu;
@@ -219,16 +262,12 @@ __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32
                 }
             }
             if (sp == 0) return best;
-            sp--;
-            const uint32_t ni = stk_get<STK>(S, sp);
-            na = __float_as_uint(words[8 * (size_t)ni + 3]);
-            nb = __float_as_uint(words[8 * (size_t)ni + 7]);
-            if (COUNT) cn++;
+            pop();
         }
         const float4 alo = nodes[2 * (size_t)na], ahi = nodes[2 * (size_t)na + 1];
         const float4 blo = nodes[2 * (size_t)nb], bhi = nodes[2 * (size_t)nb + 1];
-        const float tl = box_t(alo, ahi, o, inv, tmin, best.t);
-        const float tr = box_t(blo, bhi, o, inv, tmin, best.t);
+        float tl, tr;
+        box_t2(alo, ahi, blo, bhi, o, inv, tmin, best.t, tl, tr);
         if (COUNT) cn += 2;
         if (tl >= 0.0f && tr >= 0.0f) {
             if (sp + 1 > S.cap) {   // cannot happen with a correct depth: said, never silently dropped
@@ -236,9 +275,10 @@ __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32
                 break;
             }
             const bool left_first = tl <= tr;
-            const uint32_t far = left_first ? nb : na;
-            if (sp < STK) S.stk[sp * S.stride] = far;
-            else S.spill[(size_t)(sp - STK) * S.sstride] = far;
+            if (sp < STK) {
+                S.stk[2 * sp * S.stride] = __float_as_uint(left_first ? blo.w : alo.w);
+                S.stk[(2 * sp + 1) * S.stride] = __float_as_uint(left_first ? bhi.w : ahi.w);
+            } else S.spill[(size_t)(sp - STK) * S.sstride] = left_first ? nb : na;
             sp++;
             na = __float_as_uint(left_first ? alo.w : blo.w);
             nb = __float_as_uint(left_first ? ahi.w : bhi.w);
@@ -250,11 +290,7 @@ __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32
             nb = __float_as_uint(bhi.w);
         } else {
             if (sp == 0) break;
-            sp--;
-            const uint32_t ni = stk_get<STK>(S, sp);
-            na = __float_as_uint(words[8 * (size_t)ni + 3]);
-            nb = __float_as_uint(words[8 * (size_t)ni + 7]);
-            if (COUNT) cn++;
+            pop();
         }
     }
     return best;
