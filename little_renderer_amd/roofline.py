@@ -30,7 +30,8 @@ passes before it priced as for the LBVH (bounds 32, morton 40, sort 64 per primi
   rounds    per live cluster of each round: its list entry 4 and box 32 read, the next list's
             entry 4 written, 40 (live: the clusters summed over the rounds, the build's count)
   merges    n - 1 of them: the merged box 32, the two children's records 64 written, their
-            heights 8 read and the merged one 4 written, 108
+            heights 8 read and the merged one 4 written, 108 (the heights are priced as words of
+            their own; they travel in the boxes' spare words)
 """
 
 HBM_PEAK_GBS = 8000.0           # MI355X HBM3E
