@@ -2,9 +2,10 @@
 // scene, camera, image and sample range) share one pool of path slots that the wavefront
 // kernels keep full.
 //
-// One iteration is four kernels: regen (start new paths at the end of the ray queue), extend
-// (closest hits of the ray queue), shade (emission, next-event shadow ray, BSDF sample, Russian
-// roulette), shadow (any hit before the lamp). A path's state lives beside its ray, at its
+// One iteration is three kernels: regen (start new paths at the end of the ray queue), the walks
+// (extend: closest hits of the ray queue; shadow: any hit before the lamp, of the shadow rays that the
+// last iteration's shade made; a kernel each where they are counted or timed apart), shade (emission,
+// next-event shadow ray, BSDF sample, Russian roulette). A path's state lives beside its ray, at its
 // position in the ray queue (two queues, one per iteration parity): shade reads entry i's state
 // and writes a surviving path's state where its next ray is appended, so every state access is
 // coalesced. A path that ends frees one place of the pool; regen fills free places from the
