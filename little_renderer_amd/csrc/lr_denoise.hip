@@ -77,7 +77,7 @@ __device__ __forceinline__ V3 oct_dir(uint32_t u)
 }
 
 // a pixel's record: its packed irradiance and variance, its packed normal, its distance (a surface
-// >= 0; a lamp or the sky -2e38)
+// >= 0; a lamp or the sky -2e38; one that is not >= 0, a NaN among them, passes as a lamp does)
 __device__ __forceinline__ uint4 put_px(V3 c, float v, uint32_t n, uint32_t z)
 {
     const uint2 p = put_iv(c, v);
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(TILE *TILE) void k_dn_atrous(const uint4 *__restric
     const uint4 ck = src[k];
     const float4 c = get_iv(make_uint2(ck.x, ck.y));
     const float zp = __uint_as_float(ck.w);
-    if (c.w < 0.0f || zp < 0.0f) {   // no sample yet; a lamp, the sky: as they are
+    if (c.w < 0.0f || !(zp >= 0.0f)) {   // no sample yet; a lamp, the sky, a distance that is none (NaN): as they are
         if (last) out[k] = c.w < 0.0f ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : make_float4(c.x, c.y, c.z, 1.0f);
         else dst[k] = ck;
         return;
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(TILE *TILE) void k_dn_atrous(const uint4 *__restric
             if (i != 2 || j != 2) {
                 const float zq = __uint_as_float(sq.w);
                 if (q != k) {   // (a jittered tap may land on the pixel itself)
-                    if (s.w < 0.0f || zq < 0.0f) continue;
+                    if (s.w < 0.0f || !(zq >= 0.0f)) continue;
                     // the noisier pixel's noise: a bright outlier spreads to its neighbours as much as
                     // they take from it (the centre's alone would darken the image)
                     const float a = fabsf(lp - lum(v3(s.x, s.y, s.z))) *

@@ -11,7 +11,9 @@
 - lrh_engine_denoise equals lrh_denoise on the job's image, moments and guide; a denoised job's
   image, guide and moments are the same batched and plain.
 - At sizes off the 16 x 16 tiles, on images with lamps, sky, pixels without samples and normals all
-  round the octahedron, each number of passes equals the oracle's to its halves' steps.
+  round the octahedron, each number of passes equals the oracle's to its halves' steps; also where
+  distances are NaN, negative or -0: one that is not >= 0 passes as it is and its neighbours leave it
+  out.
 - It denoises: at 4 spp the filtered Cornell box is far closer to the converged image than the
   samples alone are, below the ceiling. (On the ceiling it is not: a pixel whose centre sees the
   ceiling and whose area is partly the lamp, hung just under the ceiling at nearly its depth and
@@ -117,8 +119,8 @@ def test_engine_denoise_is_lrh_denoise_and_batched_equals_plain(ctx):
     ps.close()
 
 
-@pytest.mark.parametrize("W,H,passes", [(1, 1, 5), (5, 3, 4), (16, 16, 1), (17, 15, 2), (33, 31, 3), (70, 49, 5)])
-def test_filter_matches_the_oracle_on_odd_sizes(ctx, W, H, passes):
+def picture(W, H):
+    """sums, moments and guide of a W x H picture of facets, lamps, sky and pixels without samples"""
     rng = np.random.default_rng(1000 * W + H)
     n = rng.integers(0, 7, (H, W))
     n[0, 0] = 4
@@ -138,16 +140,47 @@ def test_filter_matches_the_oracle_on_odd_sizes(ctx, W, H, passes):
     g[..., 7] = kind
     lum = (a[..., :3] / np.maximum(a[..., 3:], 1)) @ [0.2126, 0.7152, 0.0722]
     m = np.stack([lum * n, (lum ** 2 * 1.2) * n], -1).astype(np.float32)
+    return a, m, g
+
+
+def filtered(ctx, a, m, g, passes):
+    H, W = a.shape[:2]
     t = [torch.from_numpy(v).cuda() for v in (a, m, g)]
     out = dev((H, W, 4))
     ctx.denoise(*t, W, H, out, passes=passes)
     ctx.sync()
-    den, ref = out.cpu().numpy(), lro.denoise(a, m, g, passes=passes)
+    return out.cpu().numpy(), lro.denoise(a, m, g, passes=passes)
+
+
+@pytest.mark.parametrize("W,H,passes", [(1, 1, 5), (5, 3, 4), (16, 16, 1), (17, 15, 2), (33, 31, 3), (70, 49, 5)])
+def test_filter_matches_the_oracle_on_odd_sizes(ctx, W, H, passes):
+    den, ref = filtered(ctx, *picture(W, H), passes)
     assert np.array_equal(den[..., 3], ref[..., 3])
     rel = np.abs(den[..., :3] - ref[..., :3]) / np.maximum(np.abs(ref[..., :3]), 1e-3)
     say(f"  {W}x{H}, {passes} passes: median rel {np.median(rel):.2e}, max {rel.max():.2e}")
     # a last-bit difference may move a packed half by one step (2^-11), once a pass and again through
     # the weights that the moved half is in; most pixels meet none
+    assert np.median(rel) < 1e-5 and rel.max() < 2 * passes * 2.0 ** -11
+
+
+@pytest.mark.parametrize("passes", [1, 2, 5])
+@pytest.mark.parametrize("z", [np.nan, -1.0, -0.0, -np.inf])
+def test_odd_distances_match_the_oracle(ctx, z, passes):
+    a, m, g = picture(70, 49)
+    rng = np.random.default_rng(5)
+    odd = rng.random(g.shape[:2]) < 0.02
+    odd[:3, :3] = [[True, False, False], [False, False, True], [False, True, True]]
+    g[odd, 3] = z
+    a[odd, 3] = np.maximum(a[odd, 3], 1)
+    with np.errstate(all="ignore"):
+        den, ref = filtered(ctx, a, m, g, passes)
+        d, r = den[..., :3], ref[..., :3]
+        rel = np.abs(d - r) / np.maximum(np.abs(r), 1e-3)
+    say(f"  z {z}, {passes} passes: {odd.sum()} odd pixels, {np.isnan(r).any(-1).sum()} NaN in the oracle's image")
+    assert np.array_equal(den[..., 3], ref[..., 3])
+    assert np.array_equal(np.isnan(d), np.isnan(r))
+    assert not np.isnan(r).any()
+    # (the bound of the odd sizes' test)
     assert np.median(rel) < 1e-5 and rel.max() < 2 * passes * 2.0 ** -11
 
 
