@@ -211,8 +211,9 @@ __global__ __launch_bounds__(TILE *TILE) void k_dn_atrous(const uint4 *__restric
                     float wn = rfmax(vdot(np, nq) * __builtin_amdgcn_rsqf(vdot(nq, nq)), 0.0f);
                     for (int e = 0; e < 7; e++) wn *= wn;
                     const float expect = gx * fabsf((float)ox) + gy * fabsf((float)oy);
-                    const float b = fabsf(zp - zq) * __builtin_amdgcn_rcpf(expect + z0);
-                    w *= wn * __builtin_amdgcn_exp2f(-1.44269504f * (a + b));
+                    // (in units of 2^24: the reciprocal of a number past 2^126 would be 0)
+                    const float b = fabsf(zp - zq) * __builtin_amdgcn_rcpf(0x1p-24f * (expect + z0));
+                    w *= wn * __builtin_amdgcn_exp2f(-1.44269504f * __builtin_fmaf(0x1p-24f, b, a));
                 }
             }
             sum = vadd(sum, vscale(v3(s.x, s.y, s.z), w));
