@@ -105,7 +105,9 @@ int lrh_build_noalloc(LrhContext *c, const float *d_boxes, int n, const float *h
  * tree of triangles in the reference GPU layout: the walk of trace.wgsl traverse
  * (:270-392) for a scene of triangles. The shape id of a hit is the aux entry of its leaf.
  * Unlike the reference, the walk never drops a push: max_depth (the tree's depth, as
- * lrh_build reports it) sizes its stack, which spills from LDS to device memory. */
+ * lrh_build reports it) sizes its stack, which spills from LDS to device memory: max_depth - 8
+ * words a ray of the context's scratch memory from a depth of 15 on, none up to 14. 16 entries are
+ * there whatever max_depth says; a walk that needs more than it says is refused at lrh_sync. */
 int lrh_trace(LrhContext *c, const uint32_t *d_nodes, uint32_t root, const uint32_t *d_aux,
               const float *d_tris, const float *d_rays, int n, int any, float *d_hits, int max_depth);
 

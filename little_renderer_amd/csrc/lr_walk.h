@@ -9,8 +9,8 @@
 // entries of each ray live in LDS (interleaved by lane: no bank conflicts) and deeper ones
 // spill to device memory, sized from the tree's depth, so nothing is ever dropped. Sixteen
 // LDS entries (8 KB for a work-group of 128) leave the walk kernels at their register-bound
-// occupancy; the binary walk pushes only the farther child (two words of it, for 10 entries), so deep
-// entries are rare.
+// occupancy; the binary walk pushes only the farther child, so deep entries are rare (its entries in
+// LDS: lr_trace.hip).
 #pragma once
 
 #include "lr_device.h"
@@ -203,15 +203,15 @@ __device__ __forceinline__ uint32_t stk_get(const WalkStack &S, int sp)
 // push the farther hit child, then the nearer, and pop again), but the nearer child is not
 // pushed and popped: it stays in registers as the next entry, with its two child fields
 // (lo.w, hi.w), which its parent's box test has already loaded. A farther child's two words go to
-// the stack in its place, while they fit in LDS (S.stk holds 2 STK words a ray); past it its index
-// does, and the pop fetches them. The reference fetches the whole record of every node it pops. Same
+// the stack in its place in the first PAIRS entries (S.stk: PAIRS + STK words a ray, for STK entries);
+// past them its index does, and the pop fetches them. The reference fetches the whole record of every node it pops. Same
 // visits, same tests, same hits. Bound by the loads' data path (a wave's lanes are at different
 // nodes, so a load takes 16 cycles or more whatever its width): without the pop's two loads, and with
 // box_t2, 1920 x 1080 camera rays through 1M triangles took 2.33 ms, before 2.56 (box_t2 alone 2.49;
 // with 14 stack entries in LDS instead of 10, and fewer waves, 2.75).
 // COUNT adds the node records the reference's walk fetches past the first test of them (the root's,
 // each inner node's two children, each popped node's) and the shapes tested to cn, ct.
-template <bool ANY, bool PRIMS, bool COUNT, int STK>
+template <bool ANY, bool PRIMS, bool COUNT, int PAIRS, int STK>
 __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32_t root, const uint32_t *__restrict__ aux,
                                         const float4 *__restrict__ tris, const float4 *__restrict__ prims, uint32_t nprims,
                                         V3 o, V3 d, float tmin, float tmax, const WalkStack &S, uint32_t *overflow,
@@ -227,11 +227,11 @@ __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32
     int sp = 0;
     auto pop = [&] {
         sp--;
-        if (sp < STK) {
+        if (sp < PAIRS) {
             na = S.stk[2 * sp * S.stride];
             nb = S.stk[(2 * sp + 1) * S.stride];
         } else {
-            const uint32_t ni = S.spill[(size_t)(sp - STK) * S.sstride];
+            const uint32_t ni = sp < STK ? S.stk[(PAIRS + sp) * S.stride] : S.spill[(size_t)(sp - STK) * S.sstride];
             na = __float_as_uint(words[8 * (size_t)ni + 3]);
             nb = __float_as_uint(words[8 * (size_t)ni + 7]);
         }
@@ -275,10 +275,11 @@ __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32
                 break;
             }
             const bool left_first = tl <= tr;
-            if (sp < STK) {
+            if (sp < PAIRS) {
                 S.stk[2 * sp * S.stride] = __float_as_uint(left_first ? blo.w : alo.w);
                 S.stk[(2 * sp + 1) * S.stride] = __float_as_uint(left_first ? bhi.w : ahi.w);
-            } else S.spill[(size_t)(sp - STK) * S.sstride] = left_first ? nb : na;
+            } else if (sp < STK) S.stk[(PAIRS + sp) * S.stride] = left_first ? nb : na;
+            else S.spill[(size_t)(sp - STK) * S.sstride] = left_first ? nb : na;
             sp++;
             na = __float_as_uint(left_first ? alo.w : blo.w);
             nb = __float_as_uint(left_first ? ahi.w : bhi.w);

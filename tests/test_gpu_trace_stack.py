@@ -2,7 +2,8 @@
 bit-exact against the oracle's walk of the same tree.
 
 A tree of one long arm (its far children wait one above the other, 10 to a ray in LDS, the rest in
-device memory), and a built tree some of whose boxes and rays hold NaNs, infinities and zeros.
+device memory; 16, and none, where that is enough), also with a depth too small given: 16 entries
+are always there. And a built tree some of whose boxes and rays hold NaNs, infinities and zeros.
 """
 import numpy as np
 import pytest
@@ -33,10 +34,7 @@ def both(ctx, nodes, aux, tris, rays, depth, any_hit):
     return hits.cpu().numpy().view(np.uint32), want.view(np.uint32)
 
 
-@pytest.mark.parametrize("any_hit", [False, True])
-@pytest.mark.parametrize("arm", [2, 9, 10, 11, 12, 30])
-def test_far_children_past_lds(ctx, arm, any_hit):
-    print(f"arm {arm} any {any_hit}", flush=True)
+def arm_tree(arm, nrays):
     # node 2k+1: leaf k, far along z; node 2k+2: the arm's next, nearer; triangle k at z = 100 - k
     tris = np.zeros((arm + 1, 12), np.float32)
     for k in range(arm + 1):
@@ -53,12 +51,60 @@ def test_far_children_past_lds(ctx, arm, any_hit):
     f[2 * arm, 0:3], f[2 * arm, 4:7] = (-1, -1, 1), (4, 4, 100 - arm)
     nodes[2 * arm, 3], nodes[2 * arm, 7] = arm, 0x80000001
     rng = np.random.default_rng(arm)
-    rays = np.zeros((1000, 8), np.float32)
-    rays[:, 0:2], rays[:, 2] = rng.uniform(-1.2, 1.2, (1000, 2)), rng.uniform(-5, 90, 1000)
+    rays = np.zeros((nrays, 8), np.float32)
+    rays[:, 0:2], rays[:, 2] = rng.uniform(-1.2, 1.2, (nrays, 2)), rng.uniform(-5, 90, nrays)
     rays[:, 3], rays[:, 6], rays[:, 7] = 1e-4, 1.0, 1e30
+    return nodes, aux, tris, rays
+
+
+@pytest.mark.parametrize("any_hit", [False, True])
+@pytest.mark.parametrize("arm", [2, 3, 4, 5, 9, 10, 11, 12, 13, 14, 15, 16, 30])
+def test_far_children_past_lds(ctx, arm, any_hit):
+    print(f"arm {arm} any {any_hit}", flush=True)
+    nodes, aux, tris, rays = arm_tree(arm, 1000)
     got, want = both(ctx, nodes, aux, tris, rays, arm + 1, any_hit)
     assert (want[:, 1] != 0xFFFFFFFF).sum() > 500
     assert np.array_equal(got, want), f"{(got != want).any(1).sum()} rays differ"
+
+
+@pytest.mark.parametrize("depth", [1, 9, 14])
+@pytest.mark.parametrize("arm", [10, 11, 16])
+def test_sixteen_entries_whatever_the_depth(ctx, arm, depth):
+    print(f"arm {arm} depth {depth}", flush=True)
+    nodes, aux, tris, rays = arm_tree(arm, 1000)
+    got, want = both(ctx, nodes, aux, tris, rays, depth, False)
+    assert np.array_equal(got, want), f"{(got != want).any(1).sum()} rays differ"
+
+
+def test_too_small_a_depth_is_refused(ctx):
+    nodes, aux, tris, rays = arm_tree(30, 1000)
+    with pytest.raises(lr.LrhError):
+        both(ctx, nodes, aux, tris, rays, 20, False)
+    got, want = both(ctx, nodes, aux, tris, rays, 31, False)   # (and the context goes on)
+    assert np.array_equal(got, want)
+
+
+def test_shallow_walk_allocates_nothing_under_capture():
+    # a first small batch, then a large one captured: no scratch memory of its size, so it may be
+    s = torch.cuda.Stream()
+    c = lr.Context(0, s.cuda_stream)
+    nodes, aux, tris, rays = arm_tree(13, 100_000)
+    d = [torch.from_numpy(a).cuda() for a in (nodes.view(np.int32), aux.view(np.int32), tris, rays)]
+    hits = torch.zeros((len(rays), 4), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    c.trace(d[0], 0, d[1], d[2], d[3], 100, hits, 14)
+    c.sync()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        c.trace(d[0], 0, d[1], d[2], d[3], len(rays), hits, 14)
+    want = lro.trace_gpu_layout(nodes, 0, aux, tris, rays).view(np.uint32)
+    for _ in range(3):
+        hits.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(hits.cpu().numpy().view(np.uint32), want)
+    c.close()
 
 
 @pytest.mark.parametrize("any_hit", [False, True])
