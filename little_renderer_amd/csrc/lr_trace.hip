@@ -17,7 +17,7 @@ constexpr int DEEP_PAIRS = 10, SHALLOW_PAIRS = 4, SHALLOW = 16;
 constexpr int lds_entries(int pairs) { return pairs == SHALLOW_PAIRS ? SHALLOW : DEEP_PAIRS; }
 
 // COUNT: also sums the node records fetched (the root's, an inner node's two children's, a
-// popped node's) and the triangles tested, into counts[0], counts[1] (the algorithmic traffic)
+// popped node's where its entry was an index) and the triangles tested, into counts[0], counts[1] (the algorithmic traffic)
 template <bool ANY, bool COUNT, int PAIRS>
 __global__ __launch_bounds__(TBLOCK) void k_trace(const float4 *__restrict__ nodes, uint32_t root, const uint32_t *__restrict__ aux,
                                                     const float4 *__restrict__ tris, const float4 *__restrict__ rays, int n,

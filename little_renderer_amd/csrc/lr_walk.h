@@ -209,8 +209,8 @@ __device__ __forceinline__ uint32_t stk_get(const WalkStack &S, int sp)
 // nodes, so a load takes 16 cycles or more whatever its width): without the pop's two loads, and with
 // box_t2, 1920 x 1080 camera rays through 1M triangles took 2.33 ms, before 2.56 (box_t2 alone 2.49;
 // with 14 stack entries in LDS instead of 10, and fewer waves, 2.75).
-// COUNT adds the node records the reference's walk fetches past the first test of them (the root's,
-// each inner node's two children, each popped node's) and the shapes tested to cn, ct.
+// COUNT adds the node records fetched (the root's, each inner node's two children, each popped node's
+// past the PAIRS entries) and the shapes tested to cn, ct.
 template <bool ANY, bool PRIMS, bool COUNT, int PAIRS, int STK>
 __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32_t root, const uint32_t *__restrict__ aux,
                                         const float4 *__restrict__ tris, const float4 *__restrict__ prims, uint32_t nprims,
@@ -234,8 +234,8 @@ __device__ __forceinline__ WalkHit walk(const float4 *__restrict__ nodes, uint32
             const uint32_t ni = sp < STK ? S.stk[(PAIRS + sp) * S.stride] : S.spill[(size_t)(sp - STK) * S.sstride];
             na = __float_as_uint(words[8 * (size_t)ni + 3]);
             nb = __float_as_uint(words[8 * (size_t)ni + 7]);
+            if (COUNT) cn++;
         }
-        if (COUNT) cn++;
     };
     for (;;) {
         while (nb & LR_LEAF) {

@@ -3,7 +3,8 @@ between the compute units and memory, whatever the caches do. A kernel's rooflin
 bytes over its measured time, against the HBM peak.
 
 Walks (k_trace, k_extend, k_shadow, k_scene_trace): per ray its 32-byte ray read and its 16-byte
-hit written, per node record fetched its size (32 bytes for the reference's binary node), per shape
+hit written, per node record fetched its size (32 bytes for the reference's binary node; a node popped
+with its child words from the walk's stack is not fetched again and not counted), per shape
 tested its 48-byte triangle and 4-byte aux entry; the engine's 4-wide walks read one 48-byte slot
 for either (SLOT_BYTES). The node and shape counts are the walks' own counters on the same tree
 and rays.

@@ -76,6 +76,21 @@ def test_sixteen_entries_whatever_the_depth(ctx, arm, depth):
     assert np.array_equal(got, want), f"{(got != want).any(1).sum()} rays differ"
 
 
+@pytest.mark.parametrize("arm", [3, 4, 5, 13, 14, 30])
+def test_counts_of_what_is_fetched(ctx, arm):
+    # a ray from below takes the whole arm: every far child waits and is popped
+    nodes, aux, tris, rays = arm_tree(arm, 700)
+    rays[:, 0:3] = (-0.5, -0.5, -5)
+    d = [torch.from_numpy(a).cuda() for a in (nodes.view(np.int32), aux.view(np.int32), tris, rays)]
+    hits = torch.zeros((len(rays), 4), dtype=torch.float32, device="cuda")
+    counts = torch.zeros(2, dtype=torch.int64, device="cuda")
+    torch.cuda.synchronize()
+    ctx.trace_count(d[0], 0, d[1], d[2], d[3], len(rays), None, hits, arm + 1, counts)
+    ctx.sync()
+    held = 4 if arm + 1 <= 14 else 10    # entries that hold a child's words
+    assert counts.tolist() == [700 * (1 + 2 * arm + max(0, arm - held)), 700 * (arm + 1)]
+
+
 def test_too_small_a_depth_is_refused(ctx):
     nodes, aux, tris, rays = arm_tree(30, 1000)
     with pytest.raises(lr.LrhError):
