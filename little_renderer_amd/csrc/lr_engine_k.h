@@ -393,9 +393,9 @@ __device__ WalkHit walk4_tl(const JobDev &J, V3 o, V3 d, float tmin, float tmax,
             }
         } else {
             if (COUNT) count_node(c);
-            uint32_t key[4];
-            wide_keys(r0, r1, r2, ro, inv, tmin, best.t, key);
-            more = wide_next<STK>(key, __float_as_uint(r1.w), S, sp, cur, overflow);
+            float t[4];
+            wide_test(r0, r1, r2, ro, inv, tmin, best.t, t);
+            more = wide_next<STK>(t, __float_as_uint(r1.w), S, sp, cur, overflow);
         }
         if (!more) {
             if (sp == 0) break;

@@ -342,23 +342,24 @@ __device__ __forceinline__ void count_shape(WalkCnt &c)
 // lanes load their nodes and leaves with the same three instructions and a child needs no reference
 // of its own: nodes were 64 bytes with four references (a fourth load and four words to carry
 // through the sort), a leaf's triangle and id two arrays more, the triangle's load waiting for the id.
-// The walks are bound by their VALU instructions (a wave's lanes diverge) and the texture path: keys
-// of one word each, sorted by minima and maxima, and three loads a step took the extension walk of a
-// 54M-path queue from 32.3 to 26.1 ms, its shadow walk from 22.6 to 18.1 ms, and 300,000 rays with
-// nothing in common through 50,000 triangles from 273 to 160 us; the hits are the same.
+// The walks are bound by their VALU instructions (a wave's lanes diverge) and the texture path: three
+// loads a step and a place instead of a reference to carry took the extension walk of a 54M-path queue
+// from 32.3 to 26.1 ms, its shadow walk from 22.6 to 18.1 ms, and 300,000 rays with nothing in common
+// through 50,000 triangles from 273 to 160 us, with the children's distance and place sorted as one
+// word. That cannot tell distances within 16 ulp, nor leave equal ones where they were, and so took
+// another of the shapes that coincide (2 % of the rays at squares over one another in a plane); as two
+// words the same take 1.4 to 2.7 % longer (163.7 us the last) and every hit is the one it was.
 constexpr uint32_t LR_SLOT_F4 = 3u;   // a slot's float4s
 
 __device__ __forceinline__ const float4 *slot_at(const float4 *slots, uint32_t e) { return slots + e; }
 
-// the slab test of an inner slot's children: key k holds child k's entry distance (its bits, the low
-// four replaced by the child's place 3 k), LR_NONE where the child is missed or there is none. Each
-// plane's t is one fused multiply-add of its step, fma(q, s * inv, (corner - o) * inv) (a
-// culling test on boxes that hold the children's: its last bit decides no hit). The step s * inv has
-// the sign of inv (s > 0), and a fused multiply-add is monotone in q, so along an axis whose inv is
-// negative the high plane is the near one: each axis's near and far planes are picked once a node. The
-// keys order as the distances do (positive floats; a negative tmin's entries sort last, which
-// costs order and no hit).
-__device__ __forceinline__ void wide_keys(float4 r0, float4 r1, float4 r2, V3 o, V3 inv, float tmin, float tmax, uint32_t key[4])
+// the slab test of an inner slot's children: t[k] is child k's entry distance, 3e38 where the child is
+// missed or there is none (a hit's is at most tmax, at most 1e30: misses sort last). Each plane's t is
+// one fused multiply-add of its step, fma(q, s * inv, (corner - o) * inv) (a culling test on boxes that
+// hold the children's: its last bit decides no hit). The step s * inv has the sign of inv (s > 0), and
+// a fused multiply-add is monotone in q, so along an axis whose inv is negative the high plane is the
+// near one: each axis's near and far planes are picked once a node.
+__device__ __forceinline__ void wide_test(float4 r0, float4 r1, float4 r2, V3 o, V3 inv, float tmin, float tmax, float t[4])
 {
     const uint32_t w = __float_as_uint(r0.w);
     const float ax = ldexpf(inv.x, (int)(w << 24) >> 24), ay = ldexpf(inv.y, (int)(w << 16) >> 24);
@@ -382,52 +383,60 @@ __device__ __forceinline__ void wide_keys(float4 r0, float4 r1, float4 r2, V3 o,
         const float enter = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, tmin));
         const float leave = fminf(fminf(t1x, t1y), fminf(t1z, tmax));
         const bool none = k >= 2 && w < ((uint32_t)(k + 1) << 24);   // (a node has at least two children)
-        key[k] = none || leave < enter ? LR_NONE : ((__float_as_uint(enter) & ~15u) | LR_SLOT_F4 * k);
+        t[k] = none || leave < enter ? 3e38f : enter;
         // one child after the other: interleaving the four holds all 24 planes at once
         __builtin_amdgcn_sched_barrier(0);
     }
 }
 
-__device__ __forceinline__ void order_(uint32_t &a, uint32_t &b)
+// (equal distances stay where they are: which of them is visited first decides between shapes hit at
+// one distance)
+__device__ __forceinline__ void order_(float &ta, uint32_t &pa, float &tb, uint32_t &pb)
 {
-    const uint32_t lo = min(a, b), hi = max(a, b);
-    a = lo;
-    b = hi;
+    const bool s = tb < ta;
+    const float t = s ? tb : ta;
+    const uint32_t p = s ? pb : pa;
+    tb = s ? ta : tb;
+    pb = s ? pa : pb;
+    ta = t;
+    pa = p;
 }
 
 // The children hit, nearest first: the farther ones stacked (farthest first), the nearest the next
 // entry; false when none was hit. While three more entries fit in LDS each is written at the top
 // whether it is one or not, and the top moves past it if it is.
 template <int STK>
-__device__ __forceinline__ bool wide_next(uint32_t key[4], uint32_t base, const WalkStack &S, int &sp, uint32_t &cur,
+__device__ __forceinline__ bool wide_next(float t[4], uint32_t base, const WalkStack &S, int &sp, uint32_t &cur,
                                           uint32_t *overflow)
 {
-    order_(key[0], key[1]);   // a sorting network over 4
-    order_(key[2], key[3]);
-    order_(key[0], key[2]);
-    order_(key[1], key[3]);
-    order_(key[1], key[2]);
+    uint32_t p[4] = {0u, LR_SLOT_F4, 2u * LR_SLOT_F4, 3u * LR_SLOT_F4};
+    order_(t[0], p[0], t[1], p[1]);   // a sorting network over 4
+    order_(t[2], p[2], t[3], p[3]);
+    order_(t[0], p[0], t[2], p[2]);
+    order_(t[1], p[1], t[3], p[3]);
+    order_(t[1], p[1], t[2], p[2]);
     if (sp + 3 <= STK) {
 #pragma unroll
         for (int k = 3; k >= 1; k--) {
-            S.stk[sp * S.stride] = base + (key[k] & 15u);
-            sp += key[k] != LR_NONE ? 1 : 0;
+            S.stk[sp * S.stride] = base + p[k];
+            sp += t[k] < 3e38f ? 1 : 0;
         }
     } else {
+#pragma unroll
         for (int k = 3; k >= 1; k--) {
-            if (key[k] == LR_NONE) continue;
+            if (!(t[k] < 3e38f)) continue;
             if (sp >= S.cap) {   // cannot happen with a correct depth: said, never silently dropped
                 atomicOr(overflow, 1u);
                 return false;
             }
-            const uint32_t x = base + (key[k] & 15u);
+            const uint32_t x = base + p[k];
             if (sp < STK) S.stk[sp * S.stride] = x;
             else S.spill[(size_t)(sp - STK) * S.sstride] = x;
             sp++;
         }
     }
-    cur = base + (key[0] & 15u);
-    return key[0] != LR_NONE;
+    cur = base + p[0];
+    return t[0] < 3e38f;
 }
 
 // One step: the entry's slot loaded, an inner node's children tested (those hit stacked farthest
@@ -460,9 +469,9 @@ __device__ __forceinline__ bool walk4_step(const float4 *__restrict__ slots, con
             count_node(c);
             count_uniform(c, slots, cur);
         }
-        uint32_t key[4];
-        wide_keys(r0, r1, r2, o, inv, tmin, best.t, key);
-        more = wide_next<STK>(key, __float_as_uint(r1.w), S, sp, cur, overflow);
+        float t[4];
+        wide_test(r0, r1, r2, o, inv, tmin, best.t, t);
+        more = wide_next<STK>(t, __float_as_uint(r1.w), S, sp, cur, overflow);
     }
     if (!more) {
         if (sp == 0) return false;

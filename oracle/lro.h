@@ -100,6 +100,9 @@ typedef struct { uint64_t nodes, tris; } LroCount;
  * triangles tested, summed over the rays (optional). */
 void lro_trace_gpu_layout(const uint32_t *nodes, uint32_t root, const uint32_t *aux, const float *tris,
                           const float *rays, int nrays, int any, LroHit *hits, LroCount *count);
+/* the 4-wide walk over the same layout (root 0, leaves of one triangle): closest or first hits, the
+ * visits in the order lro_trace.c states */
+void lro_trace_wide(const uint32_t *nodes, const uint32_t *aux, const float *tris, const float *rays, int nrays, int any, LroHit *hits);
 /* the CPU's walk (bvh.c:541-663) over the SAH tree, binary or 4-wide as built */
 void lro_trace_sah(const LroSah *b, const float *tris, const float *rays, int nrays, int any, LroHit *hits);
 /* every triangle tested, in id order (the brute force); second: the second-nearest t */

@@ -68,6 +68,7 @@ def lib():
             "lro_sah_info": (None, [P, P, P, P, P]),
             "lro_sah_put_nodes": (None, [P, U, U, P, P]),
             "lro_trace_gpu_layout": (None, [P, U, P, P, P, I, I, P, P]),
+            "lro_trace_wide": (None, [P, P, P, P, I, I, P]),
             "lro_trace_sah": (None, [P, P, P, I, I, P]),
             "lro_trace_brute": (None, [P, I, P, I, I, P, P]),
             "lro_sampler_hash": (U, [U]),
@@ -250,6 +251,15 @@ def trace_gpu_layout(nodes, root, aux, tris, rays, any_hit=False, counts=False):
                                ptr(np.ascontiguousarray(tris, np.float32)), ptr(rays), n, 1 if any_hit else 0, ptr(hits),
                                ctypes.byref(c))
     return (hits, (c.nodes, c.tris)) if counts else hits
+
+
+def trace_wide(nodes, aux, tris, rays, any_hit=False):
+    """lro_trace_wide: the 4-wide walk's hits (n, 4) over a binary tree of one-triangle leaves"""
+    rays = np.ascontiguousarray(rays, np.float32)
+    hits = np.zeros((rays.shape[0], 4), np.float32)
+    lib().lro_trace_wide(ptr(np.ascontiguousarray(nodes, np.uint32)), ptr(np.ascontiguousarray(aux, np.uint32)),
+                         ptr(np.ascontiguousarray(tris, np.float32)), ptr(rays), rays.shape[0], 1 if any_hit else 0, ptr(hits))
+    return hits
 
 
 class Sah:
