@@ -114,7 +114,8 @@ struct EngCtl {
     unsigned int ordered;                   // that queue's first entries that regen put in perm's order (else 0)
     unsigned int qpar, qlen;                // the queue the walks went through, for shade: parity, length
     unsigned int overflow;                  // a walk's stack ran out (1), or met a scene not its own (2)
-    unsigned long long pad[2];
+    unsigned int order, pad0;               // regen orders the bounce rays for the extension walk
+    unsigned long long pad[1];
 };
 
 struct EngProgress {
@@ -162,7 +163,6 @@ struct EngArgs {
     unsigned long long *counts;             // node records and shapes walked (counting extend only)
     unsigned long long *ostat;              // shade's tiles: look-back status of its ordered appends
     int mult;                               // a tile is mult work-groups' widths of entries
-    int order;                              // regen orders the bounce rays for the extension walk
     int refill;                             // k_extend_rf: idle lanes of a wave that take new rays
     int refill_shadow;                      // k_shadow_rf: the same
 };

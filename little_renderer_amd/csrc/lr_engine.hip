@@ -23,11 +23,12 @@ namespace {
 
 constexpr int SBLOCK = 256;
 
-// Bounce rays are ordered by direction (order_rays, lr_engine_k.h) once a one-level scene of this many
-// shapes is rendered: 1280 x 720 x 8 samples of 4000 triangles 4.13 -> 4.05 ms, of 1000 3.38 -> 3.35,
-// of 250 3.12 -> 3.14, the Cornell room's 35 shapes 4.91 -> 5.03 (every ray visits much of so small a
-// tree). Not with two-level scenes, whose rays part inside the instances (19.3 -> 19.9 ms for two
-// frames of 5001 instances).
+// Bounce rays are ordered by direction (order_rays, lr_engine_k.h) while a job of a one-level scene of this
+// many shapes runs, and none of a two-level scene. 1280 x 720 x 8 samples of 16,000 triangles 6.28 -> 5.90
+// ms, of 4000 4.71 -> 4.52, of 1000 3.91 -> 3.85, of 500 3.76 -> 3.74, of 250 3.65 both, the Cornell
+// room's 35 shapes 4.68 -> 4.77 (every ray visits much of so small a tree); medians, runs differ by 0.3
+// %. Not with two-level scenes, whose rays part inside the instances (19.3 -> 19.9 ms for two frames of
+// 5001 instances).
 constexpr int LR_ORDER_SHAPES = 1000;
 
 __global__ __launch_bounds__(SBLOCK) void k_eng_init(EngProgress *prog, uint32_t C)
@@ -62,7 +63,7 @@ __global__ __launch_bounds__(SBLOCK) void k_zero64(long long *p, size_t n)
 // an issue record: global path indices [start, issue_end) are the job's q0, q0 + 1, ...
 __global__ void k_issue(EngCtl *ctl, unsigned long long *iq_start, uint32_t *iq_job, uint32_t *iq_q0,
                         unsigned long long rec, unsigned long long start, uint32_t jslot, uint32_t q0,
-                        unsigned long long issue_end, unsigned long long lo)
+                        unsigned long long issue_end, unsigned long long lo, uint32_t order)
 {
     iq_start[rec & (LR_ISSUE - 1)] = start;
     iq_job[rec & (LR_ISSUE - 1)] = jslot;
@@ -70,6 +71,7 @@ __global__ void k_issue(EngCtl *ctl, unsigned long long *iq_start, uint32_t *iq_
     ctl->iq_hi = rec + 1;
     ctl->issue_end = issue_end;
     ctl->iq_lo = lo;
+    ctl->order = order;
 }
 
 // wf_resolve's output (trace_wave.wgsl:357-378): float4 (sum, count) per pixel
@@ -131,6 +133,7 @@ struct HostJob {
     float rel_error = 0.0f;     // the estimated relative standard error at spp_done
     double t_submit = 0, t_done = 0;
     unsigned long long min_seq = 0;   // the first progress snapshot taken after its admission
+    bool ordered = false, two_level = false;   // its scene's: bounce rays worth ordering; of two levels
 };
 
 struct IssueRec {
@@ -200,7 +203,6 @@ struct LrhEngine {
     hipGraphExec_t gexec = nullptr;
     bool graph_ok = false;
     bool two_level = false;     // a two-level scene has been submitted: the walks that take both
-    bool order = false;         // a scene whose bounce rays are worth ordering has been submitted
     bool multi = false;         // a scene with more than one light has been submitted: shade and
                                 // shadow that take up to three shadow rays a vertex
     double clk_khz = 100000.0, clk_host0 = 0.0;
@@ -247,8 +249,7 @@ void launch_iteration(LrhEngine *e, const LrhTune &t, hipEvent_t *ev = nullptr)
     const int bt = lr_blk_index(t.block_trace), bs = lr_blk_index(t.block_shade), sk = lr_stk_index(t.stack);
     const dim3 gt(e->ncu * t.blocks_per_cu), gs(e->ncu * t.blocks_per_cu);
     const EngArgs At = args_for(e, t.stack, (size_t)gt.x * t.block_trace, t.tile, t.refill, t.refill_shadow);
-    EngArgs As = args_for(e, t.stack, 0, t.tile);
-    As.order = e->order && !e->two_level ? 1 : 0;
+    const EngArgs As = args_for(e, t.stack, 0, t.tile);
     const int tl = e->two_level ? 1 : 0, ml = e->multi ? 1 : 0, cnt = e->counting ? 1 : 0;
     const bool rf = !tl && t.refill > 0, srf = !tl && !ml && t.refill_shadow > 0;
     if (ev) (void)hipEventRecord(ev[0], e->stream);
@@ -553,14 +554,12 @@ int job_admit(LrhEngine *e, const LrhJob *j, int *slot_out)
     h.t_submit = now_ms();
     h.min_seq = e->seq_next;
     const LrhPtScene *s = j->scene;
+    h.two_level = s->two_level;
+    h.ordered = !s->two_level && s->nprims + s->ntris >= LR_ORDER_SHAPES;
     if (s->two_level && !e->two_level) {
         // from now on the walks that take two-level scenes too; the graphs already launched
         // run before this job's first paths are issued (the same stream)
         e->two_level = true;
-        e->graph_ok = false;
-    }
-    if (!s->two_level && s->nprims + s->ntris >= LR_ORDER_SHAPES && !e->order) {   // likewise, regen that orders bounce rays
-        e->order = true;
         e->graph_ok = false;
     }
     if (lr_scene_multi_light(s) && !e->multi) {   // likewise, shade and shadow for several lights
@@ -639,6 +638,19 @@ int job_admit(LrhEngine *e, const LrhJob *j, int *slot_out)
     return 0;
 }
 
+// regen orders the bounce rays (LR_ORDER_SHAPES): by the jobs running as paths are issued, so that a
+// queue of small scenes, or of large ones after instanced ones, is walked as in a new engine
+uint32_t order_bounces(const LrhEngine *e)
+{
+    uint32_t order = 0;
+    for (const HostJob &h : e->hj) {
+        if (h.state != LRH_JOB_RUNNING) continue;
+        if (h.two_level) return 0;
+        order |= h.ordered ? 1u : 0u;
+    }
+    return order;
+}
+
 // issues the next n paths of job `slot` as one record
 int issue_chunk(LrhEngine *e, int slot, unsigned long long n)
 {
@@ -647,7 +659,7 @@ int issue_chunk(LrhEngine *e, int slot, unsigned long long n)
     e->issue_end += n;
     e->recs.push_back(IssueRec{rec, start, start + n});
     hipLaunchKernelGGL(k_issue, dim3(1), dim3(1), 0, e->stream, &e->prog->ctl, e->iq_start, e->iq_job, e->iq_q0, rec,
-                       start, (uint32_t)slot, (uint32_t)h.issued, e->issue_end, issue_lo(e));
+                       start, (uint32_t)slot, (uint32_t)h.issued, e->issue_end, issue_lo(e), order_bounces(e));
     h.issued += n;
     ENG_HIP(hipGetLastError());
     return 0;

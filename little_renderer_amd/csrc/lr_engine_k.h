@@ -543,7 +543,7 @@ __global__ __launch_bounds__(BLK) void k_regen(EngArgs A)
     // leave two to each of 256 compute units, 8 to 32 rounds
     const uint32_t fill = start / (512u * BLK);
     const int rounds = fill < 16u ? 8 : (fill < 32u ? 16 : 32);
-    const bool order = A.order && start >= ORDER_MIN;
+    const bool order = ctl->order && start >= ORDER_MIN;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctl->claimed = n;
         ctl->ordered = order ? start : 0u;

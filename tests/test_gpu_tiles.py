@@ -130,3 +130,38 @@ def test_ragged_images_match_the_oracle(world, w, h):
     assert np.median(rel) < 1e-5 and np.mean(rel > 1e-3) < 0.01
     eng.close()
     ps.close()
+
+
+def test_bounce_rays_are_ordered_by_the_jobs_that_run(world):
+    # the steps of a wave of the extension walk tell the order its rays came in: a small scene's job
+    # (never ordered) after a large one's, a large one's (ordered) after an instanced one's, each as
+    # in a new engine
+    ctx, big = world
+    sc = lr.cornell(900, 700)
+    small = lr.PtScene(ctx, sc["prims"], sc["tris"], sc["mats"], 0, sc["eps"], sc["margin"])
+    _, (mtris, first, mats, inst) = glow_scene(box=True)
+    glow = lr.PtScene.instanced(ctx, mtris, first, mats, inst, eps=2e-3)
+    glow.set_sky(lr.sky(64))
+    depth = max(64, big.info()[0], glow.info()[0])
+    jobs = {"small": lr.make_job(small, sc["cam"], 900, 700, 1, seed=3),
+            "big": lr.make_job(big, lr.batch_camera(4, 900, 700), 900, 700, 1, seed=4),
+            "glow": lr.make_job(glow, lr.camera_make((-200, 20, 0), (0, 20, 0), (0, 1, 0), 40.0, 1.5), 90, 60, 1, seed=2)}
+
+    def steps(*names):
+        eng = lr.Engine(ctx, slots_log2=20, max_tree_depth=depth, image_bytes=32 << 20)
+        eng.counting(True)
+        for k in names:
+            before = eng.stats().wave_node_steps
+            i = eng.submit(jobs[k])
+            eng.drain()
+            eng.release(i)
+        n = eng.stats().wave_node_steps - before
+        eng.close()
+        return n
+
+    alone = {k: steps(k) for k in ("small", "big")}
+    assert alone["small"] == steps("small")          # (a count to compare by)
+    assert steps("big", "small") == alone["small"]
+    assert steps("glow", "big") == alone["big"]
+    glow.close()
+    small.close()
