@@ -38,7 +38,6 @@ passes before it priced as for the LBVH (bounds 32, morton 40, sort 64 per primi
 HBM_PEAK_GBS = 8000.0           # MI355X HBM3E
 
 NODE_BYTES_BINARY = 32          # the reference's node (put_nodes)
-NODE_BYTES_WIDE = 64            # a compressed 4-wide node with its four child references
 SLOT_BYTES = 48                 # the engine's walks: a 4-wide node or a leaf's shape and id
 RAY_BYTES, HIT_BYTES, SHAPE_BYTES = 32, 16, 52
 

@@ -58,6 +58,10 @@ int lro_lbvh_bottom_up(const uint32_t *sorted_codes, const uint32_t *sorted_item
 int lro_ploc(const uint32_t *sorted_codes, const uint32_t *sorted_items, const float *boxes, int n,
              uint32_t node0, uint32_t ref0, uint32_t ref_add, uint32_t *nodes, uint32_t *aux, int *depth,
              uint64_t *live);
+/* the same; *rounds_above (optional): the rounds that more than `above` clusters were left for */
+int lro_ploc_above(const uint32_t *sorted_codes, const uint32_t *sorted_items, const float *boxes, int n,
+                   uint32_t node0, uint32_t ref0, uint32_t ref_add, uint32_t *nodes, uint32_t *aux, int *depth,
+                   uint64_t *live, uint32_t above, int *rounds_above);
 /* check_tree (trace_gpu.c:768-805): 1 if nodes are one tree over exactly n leaves; its cost
  * (sum of areas / root's, in double) and depth */
 int lro_check_tree(const uint32_t *nodes, int n, uint32_t node0, double *cost, int *depth);

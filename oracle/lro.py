@@ -60,6 +60,7 @@ def lib():
             "lro_lbvh": (I, [P, P, P, I, U, U, U, P, P]),
             "lro_lbvh_bottom_up": (I, [P, P, P, I, U, U, U, P, P]),
             "lro_ploc": (I, [P, P, P, I, U, U, U, P, P, P, P]),
+            "lro_ploc_above": (I, [P, P, P, I, U, U, U, P, P, P, P, U, P]),
             "lro_check_tree": (I, [P, I, U, P, P]),
             "lro_build_tris": (I, [P, I, I, U, U, U, P, P, P]),
             "lro_sah_build": (P, [P, I, I, I, I]),
@@ -212,15 +213,19 @@ def lbvh(sc, si, boxes, node0=0, ref0=0, ref_add=0, bottom_up=False):
     return nodes, aux, depth
 
 
-def ploc(sc, si, boxes, node0=0, ref0=0, ref_add=0, live=False):
+def ploc(sc, si, boxes, node0=0, ref0=0, ref_add=0, live=False, above=None):
+    """(nodes, aux, depth, rounds), with live the clusters summed over the rounds after them, with above
+    (a number of clusters) the rounds that more than that were left for after that"""
     n = sc.shape[0]
     nodes = np.zeros((max(2 * n - 1, 1), 8), np.uint32)
     aux = np.zeros(max(n, 1), np.uint32)
     depth = ctypes.c_int()
     lv = ctypes.c_uint64()
-    rounds = lib().lro_ploc(ptr(sc), ptr(si), ptr(boxes), n, node0, ref0, ref_add, ptr(nodes), ptr(aux),
-                            ctypes.byref(depth), ctypes.byref(lv))
-    return (nodes, aux, depth.value, rounds, lv.value) if live else (nodes, aux, depth.value, rounds)
+    ra = ctypes.c_int()
+    rounds = lib().lro_ploc_above(ptr(sc), ptr(si), ptr(boxes), n, node0, ref0, ref_add, ptr(nodes), ptr(aux),
+                                  ctypes.byref(depth), ctypes.byref(lv), above or 0, ctypes.byref(ra))
+    out = (nodes, aux, depth.value, rounds)
+    return out + ((lv.value,) if live else ()) + ((ra.value,) if above is not None else ())
 
 
 def check_tree(nodes, n, node0=0):

@@ -282,7 +282,15 @@ int lro_ploc(const uint32_t *codes, const uint32_t *items, const float *boxes, i
              uint32_t node0, uint32_t ref0, uint32_t ref_add, uint32_t *nodes, uint32_t *aux, int *depth,
              uint64_t *live)
 {
+    return lro_ploc_above(codes, items, boxes, n, node0, ref0, ref_add, nodes, aux, depth, live, 0, NULL);
+}
+
+int lro_ploc_above(const uint32_t *codes, const uint32_t *items, const float *boxes, int n,
+                   uint32_t node0, uint32_t ref0, uint32_t ref_add, uint32_t *nodes, uint32_t *aux, int *depth,
+                   uint64_t *live, uint32_t above, int *rounds_above)
+{
     if (live) *live = 0;
+    if (rounds_above) *rounds_above = 0;
     if (n <= 2) {                                 /* build_queue: PLOC only above 2 (trace_gpu.c:615) */
         int d = lro_lbvh(codes, items, boxes, n, node0, ref0, ref_add, nodes, aux);
         if (depth) *depth = d;
@@ -305,6 +313,7 @@ int lro_ploc(const uint32_t *codes, const uint32_t *items, const float *boxes, i
     int rounds = 0;
     while (nc > 1) {
         if (live) *live += nc;
+        if (rounds_above && nc > above) ++*rounds_above;
         /* nn (trace_ploc.wgsl:99-128) */
         for (uint32_t i = 0; i < nc; i++) {
             const float *bi = bx + 6 * (size_t)list[i];

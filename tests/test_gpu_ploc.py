@@ -5,6 +5,10 @@ serve the others, in tiles of 352 or 864 positions a work-group, or over a list 
 LDS, from 96 clusters down in one wave. Sizes around those edges; boxes with many equal distances
 (the tie rule decides every merge); and boxes whose areas overflow, which the search leaves to the
 general one.
+
+The build's own figures too: depth, clusters, and rounds. The rounds from n down to 1024 clusters are
+launched in a number planned from n (5/6 left by each, two more), and a build counts those even where
+fewer were needed: the sizes have some where fewer are, and some where more.
 """
 import numpy as np
 import pytest
@@ -47,6 +51,13 @@ def huge(n, rng):
     return np.where(far[:, None], lo * 1e20, lo), np.where(far[:, None], lo * 1e20 + 1e18, hi)
 
 
+def planned(n):
+    r = 0
+    while n > 1024:
+        n, r = n * 5 // 6, r + 1
+    return min(r + 2, 128) if r else 0
+
+
 @pytest.mark.parametrize("make", [soup, lattice, huge])
 @pytest.mark.parametrize("n", [3, 16, 17, 31, 32, 33, 95, 96, 97, 1023, 1056, 1400, 4500, 200_000])
 def test_rounds_match_the_oracle(ctx, make, n):
@@ -61,8 +72,13 @@ def test_rounds_match_the_oracle(ctx, make, n):
     torch.cuda.synchronize()
     st = ctx.build(b, n, nodes, aux, lr.PLOC, sorted_out=srt)
     sc, si = np.split(srt.cpu().numpy().view(np.uint32), 2)
-    want, waux, depth, rounds, live = lro.ploc(sc, si, boxes, live=True)
+    want, waux, depth, rounds, live, made = lro.ploc(sc, si, boxes, live=True, above=1024)
     assert np.array_equal(aux.cpu().numpy().view(np.uint32), waux)
     got = nodes.cpu().numpy().view(np.uint32)
     assert np.array_equal(got, want), f"nodes differ at {np.nonzero((got != want).any(1))[0][:8]}"
-    assert (st.depth, st.clusters) == (depth, live)
+    print(f"  rounds {rounds}, {made} of them launched ones, {planned(n)} planned", flush=True)
+    assert (st.depth, st.clusters, st.rounds) == (depth, live, rounds + max(0, planned(n) - made))
+    if n > 1024 and make is soup:          # (either kind is among the sizes)
+        assert made < planned(n)
+    if n == 200_000 and make is not soup:
+        assert made > planned(n)

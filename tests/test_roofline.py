@@ -4,10 +4,11 @@ from little_renderer_amd import roofline as rf
 
 
 def test_walk_bytes_by_hand():
-    # 3 rays, 10 wide nodes, 4 triangles: 3 x (32 + 16) + 10 x 64 + 4 x (48 + 4)
-    assert rf.walk_bytes(3, 10, 4, rf.NODE_BYTES_WIDE) == 144 + 640 + 208
-    # the reference's binary node is 32 bytes
+    # the 4-wide walks: 3 rays, 10 nodes and 4 shapes, a slot of 48 bytes each: 3 x (32 + 16) + 14 x 48
+    assert rf.walk_bytes(3, 10, 4, rf.SLOT_BYTES, rf.SLOT_BYTES) == 144 + 672
+    # the reference's binary node is 32 bytes, a triangle and its aux entry 48 + 4
     assert rf.walk_bytes(1, 1, 0, rf.NODE_BYTES_BINARY) == 48 + 32
+    assert rf.walk_bytes(2, 5, 3, rf.NODE_BYTES_BINARY) == 96 + 160 + 156
     assert rf.walk_bytes(0, 0, 0, 64) == 0
 
 
