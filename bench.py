@@ -350,16 +350,16 @@ def kernel_traffic(run_args, regex, kname, what):
 
 
 def live_traffic(a, tune):
-    """HBM bytes per launch of the batched extension kernel (kernel_traffic: the same jobs and
-    launch shape, one batch, the extension kernel's dispatches only)."""
+    """HBM bytes per launch of the batched walks (kernel_traffic: the same jobs and launch shape, one
+    batch, the dispatches of the walks' one launch only, or with lanes refilled the extension walk's)."""
     t = tune.as_dict()
     shape = ",".join(str(t[k]) for k in ("block_trace", "stack", "block_shade", "blocks_per_cu", "tile",
                                           "iters_per_graph", "refill", "refill_shadow"))
     kname = (f"k_extend_rf<{t['block_trace']}, {t['stack']}, false>" if t["refill"] > 0
-             else f"k_extend<{t['block_trace']}, {t['stack']}, false, false>")
+             else f"k_walks<{t['block_trace']}, {t['stack']}, false, false>")
     run_args = ["--tune", shape, "--jobs", str(a.jobs), "--serve-requests", "0", "--no-cpu", "--steps", "1",
                 "--warmup", "0", "--skip-plain", "--no-traffic"]
-    return kernel_traffic(run_args, "k_extend", kname, "the extension kernel")
+    return kernel_traffic(run_args, "k_extend" if t["refill"] > 0 else "k_walks", kname, "the walks")
 
 
 def bench_batched(a, torch, lr):
@@ -457,9 +457,11 @@ def bench_batched(a, torch, lr):
     order = np.argsort([w * h * spp for (_, w, h, spp) in plan], kind="stable")
     plain_sjf = np.cumsum(dur[order]) if len(dur) == len(plan) else []
 
-    # ---- kernel times (events around each kernel, iterations launched without the graph) and the
-    # roofline of the dominant kernel: the extension walk's algorithmic bytes from its own counters
-    # (4-wide nodes x 128 B, shapes x 52 B, ray 32 B + hit 16 B per ray) over its time ----
+    # ---- kernel times (events around each kernel, iterations launched without the graph): the walks
+    # each alone, then as the timed region has them, in one launch. The roofline of the dominant
+    # kernel, the walks': their algorithmic bytes from their own counters (a 48-byte slot a node or
+    # shape, ray 32 B + hit 16 B per ray) over that launch's time ----
+    wms, wl = joint_walks(eng, batch)
     eng.profiling(True)
     k0 = eng.stats()
     batch()
@@ -473,12 +475,6 @@ def bench_batched(a, torch, lr):
     batch()
     c1 = eng.stats()
     eng.counting(False)
-    nodes = c1.node_fetches - c0.node_fetches
-    shapes = c1.shape_tests - c0.shape_tests
-    rext = c1.rays_ext - c0.rays_ext
-    alg = rf.walk_bytes(rext, nodes, shapes, rf.SLOT_BYTES, rf.SLOT_BYTES)
-    dom = max(kms, key=kms.get)
-    achieved = alg / (kms["extend"] * 1e-3) / 1e9
     traffic, traffic_detail = (None, {"why": "--no-traffic"}) if a.no_traffic else live_traffic(a, tune)
 
     out = {
@@ -509,14 +505,11 @@ def bench_batched(a, torch, lr):
         "speedup_vs_plain": rnd(value / plain_mrays, 3) if plain_mrays else None,
         "equal_error": {"images_bit_identical": same, "of": 0 if a.skip_plain else len(jobs),
                         "note": "same samples per (job, pixel, index), fixed-point sums: equal RMSE by construction"},
-        "kernel_ms_per_launch": {n: round(kms[n] / max(kl[n], 1), 4) for n in names},
-        "kernel_ms_total": {n: round(kms[n], 2) for n in names},
-        "roofline": {"bound": "hbm", "kernel": "extend", "dominant": dom, "achieved": round(achieved, 2),
-                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": traffic,
-                     "traffic_detail": traffic_detail,
-                     "alg_bytes_per_launch": alg // max(kl["extend"], 1), "node_fetches": nodes, "shape_tests": shapes,
-                     "rays": rext, "launches": kl["extend"]},
+        "kernel_ms_per_launch": {**{n: round(kms[n] / max(kl[n], 1), 4) for n in names}, "walks": round(wms / max(wl, 1), 4)},
+        "kernel_ms_total": {**{n: round(kms[n], 2) for n in names}, "walks": round(wms, 2)},
+        "roofline": dict(walks_roofline(c0, c1, wms, wl), dominant=max({"walks": wms, "regen": kms["regen"], "shade": kms["shade"]}.items(),
+                                                                       key=lambda kv: kv[1])[0],
+                         traffic=traffic, traffic_detail=traffic_detail),
     }
     out.update(walk_counts(c0, c1, kms, kl))
     # shade's roofline: its algorithmic bytes (roofline.shade_bytes: the entries shaded, the paths
@@ -552,7 +545,7 @@ def bench_caustics(a, torch, lr):
     the timed steps: the path tracer's closest-hit and shadow rays and the light tracer's
     closest-hit rays and rays towards the camera, all counted on the device. The roofline is the
     light kernels' (k_light_first + k_light_rest, a pair a chunk of 2^22 light paths: algorithmic
-    bytes from their own counters, 48 B a ray, 64 B a 4-wide node, 52 B a shape, over their time
+    bytes from their own counters, 48 B a ray, a 48-byte slot a 4-wide node or shape, over their time
     from HIP events on the engine's stream; the traffic a pair's)."""
     steps = a.steps or 5
     warm = 1 if a.warmup is None else a.warmup
@@ -882,10 +875,15 @@ def bench_instanced(a, torch, lr):
     dt = time.perf_counter() - t0
     s1 = eng.stats()
     rays = (s1.rays_ext - s0.rays_ext) + (s1.rays_shadow - s0.rays_shadow)
+
+    def one():
+        frame(0)
+        finish()
+
+    wms, wl = joint_walks(eng, one)
     eng.profiling(True)
     k0 = eng.stats()
-    frame(0)
-    finish()
+    one()
     k1 = eng.stats()
     eng.profiling(False)
     names = ["regen", "extend", "shade", "shadow"]
@@ -893,13 +891,9 @@ def bench_instanced(a, torch, lr):
     kl = {n: k1.kernel_launches[q] - k0.kernel_launches[q] for q, n in enumerate(names)}
     eng.counting(True)
     c0 = eng.stats()
-    frame(0)
-    finish()
+    one()
     c1 = eng.stats()
     eng.counting(False)
-    nodes, shapes, rext = c1.node_fetches - c0.node_fetches, c1.shape_tests - c0.shape_tests, c1.rays_ext - c0.rays_ext
-    alg = rf.walk_bytes(rext, nodes, shapes, rf.SLOT_BYTES, rf.SLOT_BYTES)
-    achieved = alg / (kms["extend"] * 1e-3) / 1e9
     ninst = len(w0["instances"])
     out = {
         "metric": METRIC + " (instanced workload)",
@@ -933,12 +927,9 @@ def bench_instanced(a, torch, lr):
         "tlas_refitted_frames": refits,
         "tlas_build_ms": round(float(np.mean(builds)), 4),
         "tlas_build_mprims_s": round(ninst / (float(np.mean(builds)) * 1e3), 2),
-        "kernel_ms_per_launch": {n: round(kms[n] / max(kl[n], 1), 4) for n in names},
-        "kernel_ms_total": {n: round(kms[n], 3) for n in names},
-        "roofline": {"bound": "hbm", "kernel": "extend", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-                     "alg_bytes_per_launch": alg // max(kl["extend"], 1), "node_fetches": nodes, "shape_tests": shapes,
-                     "rays": rext},
+        "kernel_ms_per_launch": {**{n: round(kms[n] / max(kl[n], 1), 4) for n in names}, "walks": round(wms / max(wl, 1), 4)},
+        "kernel_ms_total": {**{n: round(kms[n], 3) for n in names}, "walks": round(wms, 3)},
+        "roofline": dict(walks_roofline(c0, c1, wms, wl), traffic=None),
         **walk_counts(c0, c1, kms, kl),
         "cpu_baseline": {"value": None, "unit": "Mrays/s", "cores": None, "kind": "reference",
                          "sample": "not run for this workload: the reference's instanced CPU path is not built here"},
@@ -952,21 +943,50 @@ def bench_instanced(a, torch, lr):
     return out
 
 
+def joint_walks(eng, run):
+    """run() with the kernels timed and the two walks in the one launch they share in the timed
+    region: (its total ms, its launches); where a launch shape refills a walk's lanes, both walks' launches"""
+    eng.profiling(2)
+    k0 = eng.stats()
+    run()
+    k1 = eng.stats()
+    eng.profiling(False)
+    ms = [k1.kernel_ms[q] - k0.kernel_ms[q] for q in (1, 3)]     # (extend's place, shadow's: 0 in one launch)
+    return sum(ms), k1.kernel_launches[1] - k0.kernel_launches[1]
+
+
+def walks_roofline(c0, c1, ms, launches):
+    """the walks' launch: both walks' algorithmic bytes, from the counting run, over its time"""
+    d = lambda f: getattr(c1, f) - getattr(c0, f)
+    rays = d("rays_ext") + d("rays_shadow")
+    nodes = d("node_fetches") + d("shadow_node_fetches")
+    shapes = d("shape_tests") + d("shadow_shape_tests")
+    alg = rf.walk_bytes(rays, nodes, shapes, rf.SLOT_BYTES, rf.SLOT_BYTES)
+    achieved, frac = rf.roofline(alg, ms)
+    return {"bound": "hbm", "kernel": "walks", "launch": "k_walks: an iteration's extension and shadow rays, as timed",
+            "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(frac, 4),
+            "alg_bytes_per_launch": alg // max(launches, 1), "node_fetches": nodes, "shape_tests": shapes, "rays": rays,
+            "launches": launches}
+
+
 def walk_counts(c0, c1, kms, kl):
-    """The counting run's figures for both walks: the shadow walk's roofline (48 B per ray: the
-    ray and its light's contribution; 64 B per wide node, 52 B per shape, like the extension
-    walk's) over its profiled time, and for each walk the share of a wave's lanes at work in its
-    node steps and its shape steps (node records / (64 x the waves' node steps), and so on)."""
+    """The counting run's figures for the walks launched each alone: a roofline of either (48 B per
+    ray, a 48-byte slot a node or shape) over its profiled time, and the share of a wave's lanes at
+    work in its node steps and its shape steps (node records / (64 x the waves' node steps), and so
+    on)."""
     d = lambda f: getattr(c1, f) - getattr(c0, f)
     share = lambda a, b: round(a / (64.0 * b), 4) if b else None
-    srays, snodes, sshapes = d("rays_shadow"), d("shadow_node_fetches"), d("shadow_shape_tests")
-    salg = rf.walk_bytes(srays, snodes, sshapes, rf.SLOT_BYTES, rf.SLOT_BYTES)
-    sach = salg / (kms["shadow"] * 1e-3) / 1e9 if kms["shadow"] > 0 else 0.0
+    def alone(kernel, rays, nodes, shapes):
+        alg = rf.walk_bytes(rays, nodes, shapes, rf.SLOT_BYTES, rf.SLOT_BYTES)
+        gbs, frac = rf.roofline(alg, kms[kernel])
+        return {"bound": "hbm", "kernel": kernel, "launch": "alone", "achieved": round(gbs, 2), "peak": HBM_PEAK_GBS,
+                "unit": "GB/s", "frac": round(frac, 4), "alg_bytes_per_launch": alg // max(kl[kernel], 1),
+                "node_fetches": nodes, "shape_tests": shapes, "rays": rays}
+
+    snodes, sshapes = d("shadow_node_fetches"), d("shadow_shape_tests")
     return {
-        "shadow_roofline": {"bound": "hbm", "kernel": "shadow", "achieved": round(sach, 2), "peak": HBM_PEAK_GBS,
-                            "unit": "GB/s", "frac": round(sach / HBM_PEAK_GBS, 4),
-                            "alg_bytes_per_launch": salg // max(kl["shadow"], 1), "node_fetches": snodes,
-                            "shape_tests": sshapes, "rays": srays},
+        "extend_roofline": alone("extend", d("rays_ext"), d("node_fetches"), d("shape_tests")),
+        "shadow_roofline": alone("shadow", d("rays_shadow"), snodes, sshapes),
         "lane_shares": {"extend_node_steps": share(d("node_fetches"), d("wave_node_steps")),
                         "extend_shape_steps": share(d("shape_tests"), d("wave_shape_steps")),
                         "shadow_node_steps": share(snodes, d("shadow_wave_node_steps")),

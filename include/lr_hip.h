@@ -392,7 +392,8 @@ typedef struct {
     uint64_t jobs_done;
     uint64_t node_fetches;  /* with counting on: node records read by the extension walks */
     uint64_t shape_tests;   /* and shapes tested */
-    double kernel_ms[4];    /* with profiling on: device time of regen, extend, shade, shadow */
+    double kernel_ms[4];    /* with profiling on: device time of regen, extend, shade, shadow (profiling
+                             * 2: both walks, one launch, in extend's place and none in shadow's) */
     uint64_t kernel_launches[4];
     /* with counting on: the extension walks' wave steps (node steps, shape steps; a step is one
      * wave's pass through that part of the walk, whatever lanes take part), so that
@@ -433,7 +434,8 @@ int lrh_engine_tune_get(const LrhEngine *e, LrhTune *t);
  * steps (slower kernels) */
 int lrh_engine_counting(LrhEngine *e, int on);
 /* profiling on: lrh_engine_pump launches the iterations kernel by kernel between hipEvents on
- * the engine's stream (no graph) and sums each kernel's time into the stats */
+ * the engine's stream (no graph) and sums each kernel's time into the stats. An iteration's two
+ * walks are one launch otherwise; on = 1 launches each alone, on = 2 the one launch. */
 int lrh_engine_profiling(LrhEngine *e, int on);
 /* Admits a job (its image cleared): LRH_EAGAIN if its image or a job slot cannot be had until
  * others are released. *id names it. Its paths are issued to the device in chunks of at most

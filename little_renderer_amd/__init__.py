@@ -740,7 +740,8 @@ class Engine:
         _check(lib().lrh_engine_counting(self._e, 1 if on else 0))
 
     def profiling(self, on):
-        _check(lib().lrh_engine_profiling(self._e, 1 if on else 0))
+        """True: each kernel timed alone; 2: the two walks in the one launch they otherwise share"""
+        _check(lib().lrh_engine_profiling(self._e, int(on)))
 
     def submit(self, job):
         """the job's id, or None if it does not fit now"""

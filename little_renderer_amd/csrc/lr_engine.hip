@@ -186,8 +186,8 @@ struct LrhEngine {
     uint64_t jobs_done = 0;
     LrhTune tune{256, 16, 256, 8, 1, 8, 0, 0};   // the best measured on the batched workload (MI355X)
     bool counting = false;
-    // profiling: iterations launched one kernel at a time between events (no graph)
-    bool profiling = false;
+    // profiling: iterations launched one kernel at a time between events (no graph); 2: the walks in one launch
+    int profiling = 0;
     std::vector<hipEvent_t> pevs;
     double kms[4] = {0, 0, 0, 0};
     uint64_t klaunch[4] = {0, 0, 0, 0};
@@ -241,8 +241,16 @@ EngArgs args_for(const LrhEngine *e, int stack, size_t threads, int mult, int re
     return A;
 }
 
+bool refilled(const LrhEngine *e, int refill) { return !e->two_level && refill > 0; }
+// the walks go in one launch (not where they are counted or a walk's lanes refilled)
+bool walks_joint(const LrhEngine *e, const LrhTune &t)
+{
+    return !e->counting && !refilled(e, t.refill) && !(refilled(e, t.refill_shadow) && !e->multi);
+}
+
 // One iteration in the persistent grids of the batched form: regen, the walks, shade. ev (profiling):
-// 5 events around regen, the extension walk, the shadow walk and shade, each a launch of its own
+// 5 events around regen, the extension walk, the shadow walk and shade, each a launch of its own (profiling
+// 2: the walks' one launch in the extension walk's place, and none between the next two)
 void launch_iteration(LrhEngine *e, const LrhTune &t, hipEvent_t *ev = nullptr)
 {
     const LrEngTable &T = table();
@@ -251,12 +259,14 @@ void launch_iteration(LrhEngine *e, const LrhTune &t, hipEvent_t *ev = nullptr)
     const EngArgs At = args_for(e, t.stack, (size_t)gt.x * t.block_trace, t.tile, t.refill, t.refill_shadow);
     const EngArgs As = args_for(e, t.stack, 0, t.tile);
     const int tl = e->two_level ? 1 : 0, ml = e->multi ? 1 : 0, cnt = e->counting ? 1 : 0;
-    const bool rf = !tl && t.refill > 0, srf = !tl && !ml && t.refill_shadow > 0;
+    const bool rf = refilled(e, t.refill), srf = !ml && refilled(e, t.refill_shadow);
     if (ev) (void)hipEventRecord(ev[0], e->stream);
     T.regen[bs](gs, e->stream, As);
     if (ev) (void)hipEventRecord(ev[1], e->stream);
-    if (!ev && !cnt && !rf && !srf) T.walks[bt][sk][tl][ml](gt, e->stream, At);
-    else {
+    if ((!ev || e->profiling == 2) && walks_joint(e, t)) {
+        T.walks[bt][sk][tl][ml](gt, e->stream, At);
+        if (ev) (void)hipEventRecord(ev[2], e->stream);
+    } else {
         if (rf) T.extend_rf[bt][sk][cnt](gt, e->stream, At);
         else (cnt ? T.extend_count : T.extend)[bt][sk][tl](gt, e->stream, At);
         if (ev) (void)hipEventRecord(ev[2], e->stream);
@@ -281,10 +291,12 @@ int launch_profiled(LrhEngine *e)
     ENG_HIP(hipGetLastError());
     ENG_HIP(hipEventSynchronize(e->pevs[5 * G - 1]));
     constexpr int stat[4] = {0, 1, 3, 2};   // (the stats' order: regen, extend, shade, shadow)
+    const bool joint = e->profiling == 2 && walks_joint(e, e->tune);
     for (int i = 0; i < G; i++)
         for (int k = 0; k < 4; k++) {
             float ms = 0.0f;
             ENG_HIP(hipEventElapsedTime(&ms, e->pevs[5 * i + k], e->pevs[5 * i + k + 1]));
+            if (k == 2 && joint) continue;
             e->kms[stat[k]] += ms;
             e->klaunch[stat[k]]++;
         }
@@ -1182,7 +1194,7 @@ int lrh_engine_stats(LrhEngine *e, LrhEngineStats *st)
 int lrh_engine_profiling(LrhEngine *e, int on)
 {
     if (!e) return lr_fail(LRH_EINVAL, "lrh_engine_profiling: no engine");
-    e->profiling = on != 0;
+    e->profiling = on == 2 ? 2 : (on ? 1 : 0);
     return 0;
 }
 

@@ -115,6 +115,24 @@ def test_ordered_bounce_rays_change_no_image(world, w, h, spp, block_shade):
     eng.close()
 
 
+@pytest.mark.parametrize("on", [1, 2])
+def test_profiled_launches(world, on):
+    # timed alone (1) each walk is a launch an iteration, as they go otherwise (2) both are one
+    ctx, ps = world
+    eng = lr.Engine(ctx, slots_log2=15, max_tree_depth=max(64, ps.info()[0]), image_bytes=16 << 20)
+    job = lr.make_job(ps, lr.batch_camera(11, 190, 110), 190, 110, 3, seed=1)
+    eng.profiling(on)
+    i = eng.submit(job)
+    eng.drain()
+    eng.profiling(False)
+    st = eng.stats()
+    n = st.kernel_launches[0]
+    assert list(st.kernel_launches) == [n, n, n, n if on == 1 else 0] and n > 0
+    assert all((st.kernel_ms[k] > 0) == (st.kernel_launches[k] > 0) for k in range(4))
+    assert np.array_equal(image(eng, i, 190, 110), image(eng, eng.plain(job), 190, 110))
+    eng.close()
+
+
 @pytest.mark.parametrize("w, h", [(1, 1), (3, 65), (7, 9), (8, 8), (9, 7), (65, 3), (24, 20)])
 def test_ragged_images_match_the_oracle(world, w, h):
     ctx, _ = world
