@@ -1528,8 +1528,11 @@ __device__ __forceinline__ int pc_coord(float x, float size, bool normal_axis)
 }
 // a work-group's sums before they go to the table: PC_LDS cells keyed by their slot (open
 // addressing, 8 probes; a photon whose cell finds no room goes to the table at once). A focused
-// caustic sends many photons to a few cells, whose adds would otherwise queue at their slots.
-constexpr int PC_LDS = 256;
+// caustic sends many photons to a few cells, whose adds would otherwise queue at their slots: bound by
+// those queues, the faster the walks the longer (with 256 cells 4.2M paths of the caustics room went from
+// 4.22 to 4.72 ms as the walks' slots came; with 512 they take 2.19, and the registers' 4 waves a SIMD
+// still fit; with 1024 and 3 waves 1.96, a soup's paths the same either way).
+constexpr int PC_LDS = 512;
 struct PcLds {
     unsigned long long sum[PC_LDS][3];
     uint32_t cnt[PC_LDS];
