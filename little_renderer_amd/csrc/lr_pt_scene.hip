@@ -67,10 +67,9 @@ struct WideLeaves {
     uint32_t nprims;
 };
 
-// the leaf over aux entry e (the builders' leaves hold one shape each) into a slot
-__device__ __forceinline__ void put_leaf(const WideLeaves &L, uint32_t e, float4 *slot)
+// the leaf of shape id (the builders' leaves hold one each) into a slot
+__device__ __forceinline__ void put_leaf(const WideLeaves &L, uint32_t id, float4 *slot)
 {
-    const uint32_t id = L.aux[e];
     const float tag = __uint_as_float(LR_LEAF), idf = __uint_as_float(id);
     float4 a = make_float4(0.0f, 0.0f, 0.0f, tag), b = make_float4(0.0f, 0.0f, 0.0f, idf), c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (L.inst) {
@@ -104,7 +103,7 @@ __global__ void k_collapse_init(const float4 *__restrict__ nodes, WideTask *q0, 
     for (int l = 0; l <= levels + 1; l++) cnt[l] = 0;
     *nslots = slot0 + 1;
     if (__float_as_uint(nodes[2 * (size_t)root + 1].w) & LR_LEAF) {
-        put_leaf(L, __float_as_uint(nodes[2 * (size_t)root].w), slots + LR_SLOT_F4 * (size_t)slot0);
+        put_leaf(L, L.aux[__float_as_uint(nodes[2 * (size_t)root].w)], slots + LR_SLOT_F4 * (size_t)slot0);
         return;
     }
     q0[0] = WideTask{root, slot0};
@@ -155,9 +154,20 @@ __global__ __launch_bounds__(256) void k_collapse(const float4 *__restrict__ nod
     }
     const uint32_t base = atomicAdd(nslots, (uint32_t)n);
     uint32_t qlo[3] = {0u, 0u, 0u}, qhi[3] = {0u, 0u, 0u};
-    for (int k = 0; k < n; k++) {
-        const float4 lo = nodes[2 * (size_t)kids[k]], hi = nodes[2 * (size_t)kids[k] + 1];
-        if (__float_as_uint(hi.w) & LR_LEAF) put_leaf(L, __float_as_uint(lo.w), slots + LR_SLOT_F4 * (size_t)(base + k));
+    float4 klo[4], khi[4];
+    uint32_t id[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {   // (the children's loads in flight together, then their leaves')
+        klo[k] = nodes[2 * (size_t)kids[k < n ? k : 0]];
+        khi[k] = nodes[2 * (size_t)kids[k < n ? k : 0] + 1];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) id[k] = __float_as_uint(khi[k].w) & LR_LEAF ? L.aux[__float_as_uint(klo[k].w)] : 0u;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        if (k >= n) continue;
+        const float4 lo = klo[k], hi = khi[k];
+        if (__float_as_uint(hi.w) & LR_LEAF) put_leaf(L, id[k], slots + LR_SLOT_F4 * (size_t)(base + k));
         else qout[atomicAdd(cout, 1u)] = WideTask{kids[k], base + (uint32_t)k};
         const float cl[3] = {lo.x, lo.y, lo.z}, ch[3] = {hi.x, hi.y, hi.z};
         for (int a = 0; a < 3; a++) {
