@@ -225,7 +225,7 @@ int lrh_pt_scene_update(LrhPtScene *s, const LrhInstance *inst, int ninst, int b
 int lrh_pt_scene_move(LrhPtScene *s, const int *idx, const LrhInstance *inst, int n, int builder, LrhBuildStats *stats);
 /* A dynamic mesh's new triangles (scene_mesh_changed, scene.h:385-386): ntris must be the
  * mesh's count. They are uploaded in its place, its tree is built again on the device in its
- * place (with its 4-wide copy and leaf-order triangles), and the top level over the instances
+ * place (with its 4-wide copy, whose leaves hold the triangles), and the top level over the instances
  * is rebuilt, as their world boxes follow the mesh's (upload_instances' dynamic meshes,
  * trace_gpu.c:1486-1512). The result equals a scene made with these triangles. No job of the
  * scene may be running. stats (optional): the mesh's build. */
@@ -253,7 +253,7 @@ int lrh_pt_render(LrhContext *c, const LrhPtScene *s, const float *cam, int W, i
  * square), d_guide 8 floats (lrh_engine_guide's layout). passes 1..5 a-trous passes (holes
  * 1, 2, 4, 8, 16 apart; 5 is the reference's). d_out: float4 per pixel (the denoised mean, 1);
  * lamps and the sky as they are, pixels with no sample 0. Asynchronous on the context's
- * stream; device memory. */
+ * stream; device memory. It takes 32 bytes a pixel of the context's scratch memory. */
 int lrh_denoise(LrhContext *c, const float *d_accum, const float *d_moments, const float *d_guide, int w, int h,
                 int passes, float *d_out);
 

@@ -14,14 +14,16 @@
 // guide's normal as an octahedron's two 16-bit snorms (the numbers the reference's filter sees),
 // and the distance, whose sign carries the kind. The early passes are bound by
 // their VALU instructions (25 taps a pixel), the late ones by their gathers (a tap jittered in a hole
-// of 8 or 16 pixels is a line of its own for each lane): so a tap is one 16-byte load (as two, of
-// irradiance and guide, the passes took 59, 70, 82, 102 and 143 us, now 62, 70, 70, 71 and 80) and few
+// of 8 or 16 pixels is a line of its own for each lane): so a tap is one 16-byte load and few
 // instructions: its normal comes off the octahedron by integers' exact arithmetic with one reciprocal
-// root in the weight, and its two exponentials are one, of the sum of their arguments. The hardware's
-// reciprocals, roots and exponential are within an ulp or two: the error against 64 bits, 1.3e-4 from
-// the halves, does not move. 1280 x 720, 5 passes: 507 -> 257 us (two divisions, two roots and two
-// exponentials a tap before). Read in 16 x 16 tiles, so a work-group's taps share the L2 lines of
-// their neighbourhood.
+// root in the weight, and its two exponentials are one, of the sum of their arguments. 1280 x 720, 5
+// passes: 503 us with two loads, two divisions, two roots and two exponentials a tap, 403 with cheaper
+// weights and still two loads, 258 as it is (by pass, under a profiler that makes them a fifth to a third
+// longer: 112, 118, 118, 120 and 122 us at first, now 56, 63, 63, 63 and 76). The hardware's
+// reciprocals, roots and exponential are within an ulp or two, of which the normal's power makes the
+// most. Against 64 bits: of a whole filter 1.7e-4 as before, from the halves; of one pass on
+// the same packed pixels (64 x 33 to 300 x 200) 1.05e-6 in the 2-norm, 1.06e-6 before. Read in 16 x 16
+// tiles, so a work-group's taps share the L2 lines of their neighbourhood.
 #include <hip/hip_fp16.h>
 
 #include "lr_internal.h"

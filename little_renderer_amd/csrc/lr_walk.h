@@ -204,11 +204,11 @@ __device__ __forceinline__ uint32_t stk_get(const WalkStack &S, int sp)
 // pushed and popped: it stays in registers as the next entry, with its two child fields
 // (lo.w, hi.w), which its parent's box test has already loaded. A farther child's two words go to
 // the stack in its place in the first PAIRS entries (S.stk: PAIRS + STK words a ray, for STK entries);
-// past them its index does, and the pop fetches them. The reference fetches the whole record of every node it pops. Same
-// visits, same tests, same hits. Bound by the loads' data path (a wave's lanes are at different
-// nodes, so a load takes 16 cycles or more whatever its width): without the pop's two loads, and with
-// box_t2, 1920 x 1080 camera rays through 1M triangles took 2.33 ms, before 2.56 (box_t2 alone 2.49;
-// with 14 stack entries in LDS instead of 10, and fewer waves, 2.75).
+// past them its index does, and the pop fetches them. The reference fetches the whole record of every
+// node it pops. Same visits, same tests, same hits. Bound by the loads' data path (a wave's lanes are at
+// different nodes, so a load takes 16 cycles or more whatever its width): without the pops' two loads,
+// and with box_t2 (a third of it), 1920 x 1080 camera rays through a PLOC tree of 1M triangles take 2.02
+// ms, before 2.26; with 14 two-word entries in LDS instead of 10, and fewer waves, 18 % more.
 // COUNT adds the node records fetched (the root's, each inner node's two children, each popped node's
 // past the PAIRS entries) and the shapes tested to cn, ct.
 template <bool ANY, bool PRIMS, bool COUNT, int PAIRS, int STK>
