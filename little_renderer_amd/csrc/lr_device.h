@@ -32,6 +32,14 @@ struct alignas(16) LrNode {
     uint32_t b;
 };
 
+// a ray whose tmin the 4-wide walks' keys take (lr_walk.h): from +0 up, no -0, no NaN
+__host__ __device__ __forceinline__ bool keys_ok(float tmin)
+{
+    uint32_t b;
+    __builtin_memcpy(&b, &tmin, 4);
+    return b <= 0x7f800000u;   // (no sign bit, no NaN)
+}
+
 __device__ __forceinline__ float wmin(float a, float b) { return b < a ? b : a; }
 __device__ __forceinline__ float wmax(float a, float b) { return b > a ? b : a; }
 // r_fmin / r_fmax of lrmath.h:56-57 (the other number when b is a NaN)

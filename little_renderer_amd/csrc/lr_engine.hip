@@ -14,6 +14,7 @@
 #include <map>
 #include <vector>
 
+#include "lr_device.h"
 #include "lr_engine.h"
 
 extern "C" void lrs_blue_noise(uint16_t *rank);
@@ -203,6 +204,8 @@ struct LrhEngine {
     hipGraphExec_t gexec = nullptr;
     bool graph_ok = false;
     bool two_level = false;     // a two-level scene has been submitted: the walks that take both
+    bool apart = false;         // a scene whose eps (its rays' tmin) the one launch's walks do not take has
+                                // been submitted: the walks' own kernels (keys_ok)
     bool multi = false;         // a scene with more than one light has been submitted: shade and
                                 // shadow that take up to three shadow rays a vertex
     double clk_khz = 100000.0, clk_host0 = 0.0;
@@ -242,10 +245,11 @@ EngArgs args_for(const LrhEngine *e, int stack, size_t threads, int mult, int re
 }
 
 bool refilled(const LrhEngine *e, int refill) { return !e->two_level && refill > 0; }
-// the walks go in one launch (not where they are counted or a walk's lanes refilled)
+// the walks go in one launch (not where they are counted or a walk's lanes refilled, nor with an eps that
+// their keys do not take)
 bool walks_joint(const LrhEngine *e, const LrhTune &t)
 {
-    return !e->counting && !refilled(e, t.refill) && !(refilled(e, t.refill_shadow) && !e->multi);
+    return !e->counting && !e->apart && !refilled(e, t.refill) && !(refilled(e, t.refill_shadow) && !e->multi);
 }
 
 // One iteration in the persistent grids of the batched form: regen, the walks, shade. ev (profiling):
@@ -572,6 +576,10 @@ int job_admit(LrhEngine *e, const LrhJob *j, int *slot_out)
         // from now on the walks that take two-level scenes too; the graphs already launched
         // run before this job's first paths are issued (the same stream)
         e->two_level = true;
+        e->graph_ok = false;
+    }
+    if (!keys_ok(s->eps) && !e->apart) {   // likewise, the walks' own kernels
+        e->apart = true;
         e->graph_ok = false;
     }
     if (lr_scene_multi_light(s) && !e->multi) {   // likewise, shade and shadow for several lights
@@ -1044,9 +1052,9 @@ int lrh_engine_plain(LrhEngine *e, const LrhJob *job, int64_t *id)
         // (a vertex's shadow rays are walked with the next one's rays: once more past the last vertex)
         T.regen[bs](gs, e->stream, As);
         for (int d = 0; d <= job->max_depth + 1; d++) {
-            if (e->counting) {
-                T.extend_count[bt][sk][tl](gt, e->stream, At);
-                T.shadow_count[bt][sk][tl][ml](gt, e->stream, At);
+            if (e->counting || e->apart) {
+                (e->counting ? T.extend_count : T.extend)[bt][sk][tl](gt, e->stream, At);
+                (e->counting ? T.shadow_count : T.shadow)[bt][sk][tl][ml](gt, e->stream, At);
             } else T.walks[bt][sk][tl][ml](gt, e->stream, At);
             T.shade[bs][ml](gs, e->stream, As);
         }

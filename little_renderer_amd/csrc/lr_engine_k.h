@@ -395,7 +395,7 @@ __device__ WalkHit walk4_tl(const JobDev &J, V3 o, V3 d, float tmin, float tmax,
             if (COUNT) count_node(c);
             float t[4];
             wide_test(r0, r1, r2, ro, inv, tmin, best.t, t);
-            more = wide_next<STK>(t, __float_as_uint(r1.w), S, sp, cur, overflow);
+            more = wide_next<STK, false>(t, __float_as_uint(r1.w), S, sp, cur, overflow);
         }
         if (!more) {
             if (sp == 0) break;
@@ -612,7 +612,7 @@ __device__ __forceinline__ void add_counts(unsigned long long *c, unsigned long 
 // extend (wf_ext, trace_wave.wgsl:72-84): the closest hit of the queue's k-th ray in the walk's order,
 // through its own job's tree. TL: two-level scenes may be queued (without it, such a ray is not
 // walked: flagged, so that the host reports it).
-template <bool COUNT, bool TL, int STK>
+template <bool COUNT, bool TL, int STK, bool KEYS>
 __device__ __forceinline__ void extend_entry(const EngArgs &A, int cur, uint32_t k, uint32_t ordered, const WalkStack &S, WalkCnt &wc)
 {
     const uint32_t i = k < ordered ? A.perm[k] : k;
@@ -622,7 +622,7 @@ __device__ __forceinline__ void extend_entry(const EngArgs &A, int cur, uint32_t
     WalkHit h;
     if (TL && J.two_level) h = walk4_tl<false, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
     else if (!J.two_level)
-        h = walk4<false, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
+        h = walk4<false, COUNT, STK, KEYS>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
     else {
         atomicOr(A.overflow, 2u);
         h = WalkHit{r1.w, LR_NONE, 0.0f, 0.0f};
@@ -633,7 +633,7 @@ __device__ __forceinline__ void extend_entry(const EngArgs &A, int cur, uint32_t
 // shadow (wf_shadow, trace_wave.wgsl:335-355): any hit before the lamp; if none, the
 // contribution joins the path's radiance. Paths whose last vertex made the shadow ray end here.
 // Every lane of the wave calls this (live: it has entry i).
-template <bool COUNT, bool TL, bool MULTI, int STK>
+template <bool COUNT, bool TL, bool MULTI, int STK, bool KEYS>
 __device__ __forceinline__ void shadow_entry(const EngArgs &A, int par, uint32_t i, bool live, const WalkStack &S, WalkCnt &wc,
                                              RetireSums &R)
 {
@@ -644,7 +644,7 @@ __device__ __forceinline__ void shadow_entry(const EngArgs &A, int par, uint32_t
     bool glow = false;
     auto walk = [&](const JobDev &J, float4 r0, float4 r1) {
         if (TL && J.two_level) return walk4_tl<true, COUNT, STK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
-        if (!J.two_level) return walk4<true, COUNT, STK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
+        if (!J.two_level) return walk4<true, COUNT, STK, KEYS>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w, r1.w, S, A.overflow, wc);
         atomicOr(A.overflow, 2u);
         return WalkHit{0.0f, 0u, 0.0f, 0.0f};   // occluded: adds nothing
     };
@@ -749,9 +749,9 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_walks(En
     retire_begin(R);
     for_tiles2<BLK>(&ctl->tiles[K_EXTEND], n, m, A.mult,
                     [&](uint32_t k, bool live) {
-                        if (live) extend_entry<false, TL, STK>(A, cur, k, ordered, S, wc);
+                        if (live) extend_entry<false, TL, STK, !TL>(A, cur, k, ordered, S, wc);
                     },
-                    [&](uint32_t i, bool live) { shadow_entry<false, TL, MULTI, STK>(A, cur, i, live, S, wc, R); });
+                    [&](uint32_t i, bool live) { shadow_entry<false, TL, MULTI, STK, !TL>(A, cur, i, live, S, wc, R); });
     retire_end(A, R);
 }
 
@@ -772,7 +772,7 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_extend(E
     const WalkStack S{&stk[0][threadIdx.x], BLK, A.spill + gtid, (size_t)A.spill_stride, STK + A.spill_per};
     WalkCnt wc;
     for_tiles<BLK>(&ctl->tiles[K_EXTEND], n, A.mult, [&](uint32_t k, bool live) {
-        if (live) extend_entry<COUNT, TL, STK>(A, cur, k, ordered, S, wc);
+        if (live) extend_entry<COUNT, TL, STK, false>(A, cur, k, ordered, S, wc);
     });
     if (COUNT) add_counts(A.counts, A.counts + 8, wc);
 }
@@ -795,7 +795,7 @@ __global__ __launch_bounds__(BLK, TL ? 1 : walk_waves(BLK, STK)) void k_shadow(E
     __shared__ RetireSums R;
     retire_begin(R);
     for_tiles<BLK>(&ctl->tiles[K_SHADOW], n, A.mult,
-                   [&](uint32_t i, bool live) { shadow_entry<COUNT, TL, MULTI, STK>(A, par, i, live, S, wc, R); });
+                   [&](uint32_t i, bool live) { shadow_entry<COUNT, TL, MULTI, STK, false>(A, par, i, live, S, wc, R); });
     retire_end(A, R);
     if (COUNT) add_counts(A.counts + 4, A.counts + 9, wc);
 }
@@ -837,7 +837,7 @@ __device__ __forceinline__ void walk_start(WalkState &w, const JobDev &J, float4
 template <bool ANY, bool COUNT, int STK>
 __device__ __forceinline__ bool walk_round(WalkState &w, const WalkStack &S, uint32_t *overflow, WalkCnt &wc)
 {
-    return !walk4_step<ANY, COUNT, STK>(w.slots, w.prims, w.nprims, w.o, w.d, w.inv, w.tmin, w.best, w.sp, w.cur, S, overflow, wc);
+    return !walk4_step<ANY, COUNT, STK, false>(w.slots, w.prims, w.nprims, w.o, w.d, w.inv, w.tmin, w.best, w.sp, w.cur, S, overflow, wc);
 }
 
 // a wave's claimed queue entries not yet handed out, [rb, re), and whether the counter may still

@@ -960,8 +960,10 @@ __global__ __launch_bounds__(128) void k_scene_trace(JobDev J, const float4 *__r
     const WalkStack S{&stk[0][threadIdx.x], 128, spill + i, (size_t)n, LR_LDS_STACK + spill_per};
     WalkCnt wc;
     const WalkHit h = J.two_level ? walk4_tl<ANY, false, LR_LDS_STACK>(J, v3of(r0), v3of(r1), r0.w, r1.w, S, overflow, wc)
-                                  : walk4<ANY, false, LR_LDS_STACK>(J.slots, J.prims, J.nprims, v3of(r0),
-                                                                    v3of(r1), r0.w, r1.w, S, overflow, wc);
+                      : keys_ok(r0.w) ? walk4<ANY, false, LR_LDS_STACK, true>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w,
+                                                                              r1.w, S, overflow, wc)
+                                      : walk4<ANY, false, LR_LDS_STACK>(J.slots, J.prims, J.nprims, v3of(r0), v3of(r1), r0.w,
+                                                                        r1.w, S, overflow, wc);
     hits[i] = make_float4(h.t, __uint_as_float(h.id), h.b1, h.b2);
 }
 

@@ -133,6 +133,56 @@ def test_profiled_launches(world, on):
     eng.close()
 
 
+def test_coincident_shapes_alike_in_both_launches(world):
+    # the walks' one launch orders a node's children by other instructions than their own launches:
+    # triangles given twice, in two materials, tell one order from another
+    ctx, _ = world
+    sc = lr.batch_scene(3000, 8)
+    t = np.asarray(sc["tris"], np.float32).copy()
+    again = t.copy()
+    w = again[:, 11].view(np.uint32)
+    again[:, 11] = ((((w >> 26) + 1) % len(sc["mats"]) << 26) | (w & 0x3ffffff)).view(np.float32)
+    both = np.concatenate([t, again])[np.random.default_rng(2).permutation(2 * len(t))]
+    ps = lr.PtScene(ctx, sc["prims"], both, sc["mats"], 0, sc["eps"], sc["margin"])
+    eng = lr.Engine(ctx, slots_log2=18, max_tree_depth=max(64, ps.info()[0]), image_bytes=16 << 20)
+    job = lr.make_job(ps, lr.batch_camera(9, 300, 200), 300, 200, 3, seed=6)
+    got = []
+    for on in (0, 1, 2):
+        eng.profiling(on)
+        i = eng.submit(job)
+        eng.drain()
+        got.append(image(eng, i, 300, 200))
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    eng.close()
+    ps.close()
+
+
+def test_a_scene_whose_eps_is_not_from_zero_up(world):
+    # its rays' tmin takes the walks' own launches, from then on; the images of both forms agree
+    ctx, other = world
+    sc = lr.batch_scene(2000, 5)
+    ps = lr.PtScene(ctx, sc["prims"], sc["tris"], sc["mats"], 0, -1e-4, sc["margin"])
+    eng = lr.Engine(ctx, slots_log2=16, max_tree_depth=max(64, ps.info()[0]), image_bytes=16 << 20)
+    before = lr.make_job(other, lr.batch_camera(9, 80, 60), 80, 60, 2, seed=6)
+    i = eng.submit(before)
+    eng.drain()
+    alone = image(eng, i, 80, 60)
+    job = lr.make_job(ps, lr.batch_camera(9, 80, 60), 80, 60, 2, seed=6)
+    i, j = eng.submit(job), eng.submit(before)
+    eng.drain()
+    assert np.array_equal(image(eng, j, 80, 60), alone)
+    assert np.array_equal(image(eng, i, 80, 60), image(eng, eng.plain(job), 80, 60))
+    n0 = list(eng.stats().kernel_launches)
+    eng.profiling(2)
+    i = eng.submit(job)
+    eng.drain()
+    eng.release(i)
+    n1 = list(eng.stats().kernel_launches)
+    assert n1[3] - n0[3] == n1[1] - n0[1] > 0
+    eng.close()
+    ps.close()
+
+
 @pytest.mark.parametrize("w, h", [(1, 1), (3, 65), (7, 9), (8, 8), (9, 7), (65, 3), (24, 20)])
 def test_ragged_images_match_the_oracle(world, w, h):
     ctx, _ = world
