@@ -435,7 +435,8 @@ int lrh_engine_tune_get(const LrhEngine *e, LrhTune *t);
 int lrh_engine_counting(LrhEngine *e, int on);
 /* profiling on: lrh_engine_pump launches the iterations kernel by kernel between hipEvents on
  * the engine's stream (no graph) and sums each kernel's time into the stats. An iteration's two
- * walks are one launch otherwise; on = 1 launches each alone, on = 2 the one launch. */
+ * walks are one launch otherwise (but where they are counted, their lanes refilled, or a running
+ * job's eps is negative, -0 or NaN); on = 1 launches each alone, on = 2 as they otherwise go. */
 int lrh_engine_profiling(LrhEngine *e, int on);
 /* Admits a job (its image cleared): LRH_EAGAIN if its image or a job slot cannot be had until
  * others are released. *id names it. Its paths are issued to the device in chunks of at most

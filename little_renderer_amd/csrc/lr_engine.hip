@@ -135,6 +135,7 @@ struct HostJob {
     double t_submit = 0, t_done = 0;
     unsigned long long min_seq = 0;   // the first progress snapshot taken after its admission
     bool ordered = false, two_level = false;   // its scene's: bounce rays worth ordering; of two levels
+    bool odd_eps = false;                      // ... and an eps that is not from +0 up (keys_ok)
 };
 
 struct IssueRec {
@@ -204,8 +205,8 @@ struct LrhEngine {
     hipGraphExec_t gexec = nullptr;
     bool graph_ok = false;
     bool two_level = false;     // a two-level scene has been submitted: the walks that take both
-    bool apart = false;         // a scene whose eps (its rays' tmin) the one launch's walks do not take has
-                                // been submitted: the walks' own kernels (keys_ok)
+    bool apart = false;         // a job of a scene whose eps (its rays' tmin) the one launch's walks do not
+                                // take runs (keys_ok): the walks' own kernels
     bool multi = false;         // a scene with more than one light has been submitted: shade and
                                 // shadow that take up to three shadow rays a vertex
     double clk_khz = 100000.0, clk_host0 = 0.0;
@@ -578,8 +579,11 @@ int job_admit(LrhEngine *e, const LrhJob *j, int *slot_out)
         e->two_level = true;
         e->graph_ok = false;
     }
-    if (!keys_ok(s->eps) && !e->apart) {   // likewise, the walks' own kernels
-        e->apart = true;
+    h.odd_eps = !keys_ok(s->eps);
+    bool apart = false;
+    for (const HostJob &r : e->hj) apart = apart || (r.state == LRH_JOB_RUNNING && r.odd_eps);
+    if (apart != e->apart) {   // likewise, the walks' own kernels (until none of those jobs runs)
+        e->apart = apart;
         e->graph_ok = false;
     }
     if (lr_scene_multi_light(s) && !e->multi) {   // likewise, shade and shadow for several lights
